@@ -364,10 +364,13 @@ __global__ __launch_bounds__(64 * KW) void k_grouped_down_ks(
 // one MFMA chain (fixed order).
 // ---------------------------------------------------------------------------
 constexpr int kErWaves = 8;
-// K of the tile-resident forms, in 256-code chunks (instantiated for the
-// synthetic model's hidden 2048 and intermediate 768; other sizes take the
-// K-split forms).
-constexpr int kErChunksUp = 8, kErChunksDown = 3;
+// K of the tile-resident forms, in 256-code chunks: the SwiGLU stage is built
+// for hidden 2048, the down stage for every intermediate up to 1024 (whole
+// rows of weights in registers, 2 NCH uint4 a lane); other sizes take the
+// K-split forms, whose 8 waves have nothing to split at such a K (256 experts
+// of intermediate 512: 57.3 against 16.4 us at 32 tokens, 120 against 33.2 us
+// at 509).
+constexpr int kErChunksUp = 8, kErMaxChunksDown = 4;
 constexpr int kErAhead = 2;  // weight chunks in flight per wave ahead of the MFMAs
 
 // SwiGLU: BPW up blocks (and the matching gate blocks) per wave; x' pairs of
@@ -1193,6 +1196,10 @@ static int grouped_launch(const void* x, int64_t ldx, const uint32_t* x_pairs, c
     // tile-resident forms: 16 rows (up + gate) / 32 rows per wave
     dim3 ge1(static_cast<unsigned>(cdiv(inter, 16 * kErWaves)), max_tiles);
     dim3 ge2(static_cast<unsigned>(cdiv(hidden, 32 * kErWaves)), max_tiles);
+#define MA_GROUPED_DOWN(ADT, NCH)                                                                \
+  hipLaunchKernelGGL((k_grouped_down_er<2, ADT, NCH>), ge2, dim3(64 * kErWaves), 0, s,           \
+                     reinterpret_cast<const uint32_t*>(hp), down, hidden, down_alpha, offsets,   \
+                     ne, out);
 #define MA_GROUPED_KS(ADT)                                                                       \
   if (x_pairs && hidden == 16 * 16 * kErChunksUp)                                                \
     hipLaunchKernelGGL((k_grouped_swiglu_er<1, ADT, kErChunksUp, 1>), ge1, dim3(64 * kErWaves),  \
@@ -1206,16 +1213,19 @@ static int grouped_launch(const void* x, int64_t ldx, const uint32_t* x_pairs, c
     hipLaunchKernelGGL((k_grouped_swiglu_ks<2, ADT, 8, false>), g1, dim3(512), 0, s, xb, ldx,    \
                        x_pairs, x_corr, top_k, up_gate, inter, hidden / 16, up_gate_alpha,      \
                        offsets, pair_ids, ne, hp, hb, ldh);                                      \
-  if (inter == 16 * 16 * kErChunksDown)                                                          \
-    hipLaunchKernelGGL((k_grouped_down_er<2, ADT, kErChunksDown>), ge2, dim3(64 * kErWaves), 0,  \
-                       s, reinterpret_cast<const uint32_t*>(hp), down, hidden, down_alpha,       \
-                       offsets, ne, out);                                                        \
-  else                                                                                           \
-    hipLaunchKernelGGL((k_grouped_down_ks<4, ADT, 8, 2>), g2, dim3(512), 0, s,                   \
-                       reinterpret_cast<const uint32_t*>(hp), down, hidden, inter / 16,          \
-                       down_alpha, offsets, ne, out);
+  switch (inter / 256) {                                                                         \
+    case 1: MA_GROUPED_DOWN(ADT, 1) break;                                                       \
+    case 2: MA_GROUPED_DOWN(ADT, 2) break;                                                       \
+    case 3: MA_GROUPED_DOWN(ADT, 3) break;                                                       \
+    case kErMaxChunksDown: MA_GROUPED_DOWN(ADT, kErMaxChunksDown) break;                         \
+    default:                                                                                     \
+      hipLaunchKernelGGL((k_grouped_down_ks<4, ADT, 8, 2>), g2, dim3(512), 0, s,                 \
+                         reinterpret_cast<const uint32_t*>(hp), down, hidden, inter / 16,        \
+                         down_alpha, offsets, ne, out);                                          \
+  }
     if (alpha_dtype == MA_BF16) { MA_GROUPED_KS(MA_BF16) } else { MA_GROUPED_KS(MA_F32) }
 #undef MA_GROUPED_KS
+#undef MA_GROUPED_DOWN
   } else {
     // prefill: the tokens' x' pairs once (or those of ma_moe_route), then
     // tiles of 128 pairs x 256 weight rows.  The tiles' copy sources are
