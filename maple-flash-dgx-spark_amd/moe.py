@@ -374,18 +374,20 @@ def moe_block(x: torch.Tensor, layer: MoELayer, top_k: int, residual: torch.Tens
         y, ids, wts = moe_fused(xf, layer, top_k, residual, prefetch=prefetch)
         return y.reshape(x.shape), ids, wts
     res = None if residual is None else residual.reshape(-1, hidden)
-    if plan == "grouped" and xf.shape[0] * top_k > 16 * layer.n_experts and hidden % 16 == 0:
-        # the grouped kernels' prefill form: the top-k launch also writes x'
+    if plan == "grouped":
+        # the top-k launch also writes the x' pairs that the grouped kernels read: the decode batches'
+        # tile-resident SwiGLU and the prefill form.  (Up to 16 tokens the router alone would be one launch
+        # instead of two, but the SwiGLU that expands x itself costs more: a block of 64 experts takes 35.4
+        # against 37.4 us at 4 tokens and 44.9 against 53.7 at 16, of 256 experts 41.6 against 63.6 and 51.7
+        # against 85.8; at 32 tokens 39.3 against 49.6 us.)
+        xf = xf.contiguous()
         ids, wts, xp = router_topk(xf, layer.gate_weight, top_k, bias=layer.router_bias, pairs=True)
         y = moe_grouped(xf, layer, ids, wts, res, x_pairs=xp)
         return y.reshape(x.shape), ids, wts
     ids, wts = router_topk(xf, layer.gate_weight, top_k, bias=layer.router_bias)
-    if plan == "grouped":
-        y = moe_grouped(xf, layer, ids, wts, res)
-    else:
-        h = ternary_expert_swiglu(xf, layer.up_gate_packed, layer.up_gate_alpha, ids)
-        y = ternary_expert_down_sum(h, layer.down_packed, layer.down_alpha, ids, wts, residual=res,
-                                    round_slots=True)
+    h = ternary_expert_swiglu(xf, layer.up_gate_packed, layer.up_gate_alpha, ids)
+    y = ternary_expert_down_sum(h, layer.down_packed, layer.down_alpha, ids, wts, residual=res,
+                                round_slots=True)
     return y.reshape(x.shape), ids, wts
 
 

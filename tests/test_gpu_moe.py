@@ -141,6 +141,25 @@ def test_moe_grouped_prefill_form_other_shapes(dev, hidden, n_exp, inter, k, tok
     assert torch.equal(y2, y) and torch.equal(h2, h)
 
 
+@pytest.mark.parametrize("n_exp,inter,tokens,alpha", [
+    (8, 256, 4, torch.bfloat16), (8, 256, 16, torch.float32), (256, 512, 17, torch.float32),
+    (256, 512, 33, torch.bfloat16), (40, 1024, 65, torch.bfloat16), (40, 1280, 20, torch.float32)])
+def test_moe_block_decode_batches_other_shapes(dev, n_exp, inter, tokens, alpha):
+    """Decode batches of the MoE block (the top-k launch also writes x') at every
+    K the tile-resident down stage is built for (256, 512, 1024) and one it is
+    not (1280), rows with a stride included."""
+    L = synthetic.make_moe_layer(H, n_exp, inter, seed=21, device=dev)
+    L.up_gate_alpha, L.down_alpha = L.up_gate_alpha.to(alpha), L.down_alpha.to(alpha)
+    assert tokens * K <= 16 * n_exp  # the decode form
+    x = synthetic.randn_bf16((tokens, H + 8), 900 + tokens, dev)[:, :H]  # rows of stride H + 8
+    res = synthetic.randn_bf16((tokens, H), 901 + tokens, dev)
+    y, ids, wts = moe_block(x, L, K, residual=res)
+    torch.cuda.synchronize()
+    ref, _ = ok.moe_experts(np_f(x), ids.cpu().numpy(), wts.cpu().numpy(), *_oracle_inputs(L), residual=np_f(res))
+    assert_bf16_close(np_f(y), ref, atol_frac=2.0 ** -7, what=f"E={n_exp} I={inter} T={tokens}")
+    assert torch.equal(moe_block(x, L, K, residual=res)[0], y)
+
+
 @pytest.mark.parametrize("tokens", [8, 32, 128])
 def test_moe_layer_routed_pairs_vs_oracle(dev, layer, tokens):
     """The decoder's batched MoE half: one routing launch that also writes xn
