@@ -57,12 +57,16 @@ int ma_ternary_gemv(const void* x, int x_dtype, int64_t batch, int64_t ldx,
  * (rms_weight != NULL) and 17 tokens or more, every token's GEMM operands
  * (the x' pairs of the hi and lo halves of x * w_rms, the correction and the
  * RMS scale) are built once into the workspace by a first launch and the MFMA
- * GEMM reads them from there.  workspace: 256-byte aligned, at least
- * ma_ternary_gemv_workspace_bytes(batch, nwords, rms_weight != NULL) bytes;
- * that query returns 0 where no workspace is used (no RMSNorm, batch < 17,
- * nwords % 16 != 0), and then -- as for any input the GEMM does not take --
- * the call is ma_ternary_gemv's and workspace may be NULL.  Same values as
- * ma_ternary_gemv up to float32 summation order.  Replaces ternary_gemv,
+ * GEMM reads them from there.  From 64 tokens, with or without the RMSNorm,
+ * the operands are FP8 pieces of x (two hold bf16 x whole, four carry x *
+ * w_rms) and the codes multiply them as FP4.  workspace: 256-byte aligned, at
+ * least ma_ternary_gemv_workspace_bytes(batch, nwords, rms_weight != NULL)
+ * bytes; that query returns 0 where no workspace is used (batch < 64 without
+ * the RMSNorm, batch < 17, nwords % 16 != 0), and then -- as for any input the
+ * GEMM does not take -- the call is ma_ternary_gemv's and workspace may be
+ * NULL; from 64 tokens a smaller workspace (or NULL without the RMSNorm) takes
+ * the form of fewer tokens.  Same values as ma_ternary_gemv up to float32
+ * summation order.  Replaces ternary_gemv,
  * src/maple_run/kernels/ternary_gemv.py:261-388 (its batched path :156-258).
  */
 size_t ma_ternary_gemv_workspace_bytes(int64_t batch, int64_t nwords, int rms);

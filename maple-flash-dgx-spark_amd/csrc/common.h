@@ -363,8 +363,35 @@ __device__ __forceinline__ float block_sum256(float v, float* red) {
 
 __host__ __device__ inline int64_t cdiv(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
+// 16 weights of the input RMSNorm (float32 or bf16) for K positions 16 wd ..
+__device__ __forceinline__ void load_rms16(const void* p, int rdt, int64_t wd, float out[16]) {
+  if (rdt == MA_F32) {
+    const uint4* q = reinterpret_cast<const uint4*>(static_cast<const float*>(p) + wd * 16);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint4 v = q[i];
+      out[4 * i] = __uint_as_float(v.x);
+      out[4 * i + 1] = __uint_as_float(v.y);
+      out[4 * i + 2] = __uint_as_float(v.z);
+      out[4 * i + 3] = __uint_as_float(v.w);
+    }
+  } else {
+    const uint4* q = reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(p) + wd * 16);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const uint4 v = q[i];
+      const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        out[8 * i + 2 * j] = __uint_as_float(u[j] << 16);
+        out[8 * i + 2 * j + 1] = __uint_as_float(u[j] & 0xffff0000u);
+      }
+    }
+  }
+}
+
 // A grouped MoE combine run in front of a kernel that reads its output rows
-// (k_xprep): y[t] = sum_j wts[t, j] * slot_out[inverse[t, j]] + res[t].
+// (k_xprep, k_mx_prep): y[t] = sum_j wts[t, j] * slot_out[inverse[t, j]] + res[t].
 // The (row, weight) pairs of token t's k <= 8 slots, in every lane: lane j
 // (mod 8) loads slot j's pair (slots past k re-read the last one), then each
 // pair is read off its lane -- two loads in flight at once, where 2k uniform
@@ -392,5 +419,60 @@ struct CombineIn {
   uint16_t* x_out;           // bf16 [batch, K * 16]: the combined rows
 };
 
+// Word wd (16 values) of token t's combined row [n], rounded to bf16 and
+// stored to cb.x_out, as floats in v: the slots in order, then the residual
+// (k_combine8's arithmetic).  row, w: slot_pairs8 of the token.
+__device__ __forceinline__ void combine_word16(const CombineIn& cb, const int64_t (&crow)[8], const float (&cw)[8],
+                                               int64_t t, int64_t wd, int64_t n, float (&v)[16]) {
+  uint4 sv[8][2], r[2] = {make_uint4(0u, 0u, 0u, 0u), make_uint4(0u, 0u, 0u, 0u)};
+#pragma unroll
+  for (int j = 0; j < 8; ++j)
+    if (j < cb.topk) {
+      const uint4* src = reinterpret_cast<const uint4*>(cb.slot_out + crow[j] * n + wd * 16);
+      sv[j][0] = src[0];
+      sv[j][1] = src[1];
+    }
+  if (cb.res) {
+    const uint4* src = reinterpret_cast<const uint4*>(cb.res + t * n + wd * 16);
+    r[0] = src[0];
+    r[1] = src[1];
+  }
+#pragma unroll
+  for (int hf = 0; hf < 2; ++hf) {
+    float a[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) a[e] = 0.f;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (j >= cb.topk) break;
+      const uint32_t u[4] = {sv[j][hf].x, sv[j][hf].y, sv[j][hf].z, sv[j][hf].w};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        a[2 * q] += cw[j] * __uint_as_float(u[q] << 16);
+        a[2 * q + 1] += cw[j] * __uint_as_float(u[q] & 0xffff0000u);
+      }
+    }
+    if (cb.res) {
+      const uint32_t u[4] = {r[hf].x, r[hf].y, r[hf].z, r[hf].w};
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        a[2 * q] += __uint_as_float(u[q] << 16);
+        a[2 * q + 1] += __uint_as_float(u[q] & 0xffff0000u);
+      }
+    }
+    uint4 o;
+    o.x = pack_bf16x2_rn(a[0], a[1]);
+    o.y = pack_bf16x2_rn(a[2], a[3]);
+    o.z = pack_bf16x2_rn(a[4], a[5]);
+    o.w = pack_bf16x2_rn(a[6], a[7]);
+    reinterpret_cast<uint4*>(cb.x_out + t * n + wd * 16)[hf] = o;
+    const uint32_t ou[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      v[8 * hf + 2 * q] = __uint_as_float(ou[q] << 16);
+      v[8 * hf + 2 * q + 1] = __uint_as_float(ou[q] & 0xffff0000u);
+    }
+  }
+}
 
 }  // namespace ma

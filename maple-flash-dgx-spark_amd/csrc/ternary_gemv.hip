@@ -107,8 +107,25 @@ int launch_tgemm_xp(const uint16_t* x, int64_t batch, int64_t ldx, const uint32_
                     int64_t n_out, int64_t nwords, const void* alpha, int alpha_dt,
                     const void* rms_w, int rms_dt, float rms_eps, uint16_t* y, int64_t ldy,
                     void* workspace, hipStream_t s, const ma::CombineIn& cb);
+// Two-launch scaled 8-bit form (mx_gemm.hip), taken by ma_ternary_gemv_ws from
+// kMxMinBatch tokens.
+size_t tgemm_mx_bytes(int64_t batch, int64_t nwords, bool rms);
+int launch_tgemm_mx(const uint16_t* x, int64_t batch, int64_t ldx, const uint32_t* w, int64_t n_out, int64_t nwords,
+                    const void* alpha, int alpha_dt, const void* rms_w, int rms_dt, float rms_eps, uint16_t* y,
+                    int64_t ldy, void* workspace, hipStream_t s, const ma::CombineIn& cb);
 constexpr int64_t kMfmaMinBatch = 5;
 constexpr int64_t kXpMinBatch = 17;
+constexpr int64_t kMxMinBatch = 64;
+
+// Where that form is the faster one: the others cost in proportion to tokens x
+// rows, this one about 17 us (24 with the RMSNorm) up to 512 tokens at K = 2048.
+// They cross near 5 x 2^16 outputs (128 tokens of 2560 rows 18.1 against 16.5
+// us, 128 of 2048 12.8 against 16.7, 512 of 1024 24.5 against 17.3) and with
+// the RMSNorm near 9 x 2^16 (256 of 2560 26.7 against 23.9, 96 of 5120 21.4
+// against 23.3, 512 of 1024 26.6 against 25.1); at K = 768 and 4096 alike.
+static bool mx_faster(int64_t batch, int64_t n_out, bool rms) {
+  return batch >= kMxMinBatch && batch * n_out >= (rms ? 9 : 5) * int64_t{65536};
+}
 
 static bool mfma_ok(const void* x, int x_dtype, int64_t batch, int64_t ldx, const uint32_t* packed,
                     int64_t nwords, int packed_kn, int alpha_dtype, const void* rms_weight,
@@ -147,8 +164,9 @@ extern "C" int ma_ternary_gemv(const void* x, int x_dtype, int64_t batch, int64_
 }
 
 extern "C" size_t ma_ternary_gemv_workspace_bytes(int64_t batch, int64_t nwords, int rms) {
-  if (!rms || batch < kXpMinBatch || nwords < 1 || nwords % 16 != 0) return 0;
-  return tgemm_xp_bytes(batch, nwords);
+  if (nwords < 1 || nwords % 16 != 0) return 0;
+  if (batch >= kMxMinBatch) return tgemm_mx_bytes(batch, nwords, rms != 0);
+  return rms && batch >= kXpMinBatch ? tgemm_xp_bytes(batch, nwords) : 0;
 }
 
 extern "C" int ma_ternary_gemv_ws(const void* x, int x_dtype, int64_t batch, int64_t ldx,
@@ -165,9 +183,15 @@ extern "C" int ma_ternary_gemv_ws(const void* x, int x_dtype, int64_t batch, int
   if (!x || !packed || !row_alpha || !y) return fail(MA_EVALUE, "ternary_gemv: null pointer");
   if (ldx < nwords * 16 || ldy < n_out)
     return fail(MA_EVALUE, "ternary_gemv: leading dimension too small");
-  if (!rms_weight || batch < kXpMinBatch ||
-      !mfma_ok(x, x_dtype, batch, ldx, packed, nwords, packed_kn, alpha_dtype, rms_weight,
-               rms_dtype, y))
+  const bool mfma = mfma_ok(x, x_dtype, batch, ldx, packed, nwords, packed_kn, alpha_dtype, rms_weight,
+                            rms_dtype, y);
+  // (a workspace of less than the query's bytes still takes the forms that need less)
+  if (mfma && mx_faster(batch, n_out, rms_weight != nullptr) && workspace && !(reinterpret_cast<uintptr_t>(workspace) & 255) &&
+      workspace_bytes >= tgemm_mx_bytes(batch, nwords, rms_weight != nullptr))
+    return launch_tgemm_mx(static_cast<const uint16_t*>(x), batch, ldx, packed, n_out, nwords, row_alpha,
+                           alpha_dtype, rms_weight, rms_dtype, rms_eps, static_cast<uint16_t*>(y), ldy, workspace,
+                           static_cast<hipStream_t>(stream), ma::CombineIn{});
+  if (!rms_weight || batch < kXpMinBatch || !mfma)
     return ma_ternary_gemv(x, x_dtype, batch, ldx, packed, n_out, nwords, packed_kn, row_alpha,
                            alpha_dtype, rms_weight, rms_dtype, rms_eps, y, ldy, stream);
   const size_t need = tgemm_xp_bytes(batch, nwords);
@@ -215,6 +239,10 @@ extern "C" int ma_ternary_gemv_combine_ws(const void* slot_out, const int32_t* i
   const CombineIn cb{static_cast<const uint16_t*>(slot_out), inverse, topk_weight,
                      static_cast<int>(top_k), static_cast<const uint16_t*>(residual),
                      static_cast<uint16_t*>(x_out)};
+  if (mx_faster(batch, n_out, true) && workspace_bytes >= tgemm_mx_bytes(batch, nwords, true))
+    return launch_tgemm_mx(static_cast<const uint16_t*>(x_out), batch, nwords * 16, packed, n_out, nwords, row_alpha,
+                           alpha_dtype, rms_weight, rms_dtype, rms_eps, static_cast<uint16_t*>(y), ldy, workspace,
+                           static_cast<hipStream_t>(stream), cb);
   return launch_tgemm_xp(static_cast<const uint16_t*>(x_out), batch, nwords * 16, packed, n_out,
                          nwords, row_alpha, alpha_dtype, rms_weight, rms_dtype, rms_eps,
                          static_cast<uint16_t*>(y), ldy, workspace, static_cast<hipStream_t>(stream), cb);

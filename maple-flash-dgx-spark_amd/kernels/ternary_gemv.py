@@ -3,7 +3,7 @@
 Drop-in for reference ``src/maple_run/kernels/ternary_gemv.py:261-388``: same
 signature, argument meaning, output shape/dtype and exceptions.  The work is
 ``ma_ternary_gemv`` (one launch) or, for the RMS-folded form at 17 tokens and
-more, ``ma_ternary_gemv_ws`` (operand build + GEMM), HIP on gfx950, on the
+more and for any form at 64, ``ma_ternary_gemv_ws`` (operand build + GEMM), HIP on gfx950, on the
 current stream.
 """
 
@@ -87,7 +87,7 @@ def ternary_gemv(
         float(rms_eps),
         _lib.ptr(y), n_out,
     )
-    # With the RMSNorm folded in, from 17 tokens the MFMA GEMM's two-launch form
+    # With the RMSNorm folded in, from 17 tokens, and always from 64, a two-launch form
     # builds each token's operands once into a workspace (the query says 0 where
     # no workspace is used).
     ws_bytes = _lib.load().ma_ternary_gemv_workspace_bytes(batch, nwords, int(rms_w is not None))

@@ -361,6 +361,55 @@ def test_gemv_two_launch_small_workspace_raises(dev):
         _gemv_c("ma_ternary_gemv_ws", x, w, alpha, rms_w, None)
 
 
+@pytest.mark.parametrize("tokens,n_out,k_in,rms,alpha", [
+    (64, 5120, 256, None, torch.bfloat16),         # the fewest tokens, one pass over the step buffers
+    (65, 5129, 768, None, torch.float32),          # ragged tokens and rows, odd row count, 6 steps
+    (513, 2056, 2048, None, torch.bfloat16),       # two buffers (over 512 tiles would be; here three)
+    (2049, 2050, 256, None, torch.float32),        # over 512 tiles
+    (129, 4600, 512, torch.float32, torch.bfloat16),
+    (290, 2056, 1280, torch.bfloat16, torch.float32),  # 10 steps
+])
+def test_gemv_mx_vs_oracle(dev, tokens, n_out, k_in, rms, alpha):
+    """Projections of many tokens (ma_ternary_gemv_ws's scaled 8-bit form) at the
+    edges of its tiles, over values of very different size in one block, rows
+    with a stride; the same bits on a second run; a token with an infinity is
+    NaN and leaves the others alone."""
+    rng = np.random.default_rng(tokens)
+    w = synthetic.ternary_packed((n_out, k_in), 75, dev)
+    a = synthetic.uniform_bf16((n_out,), 0.01, 0.05, 76, dev).to(alpha)
+    x = synthetic.randn_bf16((tokens, k_in + 8), 77, dev)[:, :k_in]
+    scale = torch.from_numpy(2.0 ** rng.integers(-6, 7, size=(tokens, k_in))).to(dev)
+    x.copy_((x.double() * scale).to(torch.bfloat16))
+    rms_w = None if rms is None else (torch.rand(k_in, device=dev) + 0.5).to(rms)
+    y = ternary_gemv(x, w, a, rms_weight=rms_w, rms_eps=1e-6)
+    ref = ok.ternary_gemv(np_f(x), np_u32(w), np_f(a), rms_weight=None if rms_w is None else np_f(rms_w), rms_eps=1e-6)
+    assert_bf16_close(np_f(y), ref, what=f"T={tokens} N={n_out} K={k_in}")
+    assert torch.equal(ternary_gemv(x, w, a, rms_weight=rms_w, rms_eps=1e-6), y)
+    x[tokens // 2, 3] = float("inf")
+    z = ternary_gemv(x, w, a, rms_weight=rms_w, rms_eps=1e-6)
+    keep = torch.arange(tokens, device=dev) != tokens // 2
+    assert torch.equal(z[keep], y[keep]) and bool(z[tokens // 2].isnan().all())
+
+
+def test_gemv_mx_small_workspace_takes_the_other_forms(dev):
+    """From 64 tokens a workspace below the query's bytes, or none without the
+    RMSNorm, is taken by the forms of fewer tokens, as before; below theirs the
+    RMS-folded call is refused."""
+    from maple_amd import _lib
+    w = synthetic.ternary_packed((5120, 512), 85, dev)
+    a = synthetic.uniform_bf16((5120,), 0.01, 0.05, 86, dev)
+    x = synthetic.randn_bf16((128, 512), 87, dev)
+    rms_w = torch.rand(512, device=dev) + 0.5
+    y = _gemv_c("ma_ternary_gemv_ws", x, w, a, None, None)
+    assert torch.equal(y, _gemv_c("ma_ternary_gemv", x, w, a))
+    nbytes = _lib.load().ma_ternary_gemv_workspace_bytes(128, 32, 1)
+    ws = torch.empty(nbytes - 256, device=dev, dtype=torch.uint8)
+    ref = ok.ternary_gemv(np_f(x), np_u32(w), np_f(a), rms_weight=np_f(rms_w), rms_eps=1e-6)
+    assert_bf16_close(np_f(_gemv_c("ma_ternary_gemv_ws", x, w, a, rms_w, ws)), ref, what="smaller workspace")
+    with pytest.raises(ValueError, match="workspace"):
+        _gemv_c("ma_ternary_gemv_ws", x, w, a, rms_w, ws[:4096])
+
+
 # ---------------------------------------------------------------- RTN4 / norms
 @pytest.mark.parametrize("batch,group", [(1, 128), (1, 64), (2, 128), (4, 64), (32, 128)])
 def test_rtn4_gemv_vs_oracle(dev, batch, group):
