@@ -258,6 +258,24 @@ int ma_rtn4_gemv_ws(const void* x, int x_dtype, int64_t batch, int64_t ldx,
                     void* stream);
 
 /*
+ * ma_rtn4_gemv on the scaled 8-bit matrix instructions, from batch 5 in groups
+ * of 64 or 128 with nwords a multiple of 32 (bf16 x, [N, K/8] codes, bf16 or
+ * float32 scales and biases of one dtype; x, codes, scales and biases 16-byte
+ * aligned): x is written once into the workspace as FP8 pieces that hold it
+ * whole, and the codes multiply it as FP8.  Any other call is ma_rtn4_gemv's.
+ * Same values as ma_rtn4_gemv up to float32 summation order.  workspace:
+ * ma_rtn4_gemv_mx_workspace_bytes(batch, nwords, group_size) bytes (0: none
+ * needed), 256-byte aligned; calls sharing one must not overlap.  Replaces
+ * rtn4_gemv, src/maple_run/kernels/rtn4.py:285-415.
+ */
+size_t ma_rtn4_gemv_mx_workspace_bytes(int64_t batch, int64_t nwords, int64_t group_size);
+int ma_rtn4_gemv_mx(const void* x, int x_dtype, int64_t batch, int64_t ldx,
+                    const uint32_t* packed, int64_t n_out, int64_t nwords, int packed_kn,
+                    const void* scales, int scales_dtype, const void* biases, int biases_dtype,
+                    int64_t group_size, void* y, int64_t ldy, void* workspace, size_t workspace_bytes,
+                    void* stream);
+
+/*
  * out[i, k] = q[ids[i], k] * scale[ids[i], g] + bias[ids[i], g] in float32.
  * Replaces rtn4_embedding, src/maple_run/kernels/rtn4.py:27-47.
  */

@@ -433,8 +433,13 @@ int launch_rtn4_mfma_ws(const uint16_t* x, int64_t batch, int64_t ldx, const uin
                         int64_t n_out, int64_t nwords, int64_t group, const void* scales,
                         const void* biases, int s_dt, uint16_t* y, int64_t ldy, void* workspace,
                         hipStream_t s);
+// Scaled 8-bit form (mx_head.hip).
+int launch_rtn4_mx(const uint16_t* x, int64_t batch, int64_t ldx, const uint32_t* w, int64_t n_out, int64_t nwords,
+                   int64_t group, const void* scales, const void* biases, int s_dt, uint16_t* y, int64_t ldy,
+                   void* workspace, hipStream_t s);
 namespace ma {
 size_t rtn4_ws_bytes(int64_t batch, int64_t nwords, int64_t group);
+size_t rtn4_mx_bytes(int64_t batch, int64_t nwords, int64_t group);
 }  // namespace ma
 
 // Whether a call takes the workspace form: the batched MFMA path (bf16 x,
@@ -506,6 +511,31 @@ extern "C" int ma_rtn4_gemv_ws(const void* x, int x_dtype, int64_t batch, int64_
     return launch_rtn4_mfma_ws(static_cast<const uint16_t*>(x), batch, ldx, packed, n_out, nwords, group_size,
                                scales, biases, scales_dtype, static_cast<uint16_t*>(y), ldy, workspace,
                                static_cast<hipStream_t>(stream));
+  }
+  return ma_rtn4_gemv(x, x_dtype, batch, ldx, packed, n_out, nwords, packed_kn, scales, scales_dtype, biases,
+                      biases_dtype, group_size, y, ldy, stream);
+}
+
+extern "C" size_t ma_rtn4_gemv_mx_workspace_bytes(int64_t batch, int64_t nwords, int64_t group_size) {
+  if (batch < 5 || (group_size != 64 && group_size != 128) || nwords < 32 || nwords % 32) return 0;
+  return rtn4_mx_bytes(batch, nwords, group_size);
+}
+
+extern "C" int ma_rtn4_gemv_mx(const void* x, int x_dtype, int64_t batch, int64_t ldx, const uint32_t* packed,
+                               int64_t n_out, int64_t nwords, int packed_kn, const void* scales, int scales_dtype,
+                               const void* biases, int biases_dtype, int64_t group_size, void* y, int64_t ldy,
+                               void* workspace, size_t workspace_bytes, void* stream) {
+  const size_t need = ma_rtn4_gemv_mx_workspace_bytes(batch, nwords, group_size);
+  if (need && n_out > 0 && x_dtype == MA_BF16 && !packed_kn && scales_dtype == biases_dtype &&
+      (scales_dtype == MA_BF16 || scales_dtype == MA_F32) && ldx % 8 == 0 && ldx >= nwords * 8 && ldy >= n_out &&
+      ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(packed) | reinterpret_cast<uintptr_t>(scales) |
+        reinterpret_cast<uintptr_t>(biases)) & 15u) == 0 &&
+      (reinterpret_cast<uintptr_t>(y) & 3u) == 0) {
+    if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u) || workspace_bytes < need)
+      return fail(MA_EVALUE, "rtn4_gemv_mx: workspace missing, misaligned or under %zu bytes", need);
+    return launch_rtn4_mx(static_cast<const uint16_t*>(x), batch, ldx, packed, n_out, nwords, group_size, scales,
+                          biases, scales_dtype, static_cast<uint16_t*>(y), ldy, workspace,
+                          static_cast<hipStream_t>(stream));
   }
   return ma_rtn4_gemv(x, x_dtype, batch, ldx, packed, n_out, nwords, packed_kn, scales, scales_dtype, biases,
                       biases_dtype, group_size, y, ldy, stream);

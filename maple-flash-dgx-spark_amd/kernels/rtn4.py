@@ -12,7 +12,7 @@ from __future__ import annotations
 
 import torch
 
-from .. import _lib, workspace
+from .. import _lib
 
 _CODES_PER_WORD = 8
 HEAD_GROUP_SIZE = 64
@@ -104,12 +104,12 @@ def rtn4_gemv(
         _lib.ptr(sc), _lib.dtype_code(sc, "scales"), _lib.ptr(bs), _lib.dtype_code(bs, "biases"),
         int(group_size), _lib.ptr(y), n_out,
     )
-    # Batched calls in groups of 128 build their x' operands once into a
-    # per-stream workspace (ma_rtn4_gemv_ws); others need none.
-    nbytes = 0 if packed_kn else int(_lib.load().ma_rtn4_gemv_workspace_bytes(batch, nwords, int(group_size)))
+    # Batched calls write x once into a workspace, as the scaled 8-bit form reads it; calls that it does not take
+    # need none.
+    nbytes = 0 if packed_kn else int(_lib.load().ma_rtn4_gemv_mx_workspace_bytes(batch, nwords, int(group_size)))
     if nbytes:
-        ws = workspace.get("rtn4", x.device, nbytes, (nwords, int(group_size)))
-        _lib.call("ma_rtn4_gemv_ws", *args, _lib.ptr(ws), ws.numel(), _lib.stream_of(x))
+        ws = torch.empty(nbytes, device=x.device, dtype=torch.uint8)
+        _lib.call("ma_rtn4_gemv_mx", *args, _lib.ptr(ws), ws.numel(), _lib.stream_of(x))
     else:
         _lib.call("ma_rtn4_gemv", *args, _lib.stream_of(x))
     return y.reshape(*leading, n_out)

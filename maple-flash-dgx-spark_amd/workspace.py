@@ -11,8 +11,8 @@ workspaces, and calls on one stream are ordered by it.
 A HIP graph keeps the workspace of the stream it was captured on; replay it
 in that stream's order relative to eager calls made on the capture stream.
 (The attention workspace belongs to its KV cache, ``gqa_workspace``.)
-The pool also holds per-call scratch that a kernel rewrites on every call (the
-RTN4 GEMM's operands); it carries no timeout word and is never zeroed here.
+Per-call scratch that a kernel rewrites on every call may sit in the pool too;
+it carries no timeout word and is never zeroed here.
 
 A workspace that has to grow is replaced by a larger one (at least twice the
 size, so the replaced ones add up to less than the current one), and the one
@@ -101,7 +101,7 @@ def register_attention(ws: torch.Tensor) -> torch.Tensor:
 
 def _all(idx: int) -> list[tuple[str, torch.Tensor]]:
     """The workspaces on device ``idx`` that carry a timeout word (per-call
-    scratch kept in the pool, such as the RTN4 GEMM's operands, has none)."""
+    scratch kept in the pool has none)."""
     out = [(k[0], ws) for k, ws in list(_POOL.items()) + _RETIRED if k[1] == idx and k[0] in TIMEOUT_WORD]
     out += [("attention", ws) for ws in list(_ATTENTION.values()) if ws.device.index == idx]
     return out

@@ -438,6 +438,48 @@ def test_rtn4_mfma_batched_vs_oracle(dev, batch, group, n_out):
         assert torch.equal(rtn4_gemv(x, w, sc, bs, group_size=group), y)
 
 
+@pytest.mark.parametrize("batch,n_out,k_in,group,dtype", [
+    (5, 1003, 256, 64, torch.bfloat16),     # 4 groups: biases by FMA; odd row count
+    (32, 129, 1024, 64, torch.bfloat16),    # 16 groups: biases by the matrix units
+    (33, 515, 2048, 128, torch.bfloat16),   # 64-token tiles, 16 groups
+    (64, 256, 768, 128, torch.float32),
+    (65, 1000, 2048, 64, torch.bfloat16),   # 128 x 128 tiles
+    (129, 1029, 1280, 128, torch.bfloat16),
+    (256, 384, 512, 64, torch.float32),
+])
+def test_rtn4_mx_vs_oracle(dev, batch, n_out, k_in, group, dtype):
+    """ma_rtn4_gemv_mx at the edges of its tiles, both group sizes, both scale
+    types, values of very different size, rows with a stride; the same bits on a
+    second run; a row with an infinity is NaN and leaves the others alone."""
+    rng = np.random.default_rng(batch)
+    w, sc, bs = synthetic.rtn4_table(n_out, k_in, group, 97 + batch, dev)
+    sc, bs = sc.to(dtype), bs.to(dtype)
+    x = synthetic.randn_bf16((batch, k_in + 8), 98, dev)[:, :k_in]
+    scale = torch.from_numpy(2.0 ** rng.integers(-6, 7, size=(batch, k_in))).to(dev)
+    x.copy_((x.double() * scale).to(torch.bfloat16))
+    y = rtn4_gemv(x, w, sc, bs, group_size=group)
+    ref = ok.rtn4_gemv(np_f(x), np_u32(w), np_f(sc), np_f(bs), group_size=group)
+    assert_bf16_close(np_f(y), ref, what=f"rtn4 mx B={batch} g={group}")
+    assert torch.equal(rtn4_gemv(x, w, sc, bs, group_size=group), y)
+    x[batch // 2, 5] = float("-inf")
+    z = rtn4_gemv(x, w, sc, bs, group_size=group)
+    keep = torch.arange(batch, device=dev) != batch // 2
+    assert torch.equal(z[keep], y[keep]) and bool(z[batch // 2].isnan().all())
+
+
+def test_rtn4_mx_workspace_refused(dev):
+    from maple_amd import _lib
+    w, sc, bs = synthetic.rtn4_table(128, 256, 64, 99, dev)
+    x = synthetic.randn_bf16((6, 256), 99, dev)
+    y = torch.empty(6, 128, device=dev, dtype=torch.bfloat16)
+    nbytes = int(_lib.load().ma_rtn4_gemv_mx_workspace_bytes(6, 32, 64))
+    ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+    for p, n in ((_lib.ptr(ws), nbytes - 1), (None, nbytes), (_lib.ptr(ws[16:]), nbytes)):
+        with pytest.raises(ValueError, match="workspace"):
+            _lib.call("ma_rtn4_gemv_mx", _lib.ptr(x), _lib.BF16, 6, 256, _lib.ptr(w), 128, 32, 0, _lib.ptr(sc),
+                      _lib.BF16, _lib.ptr(bs), _lib.BF16, 64, _lib.ptr(y), 128, p, n, _lib.stream_of(x))
+
+
 @pytest.mark.parametrize("batch,n_out", [(5, 4096), (17, 4096), (32, 8192), (64, 4064)])
 def test_rtn4_workspace_form_equals_one_launch(dev, batch, n_out):
     """ma_rtn4_gemv_ws (groups of 128: x' and group sums built once, copied
