@@ -28,6 +28,7 @@
 #include <mutex>
 
 #include "mfma.h"
+#include "mx.h"
 
 namespace ma {
 
@@ -699,196 +700,209 @@ __global__ __launch_bounds__(256) void k_combine8(const uint16_t* __restrict__ o
 }
 
 // ---------------------------------------------------------------------------
-// Prefill form (many pairs per expert): tiles of 128 pairs x 256 weight rows,
-// eight waves (4 along the rows x 2 along the pairs, 64 x 64 each), K walked
-// in steps of 8 words (128 codes).  The pairs' x' operands of a step (32 KB)
-// are copied into LDS by the LDS DMA (global_load_lds_dwordx4: no staging
-// registers), double-buffered: the next step's copy and weights are in flight
-// during this step's MFMAs, one barrier per step.  That keeps a workgroup
-// under 128 VGPRs and 70 KB of LDS, so two run on a CU.  x' pairs and the
-// per-token correction are built once per token (k_gp_prep), so staging is a
-// copy.  Each lane expands its own weight words in registers, half a word
-// (the 4 operand dwords one MFMA takes) at a time: a lane group g takes
-// words 2g and 2g+1 of a step, substep s (K = 32) the pairs 4(s & 1)..+3 of
-// word 2g + (s >> 1) -- the same K permutation on both operands.  Tiles go to
-// workgroups so that the row tiles of one pair tile share an XCD (workgroups
-// are placed on the 8 XCDs round-robin), which keeps that tile's x' in one L2.
+// Prefill form (many pairs per expert): tiles of 64 or 32 pairs x 256 weight
+// rows, four waves of 64 rows, K walked in steps of 8 words (128 codes) on
+// v_mfma_scale_f32_16x16x128_f8f6f4: the codes as FP4, the activations as mx
+// rows of two FP8 pieces (mx.h), which hold bf16 values whole.  A step's mx
+// rows of the pairs are copied into LDS by the LDS DMA
+// (global_load_lds_dwordx4: no staging registers), one step ahead with the
+// step's weights, one barrier per step; three workgroups run on a CU (two steps
+// ahead was no faster: 194 against 189 us a block of 2048 tokens).  The
+// tokens' mx rows are written once (launch_mx_prep_wide) and h's by the SwiGLU
+// epilogue, so staging is a copy.  Each lane expands its own weight words with
+// two ANDs and a shift a word: words 4g .. 4g+3 of two steps' 16 for lane group
+// g, loaded at once (64 bytes of a row), the first two in the even step.  Tiles go to workgroups so that the row tiles of one pair tile share an
+// XCD (workgroups are placed on the 8 XCDs round-robin), which keeps that
+// tile's rows in one L2.
+//
+// 2048 tokens x 8 on 64 experts (103 GFLOP SwiGLU, 52 down): 104 and 60 us with
+// 32 bytes of a row at a time, 121 and 69 as bf16 tiles of 128 pairs, whose
+// matrix units waited for the expansion (12 instructions a word) and multiplied
+// a quarter of padding; with 64 bytes at a time the whole block went from 189 to
+// 176 us (237 as bf16).  Bound by issue: the matrix units work 58 % of the time,
+// the epilogue and the addresses take most of the rest.
 // ---------------------------------------------------------------------------
 namespace gp {
-constexpr int kTok = 128;    // pairs per tile
 constexpr int kRows = 256;   // weight rows per tile (SwiGLU: 128 up + the 128 matching gate rows)
 constexpr int kWords = 8;    // packed words of K per step
-constexpr int kWaves = 8;
-constexpr int kThreads = 64 * kWaves;
+constexpr int kPieces = 2;
+constexpr int kChunks = 8 * kPieces;  // 16-byte chunks of an mx row per step
 constexpr int kXcds = 8;
-// One step's x' in LDS: 16-byte slot p * 16 + (c ^ (p % 16)) holds chunk c
-// (word c / 2, half c % 2) of pair p -- each pair's 256 bytes in one run, the
-// chunks XOR-swizzled so that the B reads (16 pairs of one chunk) hit 16
-// different bank groups; the DMA fills slots in order, so each copy's source
-// is chosen to match.
-constexpr int kXsDwords = kTok * 2 * kWords * 4;  // one buffer (32 KB)
-// After the K loop the same LDS stages the output tile for coalesced stores:
-// h as [pair][128 outputs] (rows padded to 136 bf16), the down outputs as
+// After the K loop a buffer stages the output tile for coalesced stores: h as
+// [pair][one step of an mx row] (256 bytes padded to 272), the down outputs as
 // [pair][256 rows] (rows padded to 264 bf16); the padding keeps the 16 pair
 // columns of a lane group on different banks and every row 16-byte aligned.
-constexpr int kHRow = 136, kORow = 264;
-// Buffer A also stages the output tile: all of h (128 x 136 bf16), or half of
-// the down tile's pairs at a time (64 x 264 bf16).
-constexpr int kXaDwords = (kTok * kHRow / 2 > kTok / 2 * kORow / 2) ? kTok * kHRow / 2 : kTok / 2 * kORow / 2;
-static_assert(kXaDwords >= kXsDwords, "buffer A holds a step");
+constexpr int kHRow = 272, kORow = 264;
+// Tiles of TOK pairs: 4 waves of 64 rows each over all of the pairs.
+template <int TOK>
+struct Tile {
+  static constexpr int kRb = 4, kNb = TOK / 16;  // blocks of 16 rows and of 16 pairs a wave
+  static constexpr int kThreads = 256;
+  static constexpr int kWaves = TOK == 64 ? 3 : 4;          // per SIMD, at most
+  static constexpr int kCopies = TOK * kChunks / kThreads;  // per thread and step
+  // One step's mx rows in LDS: 16-byte slot p * 16 + (c ^ (p % 16)) holds
+  // chunk c (piece c / 8, bytes 16 (c % 8) ..+15) of pair p -- each pair's 256
+  // bytes in one run, the chunks XOR-swizzled so that the B reads (16 pairs of
+  // one chunk) hit 16 different bank groups; the DMA fills slots in order, so
+  // each copy's source is chosen to match.
+  static constexpr int kXsDwords = TOK * kChunks * 4;
+  // Buffer A also stages the output tile: all of h, or half of the down tile's
+  // pairs at a time.
+  static constexpr int kOut = TOK / 2 * kORow / 2, kH = TOK * kHRow / 4;
+  static constexpr int kXaDwords = kH > kOut ? (kH > kXsDwords ? kH : kXsDwords) : (kOut > kXsDwords ? kOut : kXsDwords);
+};
 }  // namespace gp
 
-// x' pairs of every token once: xp [T, nwords * 8] (word w: pair j =
-// (f_j x[16w+j], f_j x[16w+j+8])) and xc[t] = sum (f + 1) x over the row, in
-// a fixed order.
-__global__ __launch_bounds__(128) void k_gp_prep(const uint16_t* __restrict__ x, int64_t ldx,
-                                                 int64_t nwords, uint32_t* __restrict__ xp,
-                                                 float* __restrict__ xc) {
-  __shared__ float red[2];
-  const int64_t t = blockIdx.x;
-  const int tid = threadIdx.x;
-  float c = 0.f;
-  for (int64_t wd = tid; wd < nwords; wd += 128) {
-    const uint4* src = reinterpret_cast<const uint4*>(x + t * ldx + wd * 16);
-    uint32_t pr[8];
-    c += x16_to_pairs(src[0], src[1], pr);
-    uint4* dst = reinterpret_cast<uint4*>(xp + (t * nwords + wd) * 8);
-    dst[0] = make_uint4(pr[0], pr[1], pr[2], pr[3]);
-    dst[1] = make_uint4(pr[4], pr[5], pr[6], pr[7]);
-  }
-  c = group_sum<64>(c);
-  if ((tid & 63) == 0) red[tid >> 6] = c;
-  __syncthreads();
-  if (tid == 0) xc[t] = red[0] + red[1];
-}
-
 // Tile of workgroup L (workgroups go to the 8 XCDs round-robin: L on XCD
-// L % 8, the XCD's slot L / 8).  The M pair tiles (experts in order, each
-// expert's tiles consecutive) are cut into 8 contiguous ranges of ceil(M / 8),
-// one per XCD, and an XCD's slots walk its range pair tile by pair tile, the
-// row tiles of a pair tile together: so an expert's pair tiles run on one
-// XCD (two at a range boundary) and read its codes through one L2, and the
-// row tiles of a pair tile share its x'.  M is counted from the dispatch
-// offsets (the grid is sized for the most tiles T k / 128 + E).  Returns
-// false for the workgroups past the XCD's range.
+// L % 8, the XCD's slot L / 8).  The M x n_rtiles tiles (pair tiles with their
+// experts in order, the row tiles of a pair tile together) are cut into 8
+// contiguous ranges of equal length, one per XCD: so an expert's pair tiles run
+// on one XCD (two at a range boundary) and read its codes through one L2, the
+// row tiles of a pair tile share its mx rows, and no XCD has more than one tile
+// above its share.  M is counted from the dispatch offsets (the grid is sized
+// for the most tiles T k / TOK + E).  Returns false for the workgroups past the
+// XCD's range.
+template <int TOK>
 __device__ __forceinline__ bool gp_tile(const int32_t* __restrict__ offsets, int n_exp, int n_rtiles, int& mtile,
                                         int& rtile) {
   const int lane = threadIdx.x & 63;
   int m = 0;  // pair tiles of every expert
   for (int base = 0; base < n_exp; base += 64) {
     const int ee = base + lane;
-    m += ee < n_exp ? (offsets[ee + 1] - offsets[ee] + gp::kTok - 1) / gp::kTok : 0;
+    m += ee < n_exp ? (offsets[ee + 1] - offsets[ee] + TOK - 1) / TOK : 0;
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) m += __shfl_xor(m, off, 64);
   m = __builtin_amdgcn_readfirstlane(m);
   const int L = blockIdx.x, xcd = L % gp::kXcds, slot = L / gp::kXcds;
-  const int per = (m + gp::kXcds - 1) / gp::kXcds;
-  const int local = slot / n_rtiles;
-  mtile = xcd * per + local;
-  rtile = slot % n_rtiles;
-  return local < per && mtile < m;
+  const int per = (m * n_rtiles + gp::kXcds - 1) / gp::kXcds;
+  const int idx = xcd * per + slot;
+  mtile = idx / n_rtiles;
+  rtile = idx % n_rtiles;
+  return slot < per && mtile < m;
 }
 
-// One K step of a wave: 4 row blocks x 4 pair blocks x 4 substeps of
-// v_mfma_f32_16x16x32_bf16.  wq: the lane's two words of its 4 row blocks;
-// xsb: the step's x' in the swizzled layout (pair col0 + 16 nb + r16 has
-// p % 16 == r16).
-__device__ __forceinline__ void gp_step(const uint2 (&wq)[4], const uint32_t* __restrict__ xsb,
-                                        int g, int r16, int col0, f32x4_t (&acc)[4][4],
-                                        const ExpandConsts& kc) {
+// One K step of a wave: RB row blocks x NB pair blocks x 2 pieces of
+// v_mfma_scale_f32_16x16x128_f8f6f4.  a: the lane's two words of its row
+// blocks, expanded; xsb, ssb: the step's mx rows in the swizzled layout (pair
+// 16 nb + r16 has p % 16 == r16) and their scale words.
+// send issues the next step's copies and loads, behind the first products: the
+// matrix unit works while their addresses are formed.
+template <int RB, int NB, typename F>
+__device__ __forceinline__ void gp_step(const uint32_t (&a)[RB][4], const uint32_t* __restrict__ xsb,
+                                        const uint32_t* __restrict__ ssb, int g, int r16,
+                                        mx_f32x4_t (&acc)[RB][NB], F&& send) {
+  // byte offset of chunk g of column r16: chunk c + g of the same column
+  // is at that offset ^ 16 c (c a multiple of 4), 16 columns on 4 KB further.
+  // (Recomputed each step: hoisted out of the loop, the sixteen addresses cost
+  // the registers the products need.)
+  uint32_t off = static_cast<uint32_t>(r16 * gp::kChunks + (g ^ r16)) * 16;
+  uint32_t soff = static_cast<uint32_t>(r16) * 4 + g;
+  asm volatile("" : "+v"(off), "+v"(soff));
+  auto read = [&](int i) {  // piece i % 2 of pair block i / 2
+    const char* xc = reinterpret_cast<const char*>(xsb) + 4096 * (i / 2);
+    return mx_operand(*reinterpret_cast<const uint4*>(xc + (off ^ (128 * (i % 2)))),
+                      *reinterpret_cast<const uint4*>(xc + (off ^ (128 * (i % 2) + 64))));
+  };
+  // One block's reads go out ahead of the previous one's products, and no
+  // further: hoisted to the top of the step, all of them need more registers
+  // than there are.
+  int sb = reinterpret_cast<const uint8_t*>(ssb)[soff];
+  i32x8_t b = read(0);
 #pragma unroll
-  for (int ww = 0; ww < 2; ++ww) {
+  for (int i = 0; i < NB * gp::kPieces; ++i) {
+    const int nb = i / 2, p = i % 2;
+    i32x8_t bn = b;
+    int sn = sb;
+    if (i + 1 < NB * gp::kPieces) bn = read(i + 1);
+    if (p == 1 && nb + 1 < NB) sn = reinterpret_cast<const uint8_t*>(ssb)[soff + 64 * (nb + 1)];
+    MA_ISSUE_FENCE();
 #pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const int c = (2 * g + ww) * 2 + hh;
-      uint4 b[4];
+    for (int mb = 0; mb < RB; ++mb) acc[mb][nb] = mx_mfma_fp4(a[mb], b, acc[mb][nb], mx_piece_scale(p), sb);
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb)
-        b[nb] = *reinterpret_cast<const uint4*>(xsb + ((col0 + nb * 16 + r16) * 16 + (c ^ r16)) * 4);
+    for (int mb = 0; mb < RB; mb += 4) mx_pin(acc[mb][nb], acc[mb + 1][nb], acc[mb + 2][nb], acc[mb + 3][nb]);
+    if (i == 0) {
+      MA_ISSUE_FENCE();
+      send();
+      MA_ISSUE_FENCE();
+    }
+    b = bn;
+    sb = sn;
+  }
+}
+
+// A step's copies: copy i of thread tid fills slot S = tid + threads * i (so
+// each wave's copy i fills 64 consecutive slots, as the LDS DMA writes them)
+// with chunk c = (S % 16) ^ (p % 16) of pair p = S / 16; then the pairs' scale
+// words, one by each of the first TOK threads.  rows[p] is pair p's row in
+// base (16 nsteps chunks a row, nsteps scale words a row).
+typedef __attribute__((address_space(3))) void* lds_void_t;
+template <int TOK>
+struct GpDma {
+  using T = gp::Tile<TOK>;
+  const uint4* base;        // the same in every lane
+  uint32_t off[T::kCopies];  // copy i's source at step 0, in chunks from base (< 2^32: checked by the host)
+  const uint32_t* scale;    // this thread's scale word of step 0 (threads below TOK)
+
+  __device__ __forceinline__ GpDma(const uint32_t* b, const uint32_t* scales, int64_t nsteps, const int32_t* rows)
+      : base(reinterpret_cast<const uint4*>(b)),
+        scale(scales + static_cast<int64_t>(rows[threadIdx.x % TOK]) * nsteps) {
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb) {
-        const uint4 a = expand_half(ww ? wq[mb].y : wq[mb].x, hh, kc);
-#pragma unroll
-        for (int nb = 0; nb < 4; ++nb) acc[mb][nb] = mfma_bf16(a, b[nb], acc[mb][nb]);
-      }
+    for (int i = 0; i < T::kCopies; ++i) {
+      const int S = threadIdx.x + T::kThreads * i, p = S / 16, c = (S % 16) ^ (p % 16);
+      off[i] = static_cast<uint32_t>(static_cast<int64_t>(rows[p]) * nsteps * gp::kChunks + c);
     }
   }
-}
 
-// A step's x' copies: 2048 slots of 16 B, 4 per thread; copy i of thread tid
-// fills slot S = tid + 512 i (so each wave's copy i fills 64 consecutive
-// slots, as the LDS DMA writes them) with chunk c = (S % 16) ^ (p % 16) of
-// pair p = S / 16.  rows[p] is pair p's row in the uint32 array base (row
-// length ld); src[i] is copy i's source at K word 0.
-// The four offsets live in LDS (soff[thread], read back at each step): in
-// registers they pushed the K loop past its 128 VGPRs, and the compiler
-// reloaded a spilled value from scratch memory at every step.
-struct GpDma {
-  const uint32_t* base;  // the same in every lane
-  const uint4* soff;     // LDS: soff[t].x .. .w = thread t's copy i source at K word 0, in uint32 from base
-                         // (< 2^32: checked by the host)
-};
-__device__ __forceinline__ GpDma gp_dma_sources(const uint32_t* base, int64_t ld, const int32_t* rows,
-                                                uint4* soff) {
-  uint32_t o[4];
+  // The copies of step k into the LDS buffers (in flight until the issuing
+  // wave's vector memory counter drains).
+  __device__ __forceinline__ void copy(int64_t k, uint32_t* xsb, uint32_t* ssb) const {
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int S = threadIdx.x + gp::kThreads * i, p = S / 16, c = (S % 16) ^ (p % 16);
-    o[i] = static_cast<uint32_t>(static_cast<int64_t>(rows[p]) * ld + (c >> 1) * 8 + 4 * (c & 1));
+    for (int i = 0; i < T::kCopies; ++i)
+      __builtin_amdgcn_global_load_lds(base + k * gp::kChunks + off[i],
+                                       (lds_void_t)(xsb + 4 * (64 * wv + T::kThreads * i)), 16, 0, 0);
+    if (64 * wv < TOK && threadIdx.x < TOK)
+      __builtin_amdgcn_global_load_lds(scale + k, (lds_void_t)(ssb + 64 * wv), 4, 0, 0);
   }
-  soff[threadIdx.x] = make_uint4(o[0], o[1], o[2], o[3]);  // read back only by this thread
-  return GpDma{base, soff};
-}
-typedef __attribute__((address_space(3))) void* lds_void_t;
-// s_waitcnt immediate (gfx9 encoding): vmcnt(4), expcnt and lgkmcnt left open.
-constexpr int kVmcnt4 = 0x4 | (0x7 << 4) | (0xF << 8);
-// vmcnt(4) and lgkmcnt(0), expcnt left open.
-constexpr int kVmcnt4Lgkm0 = 0x4 | (0x7 << 4);
+};
+// s_waitcnt immediate (gfx9 encoding): vmcnt(n) and lgkmcnt(0), expcnt left open.
+constexpr int gp_vmcnt(int n) { return n | (0x7 << 4); }
 
-// The copies of the step at K word k0 into the LDS buffer xsb (in flight
-// until the issuing wave's vector memory counter drains).
-__device__ __forceinline__ void gp_dma(const GpDma& d, int64_t k0, uint32_t* xsb) {
-  const int wv = threadIdx.x >> 6;
-  const uint4 o4 = d.soff[threadIdx.x];
-  const uint32_t off[4] = {o4.x, o4.y, o4.z, o4.w};
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-    __builtin_amdgcn_global_load_lds(d.base + off[i] + k0 * 8,
-                                     (lds_void_t)(xsb + 4 * (64 * wv + gp::kThreads * i)), 16, 0, 0);
-}
-
-// One step of the K loop: take this step's weights out of w, issue the next
-// step's x' copies into ``nxt`` (if there is a next step) and its weights
-// into w, then this step's MFMAs on ``cur``, then wait for the copies and
-// meet at the barrier.  The weights move to their own registers at the top,
-// after the wait that covers their loads: a copy at the end of the step
-// would have to wait for the loads just issued, in the middle of the step.
-__device__ __forceinline__ void gp_kstep(const uint32_t* rp, const int64_t (&moff)[4], int64_t k0, int64_t nwk,
-                                         const GpDma& d, const uint32_t* cur, uint32_t* nxt,
-                                         uint2 (&w)[4], int g, int r16, int col0, f32x4_t (&acc)[4][4],
-                                         const ExpandConsts& kc) {
+// One step of the K loop: expand this step's weights, issue the next step's
+// copies into the other buffers (if there is a next step) and, in an odd step,
+// the next two steps' weights into w, with this step's MFMAs, then wait for the
+// copies and meet at the barrier.
+template <int TOK, bool ODD>
+__device__ __forceinline__ void gp_kstep(const uint32_t* rp, uint32_t loff, const int64_t (&moff)[gp::Tile<TOK>::kRb],
+                                         int64_t k, int64_t nsteps, const GpDma<TOK>& d, const uint32_t* cur,
+                                         const uint32_t* cur_s, uint32_t* nxt, uint32_t* nxt_s,
+                                         uint4 (&w)[gp::Tile<TOK>::kRb], int g, int r16,
+                                         mx_f32x4_t (&acc)[gp::Tile<TOK>::kRb][gp::Tile<TOK>::kNb]) {
   using namespace gp;
-  const int64_t kn = k0 + kWords < nwk ? k0 + kWords : k0;
-  // This step's weights (loaded during the last step) are in: nothing else
-  // is outstanding, so the copies and loads below are all this wave has in
-  // flight during the MFMAs.
+  constexpr int RB = Tile<TOK>::kRb;
+  // This step's weights are in (an even step's were loaded during the last):
+  // nothing else is outstanding, so the copies and loads below are all this
+  // wave has in flight during the MFMAs.
   __builtin_amdgcn_s_waitcnt(0);
   MA_ISSUE_FENCE();
-  uint2 wq[4];
+  uint32_t a[RB][4];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb) wq[mb] = w[mb];
+  for (int mb = 0; mb < RB; ++mb) mx_expand2(ODD ? make_uint2(w[mb].z, w[mb].w) : make_uint2(w[mb].x, w[mb].y), a[mb]);
   MA_ISSUE_FENCE();
-  if (k0 + kWords < nwk) gp_dma(d, kn, nxt);
-  MA_ISSUE_FENCE();  // the copies are issued before the weights
+  gp_step<RB, Tile<TOK>::kNb>(a, cur, cur_s, g, r16, acc, [&]() {
+    if (!ODD || k + 1 < nsteps) d.copy(k + 1, nxt, nxt_s);
+    if constexpr (ODD) {
+      MA_ISSUE_FENCE();  // the copies are issued before the weights
+      const int64_t kn = k + 1 < nsteps ? k + 1 : k - 1;
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb) w[mb] = *reinterpret_cast<const uint2*>(rp + moff[mb] + kn);
-  MA_ISSUE_FENCE();  // the next step's loads go out before this step's MFMAs
-  gp_step(wq, cur, g, r16, col0, acc, kc);
-  // This wave's copies have landed: at most the 4 weight loads issued after
+      for (int mb = 0; mb < RB; ++mb) w[mb] = *reinterpret_cast<const uint4*>(rp + moff[mb] + kn * kWords + loff);
+    }
+  });
+  // This wave's copies have landed: at most the weight loads issued after
   // them are outstanding (vector memory completes in issue order); those
   // are waited for where the next step uses them.
-  __builtin_amdgcn_s_waitcnt(kVmcnt4Lgkm0);
+  __builtin_amdgcn_s_waitcnt(gp_vmcnt(ODD ? RB : 0));
   // The next buffer is in and this one is free to refill once every wave is
   // here.  A plain barrier: __syncthreads' fence would also wait for the
   // weight loads just issued (it drains every outstanding write to LDS, and
@@ -901,168 +915,198 @@ __device__ __forceinline__ void gp_kstep(const uint32_t* rp, const int64_t (&mof
   MA_ISSUE_FENCE();
 }
 
-// The K loop shared by both stages: acc += W x x', the lane's weight row of
-// block mb at rp + moff[mb] (moff the same in every lane; nwk words), the
-// pairs' x' rows in d; weights one step ahead in registers, x' one step ahead
-// by DMA into the other LDS buffer.  The two buffers are distinct arrays and
-// the loop is unrolled by two, so the compiler sees that a step's LDS reads
-// and the copies in flight into the other buffer do not overlap (it would
-// otherwise wait for the copies before the reads).
-__device__ __forceinline__ void gp_kloop(const uint32_t* rp, const int64_t (&moff)[4], int64_t nwk, const GpDma& d,
-                                         uint32_t* xa, uint32_t* xb, int g, int r16, int col0,
-                                         f32x4_t (&acc)[4][4]) {
+// The K loop shared by both stages: acc += W x, the lane's weight row of
+// block mb at rp + moff[mb] + loff (rp and moff the same in every lane; nwk
+// words), the pairs' mx rows in d; weights one step ahead in registers, mx rows
+// one step ahead by DMA into the other LDS buffer.  The two buffers are
+// distinct arrays and the loop is unrolled by two, so the compiler sees that a
+// step's LDS reads and the copies in flight into the other buffer do not
+// overlap (it would otherwise wait for the copies before the reads).
+template <int TOK>
+__device__ __forceinline__ void gp_kloop(const uint32_t* rp, uint32_t loff, const int64_t (&moff)[gp::Tile<TOK>::kRb],
+                                         int64_t nwk, const GpDma<TOK>& d, uint32_t* xa, uint32_t* xb, uint32_t* sa,
+                                         uint32_t* sb, int g, int r16,
+                                         mx_f32x4_t (&acc)[gp::Tile<TOK>::kRb][gp::Tile<TOK>::kNb]) {
   using namespace gp;
-  const ExpandConsts kc;
-  uint2 wq[4];
+  constexpr int RB = Tile<TOK>::kRb;
+  const int64_t nsteps = nwk / kWords;
+  uint4 w[RB];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb) wq[mb] = *reinterpret_cast<const uint2*>(rp + moff[mb]);
-  gp_dma(d, 0, xa);
+  for (int mb = 0; mb < RB; ++mb) w[mb] = *reinterpret_cast<const uint4*>(rp + moff[mb] + loff);
+  d.copy(0, xa, sa);
   __builtin_amdgcn_s_waitcnt(0);  // this wave's copies have landed
   __syncthreads();                // and every other wave's
-  for (int64_t k0 = 0; k0 < nwk; k0 += 2 * kWords) {
-    gp_kstep(rp, moff, k0, nwk, d, xa, xb, wq, g, r16, col0, acc, kc);
-    if (k0 + kWords < nwk) gp_kstep(rp, moff, k0 + kWords, nwk, d, xb, xa, wq, g, r16, col0, acc, kc);
+  for (int64_t k = 0; k < nsteps; k += 2) {  // K is a multiple of 256: nsteps is even
+    gp_kstep<TOK, false>(rp, loff, moff, k, nsteps, d, xa, sa, xb, sb, w, g, r16, acc);
+    gp_kstep<TOK, true>(rp, loff, moff, k + 1, nsteps, d, xb, sb, xa, sa, w, g, r16, acc);
   }
 }
 
 // SwiGLU stage: h = SwiGLU(up, gate) of 128 outputs (rows [o, o+128) of the
-// up half and the matching gate rows) for a tile of 128 pairs of expert e,
-// rounded to bf16 and written in the x' pair layout the down stage reads (hp)
-// and optionally in slot order (h); hcorr[pos * n_rtiles + rtile] gets the
-// tile's part of the down stage's correction sum (f + 1) h.
-template <int ADT>
-__global__ __launch_bounds__(gp::kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_gp_swiglu(
-    const uint32_t* __restrict__ xp, const float* __restrict__ xc, int64_t topk,
+// up half and the matching gate rows) for a tile of TOK pairs of expert e,
+// rounded to bf16 and written as half of steps 2 (rtile / 2) and 2 (rtile / 2)
+// + 1 of the pair's mx row (hp, scale words hs) and optionally in slot order (h); hcorr[pos * n_rtiles + rtile]
+// gets the tile's part of the down stage's correction sum h.
+template <int ADT, int TOK>
+__global__ __launch_bounds__(gp::Tile<TOK>::kThreads) __attribute__((amdgpu_waves_per_eu(gp::Tile<TOK>::kWaves, gp::Tile<TOK>::kWaves))) void k_gp_swiglu(
+    const uint32_t* __restrict__ xq, const uint32_t* __restrict__ xs, const float2* __restrict__ xc, int64_t topk,
     const uint32_t* __restrict__ w, int64_t n_half, int64_t nwords,
     const void* __restrict__ alpha, const int32_t* __restrict__ offsets,
-    const int32_t* __restrict__ pair_ids, int n_exp, uint16_t* __restrict__ hp,
+    const int32_t* __restrict__ pair_ids, int n_exp, uint16_t* __restrict__ hp, uint32_t* __restrict__ hs,
     float* __restrict__ hcorr, uint16_t* __restrict__ h, int64_t ldh) {
   using namespace gp;
-  __shared__ __align__(16) uint32_t xa[kXaDwords];
-  __shared__ __align__(16) uint32_t xb[kXsDwords];
+  using T = Tile<TOK>;
+  constexpr int kTok = TOK, kThreads = T::kThreads, RB = T::kRb, NB = T::kNb;
+  __shared__ __align__(16) uint32_t xa[T::kXaDwords];
+  __shared__ __align__(16) uint32_t xb[T::kXsDwords];
+  __shared__ uint32_t sa[kTok], sb[kTok], hsc[kTok];
   __shared__ float cst[kTok], hcp[4][kTok];
   __shared__ int32_t tokrow[kTok], pid[kTok];
-  __shared__ uint4 dsoff[kThreads];
   const int n_rtiles = static_cast<int>((n_half + kRows / 2 - 1) / (kRows / 2));
   int mtile, rtile;
-  if (!gp_tile(offsets, n_exp, n_rtiles, mtile, rtile)) return;
+  if (!gp_tile<TOK>(offsets, n_exp, n_rtiles, mtile, rtile)) return;
   int e, pos0, np;
   if (!decode_tile(offsets, n_exp, mtile, kTok, e, pos0, np)) return;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int wr = wv & 3, wm = wv >> 2, r16 = lane & 15, g = lane >> 4;
+  e = __builtin_amdgcn_readfirstlane(e);  // the same in every lane: the weights' addresses stay scalar
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
   if (tid < kTok) {
     const int p = tid < np ? pair_ids[pos0 + tid] : -1;
     pid[tid] = p;
     const int t = p >= 0 ? static_cast<int>(p / topk) : 0;
     tokrow[tid] = t;
-    cst[tid] = p >= 0 ? xc[t] : 0.f;
+    cst[tid] = p >= 0 ? xc[t].x : 0.f;
   }
-  const int64_t o0 = static_cast<int64_t>(rtile) * (kRows / 2) + wr * 32;  // this wave's first output
+  const int64_t o0 = static_cast<int64_t>(rtile) * (kRows / 2) + wv * 8 * RB;  // this wave's first output
   const uint32_t* we = w + static_cast<int64_t>(e) * 2 * n_half * nwords;
   // (n_half % 128 == 0: every row of the tile exists)
-  const uint32_t* rp = we + (o0 + r16) * nwords + 2 * g;
-  int64_t moff[4];
+  const uint32_t* rp = we + o0 * nwords;
+  const uint32_t loff = static_cast<uint32_t>(r16 * nwords + 4 * g);
+  int64_t moff[RB];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb) moff[mb] = (16 * (mb & 1) + (mb >> 1) * n_half) * nwords;
+  for (int mb = 0; mb < RB; ++mb) moff[mb] = (16 * (mb % (RB / 2)) + (mb / (RB / 2)) * n_half) * nwords;
   __syncthreads();  // tokrow
-  const GpDma xsrc = gp_dma_sources(xp, nwords * 8, tokrow, dsoff);
-  f32x4_t acc[4][4];
+  const GpDma<TOK> xsrc(xq, xs, nwords / kWords, tokrow);
+  mx_f32x4_t acc[RB][NB];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
+  for (int mb = 0; mb < RB; ++mb)
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) acc[mb][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  gp_kloop(rp, moff, nwords, xsrc, xa, xb, g, r16, wm * 64, acc);
+    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = mx_f32x4_t{0.f, 0.f, 0.f, 0.f};
+  gp_kloop<TOK>(rp, loff, moff, nwords, xsrc, xa, xb, sa, sb, g, r16, acc);
   // Epilogue: lane (r16, g) of row block mb holds rows 4g..4g+3 of the block
-  // for pair column wm*64 + nb*16 + r16.  h goes to LDS in the x' pair layout
-  // of its 8 words (the loop's last barrier has freed the LDS), then out in
-  // 16-byte pieces, each pair's 256 bytes contiguous.
-  // Output i = o0 + 16 mb + 4 g + r (< n_half: n_half % 128 == 0) sits at
-  // position 4 g + r of its 16-output word, i.e. pair j = (4 g + r) & 7 (so
-  // pair_scale(j) = pair_scale(r)), half g >> 1, word 2 wr + mb of the tile.
-  uint16_t* hst = reinterpret_cast<uint16_t*>(xa);
-  const int64_t otile = static_cast<int64_t>(rtile) * (kRows / 2);
+  // for pair column 16 nb + r16.  h goes to LDS as its parts of two steps of
+  // its mx row (the loop's last barrier has freed the LDS), then out in 16-byte
+  // pieces, each pair's in runs of 64 bytes.  Output i = o0 + 16 mb + 4 g + r
+  // (< n_half: n_half % 128 == 0) is value 4 g + r of a word: byte 2 g + r / 2
+  // of its 16 bytes, + 8 for odd r.  The wave's 32 outputs are words 2 wv and
+  // 2 wv + 1 of the tile's 8, so block 2 (rtile & 1) + wv / 2 of step wv & 1 of
+  // the two: in LDS byte 128 (wv & 1) + 64 piece + 32 (wv / 2) of the pair's row.
+  uint8_t* hst = reinterpret_cast<uint8_t*>(xa);
   const int64_t abase = static_cast<int64_t>(e) * 2 * n_half;
-  float au[2][4], ag[2][4];
 #pragma unroll
-  for (int mb = 0; mb < 2; ++mb)
+  for (int q = 0; q < RB / 4; ++q) {
+    const int blk = (wv & 1) * 2 + wv / 2;
+    float au[2][4], ag[2][4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t i = o0 + 16 * mb + 4 * g + r;
-      au[mb][r] = ld_t<ADT>(alpha, abase + i);
-      ag[mb][r] = ld_t<ADT>(alpha, abase + n_half + i);
-    }
-  float cc[4];
+    for (int m = 0; m < 2; ++m)
 #pragma unroll
-  for (int nb = 0; nb < 4; ++nb) cc[nb] = cst[wm * 64 + nb * 16 + r16];
-  const int hbase = (2 * wr * 8) * 2 + (g >> 1);
-  float hcl[4] = {0.f, 0.f, 0.f, 0.f};
+      for (int r = 0; r < 4; ++r) {
+        const int64_t i = o0 + 32 * q + 16 * m + 4 * g + r;
+        au[m][r] = ld_t<ADT>(alpha, abase + i);
+        ag[m][r] = ld_t<ADT>(alpha, abase + n_half + i);
+      }
 #pragma unroll
-  for (int mb = 0; mb < 2; ++mb) {
+    for (int nb = 0; nb < NB; ++nb) {
+      const int col = nb * 16 + r16;
+      const float cc = cst[col];
+      float hv[2][4], hsum = 0.f;
+      uint32_t ex = 0;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int j = (4 * g + r) & 7;
-      const float f = pair_scale(r);
-      const int hoff = hbase + (mb * 8 + j) * 2;
+      for (int m = 0; m < 2; ++m)
 #pragma unroll
-      for (int nb = 0; nb < 4; ++nb) {
-        const int col = wm * 64 + nb * 16 + r16;
-        const float up = au[mb][r] * (acc[mb][nb][r] - cc[nb]);
-        const float gt = ag[mb][r] * (acc[mb + 2][nb][r] - cc[nb]);
-        const uint16_t hb = f32_to_bf16(swiglu_act(up, gt));
-        const float hv = bf16_to_f32(hb);
-        hst[col * kHRow + hoff] = static_cast<uint16_t>(bf16_bits_exact(hv * f));  // exact: power-of-two scale
-        // (+0.0 for the pad columns: hcl starts at +0.0, so no sum changes)
-        hcl[nb] += col < np ? (f + 1.0f) * hv : 0.0f;
-        if (h) {
-          if (col < np) h[static_cast<int64_t>(pid[col]) * ldh + o0 + 16 * mb + 4 * g + r] = hb;
+        for (int r = 0; r < 4; ++r) {
+          const float up = au[m][r] * (acc[2 * q + m][nb][r] - cc);
+          const float gt = ag[m][r] * (acc[RB / 2 + 2 * q + m][nb][r] - cc);
+          const uint16_t hb = f32_to_bf16(swiglu_act(up, gt));
+          hv[m][r] = bf16_to_f32(hb);
+          hsum += hv[m][r];
+          ex = mx_exponent(ex, hv[m][r]);
+          if (h) {
+            if (col < np) h[static_cast<int64_t>(pid[col]) * ldh + o0 + 32 * q + 16 * m + 4 * g + r] = hb;
+          }
         }
+      // over the lane groups: the block's exponent and sum
+      uint32_t eo = __shfl_xor(ex, 16, 64);
+      ex = ex > eo ? ex : eo;
+      eo = __shfl_xor(ex, 32, 64);
+      ex = ex > eo ? ex : eo;
+      hsum += __shfl_xor(hsum, 16, 64);
+      hsum += __shfl_xor(hsum, 32, 64);
+      const float f = mx_factor(ex);
+#pragma unroll
+      for (int m = 0; m < 2; ++m) {
+        float v[4] = {hv[m][0] * f, hv[m][2] * f, hv[m][1] * f, hv[m][3] * f};
+#pragma unroll
+        for (int p = 0; p < kPieces; ++p) {
+          const uint32_t w4 = mx_piece4(v);
+          uint16_t* dst = reinterpret_cast<uint16_t*>(hst + col * kHRow + 128 * (wv & 1) + 64 * p + 32 * (wv / 2) + 16 * m + 2 * g);
+          dst[0] = static_cast<uint16_t>(w4);
+          dst[4] = static_cast<uint16_t>(w4 >> 16);
+        }
+      }
+      if (g == 0) {
+        hcp[blk][col] = hsum;
+        reinterpret_cast<uint8_t*>(hsc + col)[blk] = static_cast<uint8_t>(mx_scale_byte(ex));
       }
     }
   }
-  // the tile's correction part per pair: lane groups, then row waves, in order
-#pragma unroll
-  for (int nb = 0; nb < 4; ++nb) {
-    float v = hcl[nb];
-    v += __shfl_xor(v, 16, 64);
-    v += __shfl_xor(v, 32, 64);
-    if (g == 0) hcp[wr][wm * 64 + nb * 16 + r16] = v;
-  }
   __syncthreads();
+  // the tile's correction part per pair: blocks in order
   if (tid < np) {
     const float v = ((hcp[0][tid] + hcp[1][tid]) + hcp[2][tid]) + hcp[3][tid];
     hcorr[static_cast<int64_t>(pos0 + tid) * n_rtiles + rtile] = v;
   }
-  // the tile's h (n_half % 128 == 0: whole words), 16 B per copy
+  // the scale bytes of the tile's two blocks of each step
+  if (tid < 2 * np) {
+    const int col = tid >> 1, st = tid & 1;
+    reinterpret_cast<uint16_t*>(hs + static_cast<int64_t>(pos0 + col) * n_rtiles + (rtile & ~1) + st)[rtile & 1] =
+        reinterpret_cast<const uint16_t*>(hsc + col)[st];
+  }
+  // the tile's h (n_half % 256 == 0: whole pairs of steps), 16 B per copy
 #pragma unroll
   for (int k = 0; k < kTok * 16 / kThreads; ++k) {
     const int c = tid + kThreads * k, col = c / 16, part = c % 16;
     if (col < np)
-      *reinterpret_cast<uint4*>(hp + static_cast<int64_t>(pos0 + col) * n_half + otile + part * 8) =
-          *reinterpret_cast<const uint4*>(hst + col * kHRow + part * 8);
+      *reinterpret_cast<uint4*>(hp + (static_cast<int64_t>(pos0 + col) * n_rtiles + (rtile & ~1) + part / 8) * kMxStep +
+                                64 * (part / 4 & 1) + 32 * (rtile & 1) + 8 * (part & 3)) =
+          *reinterpret_cast<const uint4*>(hst + col * kHRow + part * 16);
   }
 }
 
 // Down stage: out[pos, n] = bf16(alpha[e, n] * sum_k (c - 1) h) for a tile of
-// 128 pairs and 256 output rows; the correction is the sum of the SwiGLU
+// TOK pairs and 256 output rows; the correction is the sum of the SwiGLU
 // stage's n_ctiles parts, added in tile order.
-template <int ADT>
-__global__ __launch_bounds__(gp::kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_gp_down(
-    const uint32_t* __restrict__ hp, const float* __restrict__ hcorr, int n_ctiles,
+template <int ADT, int TOK>
+__global__ __launch_bounds__(gp::Tile<TOK>::kThreads) __attribute__((amdgpu_waves_per_eu(gp::Tile<TOK>::kWaves, gp::Tile<TOK>::kWaves))) void k_gp_down(
+    const uint32_t* __restrict__ hp, const uint32_t* __restrict__ hs, const float* __restrict__ hcorr, int n_ctiles,
     const uint32_t* __restrict__ w, int64_t n_out, int64_t nwk, const void* __restrict__ alpha,
     const int32_t* __restrict__ offsets, int n_exp, uint16_t* __restrict__ out) {
   using namespace gp;
-  __shared__ __align__(16) uint32_t xa[kXaDwords];
-  __shared__ __align__(16) uint32_t xb[kXsDwords];
+  using T = Tile<TOK>;
+  constexpr int kTok = TOK, kThreads = T::kThreads, RB = T::kRb, NB = T::kNb;
+  __shared__ __align__(16) uint32_t xa[T::kXaDwords];
+  __shared__ __align__(16) uint32_t xb[T::kXsDwords];
+  __shared__ uint32_t sa[kTok], sb[kTok];
   __shared__ float cst[kTok];
   __shared__ int32_t prow[kTok];
-  __shared__ uint4 dsoff[kThreads];
   const int n_rtiles = static_cast<int>((n_out + kRows - 1) / kRows);
   int mtile, rtile;
-  if (!gp_tile(offsets, n_exp, n_rtiles, mtile, rtile)) return;
+  if (!gp_tile<TOK>(offsets, n_exp, n_rtiles, mtile, rtile)) return;
   int e, pos0, np;
   if (!decode_tile(offsets, n_exp, mtile, kTok, e, pos0, np)) return;
-  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int wr = wv & 3, wm = wv >> 2, r16 = lane & 15, g = lane >> 4;
+  e = __builtin_amdgcn_readfirstlane(e);  // the same in every lane: the weights' addresses stay scalar
+  const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
   if (tid < kTok) {
     float c = 0.f;
     if (tid < np)
@@ -1070,49 +1114,50 @@ __global__ __launch_bounds__(gp::kThreads) __attribute__((amdgpu_waves_per_eu(4,
     cst[tid] = c;
     prow[tid] = pos0 + (tid < np ? tid : np - 1);
   }
-  const int64_t n0 = static_cast<int64_t>(rtile) * kRows + wr * 64;
+  const int64_t n0 = static_cast<int64_t>(rtile) * kRows + wv * 16 * RB;
   const uint32_t* we = w + static_cast<int64_t>(e) * n_out * nwk;
   // (n_out % 256 == 0: every row of the tile exists)
-  const uint32_t* rp = we + (n0 + r16) * nwk + 2 * g;
-  int64_t moff[4];
+  const uint32_t* rp = we + n0 * nwk;
+  const uint32_t loff = static_cast<uint32_t>(r16 * nwk + 4 * g);
+  int64_t moff[RB];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb) moff[mb] = 16 * mb * nwk;
+  for (int mb = 0; mb < RB; ++mb) moff[mb] = 16 * mb * nwk;
   __syncthreads();  // prow
-  const GpDma xsrc = gp_dma_sources(hp, nwk * 8, prow, dsoff);
-  f32x4_t acc[4][4];
+  const GpDma<TOK> xsrc(hp, hs, nwk / kWords, prow);
+  mx_f32x4_t acc[RB][NB];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb)
+  for (int mb = 0; mb < RB; ++mb)
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) acc[mb][nb] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  gp_kloop(rp, moff, nwk, xsrc, xa, xb, g, r16, wm * 64, acc);
+    for (int nb = 0; nb < NB; ++nb) acc[mb][nb] = mx_f32x4_t{0.f, 0.f, 0.f, 0.f};
+  gp_kloop<TOK>(rp, loff, moff, nwk, xsrc, xa, xb, sa, sb, g, r16, acc);
   // The tile goes out through LDS buffer A as [pair][256 rows], half of the
-  // pairs at a time (the waves holding them write, then every thread copies
-  // them out in 16-byte pieces, each pair's 512 bytes contiguous; n_out % 256
-  // == 0).  The loop's last barrier has freed the buffer.
-  uint2 v[4][4];
+  // pairs at a time (every wave writes its rows, then every thread copies them
+  // out in 16-byte pieces, each pair's 512 bytes contiguous; n_out % 256 == 0).
+  // The loop's last barrier has freed the buffer.
+  uint2 v[RB][NB];
 #pragma unroll
-  for (int mb = 0; mb < 4; ++mb) {
+  for (int mb = 0; mb < RB; ++mb) {
     const int64_t n = n0 + 16 * mb + 4 * g;
     float a[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) a[r] = ld_t<ADT>(alpha, static_cast<int64_t>(e) * n_out + (n + r < n_out ? n + r : n_out - 1));
 #pragma unroll
-    for (int nb = 0; nb < 4; ++nb) {
-      const float c = cst[wm * 64 + nb * 16 + r16];
+    for (int nb = 0; nb < NB; ++nb) {
+      const float c = cst[nb * 16 + r16];
       v[mb][nb].x = pack_bf16x2_rn(a[0] * (acc[mb][nb][0] - c), a[1] * (acc[mb][nb][1] - c));
       v[mb][nb].y = pack_bf16x2_rn(a[2] * (acc[mb][nb][2] - c), a[3] * (acc[mb][nb][3] - c));
     }
   }
   uint16_t* ost = reinterpret_cast<uint16_t*>(xa);
   const int64_t ntile0 = static_cast<int64_t>(rtile) * kRows;
+#pragma unroll
   for (int half = 0; half < 2; ++half) {
-    if (wm == half) {
 #pragma unroll
-      for (int mb = 0; mb < 4; ++mb)
+    for (int mb = 0; mb < RB; ++mb)
 #pragma unroll
-        for (int nb = 0; nb < 4; ++nb)
-          *reinterpret_cast<uint2*>(ost + (nb * 16 + r16) * kORow + wr * 64 + 16 * mb + 4 * g) = v[mb][nb];
-    }
+      for (int nb = 0; nb < NB / 2; ++nb)
+        *reinterpret_cast<uint2*>(ost + (nb * 16 + r16) * kORow + wv * 16 * RB + 16 * mb + 4 * g) =
+            v[mb][half * (NB / 2) + nb];
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < kTok / 2 * 32 / kThreads; ++k) {
@@ -1132,21 +1177,26 @@ using namespace ma;
 // Up to this many pairs per expert on average (decode batches) the K-split
 // kernels run; above it (prefill) the LDS-staged tiles of up to 64 pairs.
 constexpr int64_t kKsMaxPairsPerExpert = 16;
+// Up to this many the prefill form's tiles hold 32 pairs instead of 64 (64
+// experts: at 64 pairs an expert 94 against 97 us a block, at 96 104 against
+// 121; 256 experts at 64 209 against 243).
+constexpr int64_t kSmallTilePairsPerExpert = 48;
 
 static size_t align256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
 
-// Workspace of one call: pair-format h [P, inter] bf16, per-pair down outputs
-// [P, hidden] bf16; in the prefill form also the x' pairs of the tokens
-// [T, hidden / 2] uint32, their corrections [T] float32 and the SwiGLU tiles'
-// correction parts [P, inter / 128] float32.
+// Workspace of one call: h [P, inter] in 16 bits a value (pairs, or mx rows),
+// per-pair down outputs [P, hidden] bf16; in the prefill form also the mx rows
+// of the tokens (2 bytes a value), their sums and scale words, and h's scale
+// words and the SwiGLU tiles' correction parts [P, inter / 128].
 static bool grouped_prefill_form(int64_t n_pairs, int64_t n_experts) {
   return n_pairs > kKsMaxPairsPerExpert * n_experts;
 }
 static size_t grouped_bytes(int64_t n_pairs, int64_t tokens, int64_t inter, int64_t hidden, bool prefill) {
   size_t b = align256(static_cast<size_t>(n_pairs) * inter * 2) + align256(static_cast<size_t>(n_pairs) * hidden * 2);
   if (prefill)
-    b += align256(static_cast<size_t>(tokens) * hidden * 2) + align256(static_cast<size_t>(tokens) * 4) +
-         align256(static_cast<size_t>(n_pairs) * cdiv(inter, gp::kRows / 2) * 4);
+    b += align256(static_cast<size_t>(tokens) * hidden * 2) + align256(static_cast<size_t>(tokens) * 8) +
+         align256(static_cast<size_t>(tokens) * (hidden / kMxStep) * 4) +
+         2 * align256(static_cast<size_t>(n_pairs) * cdiv(inter, gp::kRows / 2) * 4);
   return b;
 }
 
@@ -1227,40 +1277,42 @@ static int grouped_launch(const void* x, int64_t ldx, const uint32_t* x_pairs, c
 #undef MA_GROUPED_KS
 #undef MA_GROUPED_DOWN
   } else {
-    // prefill: the tokens' x' pairs once (or those of ma_moe_route), then
+    // prefill: the tokens' mx rows once (x_pairs are the decode form's), then
     // tiles of 128 pairs x 256 weight rows.  The tiles' copy sources are
-    // 32-bit uint32 offsets into x' and h.
+    // 32-bit offsets in 16-byte chunks into the mx rows of x and h.
     if (static_cast<uint64_t>(tokens) * hidden / 2 >= (uint64_t{1} << 32) ||
         static_cast<uint64_t>(n_pairs) * inter / 2 >= (uint64_t{1} << 32))
       return fail(MA_EVALUE, "moe_grouped: %lld tokens x hidden %lld (or their pairs x intermediate %lld) "
                   "exceed the 16 GiB the batched kernels address; split the batch",
                   (long long)tokens, (long long)hidden, (long long)inter);
     char* p = reinterpret_cast<char*>(out) + align256(static_cast<size_t>(n_pairs) * hidden * 2);
-    const uint32_t* xpp = x_pairs;
-    const float* xcc = x_corr;
-    if (!x_pairs) {
-      uint32_t* xw = reinterpret_cast<uint32_t*>(p);
-      float* cw = reinterpret_cast<float*>(p + align256(static_cast<size_t>(tokens) * hidden * 2));
-      hipLaunchKernelGGL(k_gp_prep, dim3(static_cast<unsigned>(tokens)), dim3(128), 0, s, xb, ldx, hidden / 16, xw, cw);
-      xpp = xw;
-      xcc = cw;
-    }
-    float* hcorr = reinterpret_cast<float*>(p + align256(static_cast<size_t>(tokens) * hidden * 2) +
-                                            align256(static_cast<size_t>(tokens) * 4));
-    const int64_t mtiles = cdiv(n_pairs, gp::kTok) + n_experts;  // an upper bound
+    auto take = [&p](size_t bytes) {
+      char* q = p;
+      p += align256(bytes);
+      return q;
+    };
+    const int64_t xsteps = hidden / kMxStep, hsteps = cdiv(inter, gp::kRows / 2);
+    uint32_t* xq = reinterpret_cast<uint32_t*>(take(static_cast<size_t>(tokens) * hidden * 2));
+    float2* xc = reinterpret_cast<float2*>(take(static_cast<size_t>(tokens) * 8));
+    uint32_t* xs = reinterpret_cast<uint32_t*>(take(static_cast<size_t>(tokens) * xsteps * 4));
+    uint32_t* hs = reinterpret_cast<uint32_t*>(take(static_cast<size_t>(n_pairs) * hsteps * 4));
+    float* hcorr = reinterpret_cast<float*>(take(static_cast<size_t>(n_pairs) * hsteps * 4));
+    launch_mx_prep_wide(xb, ldx, tokens, hidden / 16, xq, xs, xc, s);
+    const int64_t tok = n_pairs > kSmallTilePairsPerExpert * n_experts ? 64 : 32;
+    const int64_t mtiles = cdiv(n_pairs, tok) + n_experts;  // an upper bound
     const int64_t mt8 = cdiv(mtiles, gp::kXcds) * gp::kXcds;
     const int rt1 = static_cast<int>(cdiv(inter, gp::kRows / 2)), rt2 = static_cast<int>(cdiv(hidden, gp::kRows));
     const dim3 g1(static_cast<unsigned>(mt8 * rt1)), g2(static_cast<unsigned>(mt8 * rt2));
-#define MA_GP(ADT)                                                                                 \
-  hipLaunchKernelGGL((k_gp_swiglu<ADT>), g1, dim3(gp::kThreads), 0, s, xpp, xcc, top_k, up_gate, \
-                     inter, hidden / 16, up_gate_alpha, offsets, pair_ids, ne, hp, hcorr, hb, ldh);  \
-  hipLaunchKernelGGL((k_gp_down<ADT>), g2, dim3(gp::kThreads), 0, s,                              \
-                     reinterpret_cast<const uint32_t*>(hp), hcorr, rt1, down, hidden, inter / 16, \
+#define MA_GP(ADT, TOK)                                                                            \
+  hipLaunchKernelGGL((k_gp_swiglu<ADT, TOK>), g1, dim3(gp::Tile<TOK>::kThreads), 0, s, xq, xs, xc, top_k, up_gate, \
+                     inter, hidden / 16, up_gate_alpha, offsets, pair_ids, ne, hp, hs, hcorr, hb, ldh);  \
+  hipLaunchKernelGGL((k_gp_down<ADT, TOK>), g2, dim3(gp::Tile<TOK>::kThreads), 0, s,               \
+                     reinterpret_cast<const uint32_t*>(hp), hs, hcorr, rt1, down, hidden, inter / 16, \
                      down_alpha, offsets, ne, out);
     if (alpha_dtype == MA_BF16) {
-      MA_GP(MA_BF16)
+      if (tok == 64) { MA_GP(MA_BF16, 64) } else { MA_GP(MA_BF16, 32) }
     } else {
-      MA_GP(MA_F32)
+      if (tok == 64) { MA_GP(MA_F32, 64) } else { MA_GP(MA_F32, 32) }
     }
 #undef MA_GP
   }
@@ -1311,7 +1363,12 @@ extern "C" int ma_moe_grouped(const void* x, int64_t ldx, const uint32_t* x_pair
 // device on that device's first call.
 // ---------------------------------------------------------------------------
 constexpr size_t kGroupedScratchBytes = size_t{16} << 20;
-static __device__ __align__(256) uint8_t scratch[kGroupedScratchBytes];
+// Scale words and the tokens' sums have room of their own: a call counts its
+// rows, outputs and correction parts (grouped_counted_bytes) against the 16
+// MiB.  What the whole layout takes beyond that count is at most 1/32 of it
+// (4 bytes beside each 256 of a row or a pair's h) and some alignment.
+constexpr size_t kGroupedScratchExtra = size_t{1} << 20;
+static __device__ __align__(256) uint8_t scratch[kGroupedScratchBytes + kGroupedScratchExtra];
 
 static void* grouped_scratch_ptr() {
   static std::mutex mu;
@@ -1333,6 +1390,14 @@ static void* grouped_scratch_ptr() {
   return ptrs[dev];
 }
 
+static size_t grouped_counted_bytes(int64_t n_pairs, int64_t tokens, int64_t inter, int64_t hidden, bool prefill) {
+  size_t b = align256(static_cast<size_t>(n_pairs) * inter * 2) + align256(static_cast<size_t>(n_pairs) * hidden * 2);
+  if (prefill)
+    b += align256(static_cast<size_t>(tokens) * hidden * 2) + align256(static_cast<size_t>(tokens) * 4) +
+         align256(static_cast<size_t>(n_pairs) * cdiv(inter, gp::kRows / 2) * 4);
+  return b;
+}
+
 extern "C" size_t ma_moe_grouped_noalloc_max_bytes(void) { return kGroupedScratchBytes; }
 
 extern "C" int ma_moe_grouped_noalloc(const void* x, int64_t ldx, const uint32_t* x_pairs,
@@ -1352,8 +1417,10 @@ extern "C" int ma_moe_grouped_noalloc(const void* x, int64_t ldx, const uint32_t
     return fail(MA_EVALUE, "%s: y is required (the per-pair outputs stay in the internal scratch)", what);
   const int64_t n_pairs = tokens * top_k;
   if (n_pairs == 0) return MA_OK;
-  const size_t need = grouped_bytes(n_pairs, tokens, inter, hidden, grouped_prefill_form(n_pairs, n_experts));
-  if (need > kGroupedScratchBytes)
+  const bool prefill = grouped_prefill_form(n_pairs, n_experts);
+  const size_t need = grouped_counted_bytes(n_pairs, tokens, inter, hidden, prefill);
+  if (need > kGroupedScratchBytes ||
+      grouped_bytes(n_pairs, tokens, inter, hidden, prefill) > sizeof(scratch))
     return fail(MA_EVALUE,
                 "%s: %lld (token, expert) pairs need %zu bytes of staging; the built-in scratch holds %zu "
                 "(use ma_moe_grouped with a workspace)",

@@ -215,6 +215,8 @@ def moe_fused(x: torch.Tensor, layer: MoELayer, top_k: int, residual: torch.Tens
 
 
 ROUTE_MAX_TOKENS = 1024
+# Pairs per expert, on average, up to which ma_moe_grouped takes its decode form.
+GROUPED_DECODE_PAIRS = 16
 
 
 def route_supported(layer: MoELayer, top_k: int, x: torch.Tensor) -> bool:
@@ -375,13 +377,17 @@ def moe_block(x: torch.Tensor, layer: MoELayer, top_k: int, residual: torch.Tens
         return y.reshape(x.shape), ids, wts
     res = None if residual is None else residual.reshape(-1, hidden)
     if plan == "grouped":
-        # the top-k launch also writes the x' pairs that the grouped kernels read: the decode batches'
-        # tile-resident SwiGLU and the prefill form.  (Up to 16 tokens the router alone would be one launch
-        # instead of two, but the SwiGLU that expands x itself costs more: a block of 64 experts takes 35.4
-        # against 37.4 us at 4 tokens and 44.9 against 53.7 at 16, of 256 experts 41.6 against 63.6 and 51.7
-        # against 85.8; at 32 tokens 39.3 against 49.6 us.)
+        # Decode batches: the top-k launch also writes the x' pairs that the tile-resident SwiGLU reads.  (Up to
+        # 16 tokens the router alone would be one launch instead of two, but the SwiGLU that expands x itself
+        # costs more: a block of 64 experts takes 35.4 against 37.4 us at 4 tokens and 44.9 against 53.7 at 16,
+        # of 256 experts 41.6 against 63.6 and 51.7 against 85.8; at 32 tokens 39.3 against 49.6 us.)  The
+        # prefill form reads x in another layout, which its own launch writes.
         xf = xf.contiguous()
-        ids, wts, xp = router_topk(xf, layer.gate_weight, top_k, bias=layer.router_bias, pairs=True)
+        if xf.shape[0] * top_k > GROUPED_DECODE_PAIRS * layer.n_experts:
+            ids, wts = router_topk(xf, layer.gate_weight, top_k, bias=layer.router_bias)
+            xp = None
+        else:
+            ids, wts, xp = router_topk(xf, layer.gate_weight, top_k, bias=layer.router_bias, pairs=True)
         y = moe_grouped(xf, layer, ids, wts, res, x_pairs=xp)
         return y.reshape(x.shape), ids, wts
     ids, wts = router_topk(xf, layer.gate_weight, top_k, bias=layer.router_bias)

@@ -141,6 +141,34 @@ def test_moe_grouped_prefill_form_other_shapes(dev, hidden, n_exp, inter, k, tok
     assert torch.equal(y2, y) and torch.equal(h2, h)
 
 
+@pytest.mark.parametrize("hidden,n_exp,inter,k,tokens,alpha", [
+    (256, 4, 256, 2, 97, torch.bfloat16),   # over 48 pairs an expert: 64-pair tiles; 2 steps a stage
+    (512, 3, 512, 1, 193, torch.float32),   # one slot a token, about one pair past a tile
+    (256, 5, 768, 5, 64, torch.bfloat16),   # every expert holds 64 pairs, one whole tile
+    (1024, 8, 256, 2, 95, torch.float32),   # 32-pair tiles
+    (256, 2, 256, 2, 17, torch.bfloat16)])  # the fewest pairs of the form
+def test_moe_grouped_prefill_tiles_edges(dev, hidden, n_exp, inter, k, tokens, alpha):
+    """The prefill form at the edges of its 32- and 64-pair tiles: h and y against
+    the oracle on the kernel's own routing, the same bits on a second run, and a
+    token with an infinity leaves the others alone."""
+    L = synthetic.make_moe_layer(hidden, n_exp, inter, seed=13, device=dev)
+    L.up_gate_alpha, L.down_alpha = L.up_gate_alpha.to(alpha), L.down_alpha.to(alpha)
+    assert tokens * k > 16 * n_exp  # the prefill form
+    x = synthetic.randn_bf16((tokens, hidden + 8), 600 + tokens, dev)[:, :hidden]
+    ids, wts = router_topk(x, L.gate_weight, k)
+    y, h = moe_grouped(x, L, ids, wts, return_h=True)
+    ref, href = ok.moe_experts(np_f(x), ids.cpu().numpy(), wts.cpu().numpy(), *_oracle_inputs(L))
+    assert_bf16_close(np_f(h), href, what=f"h H={hidden} I={inter} T={tokens}")
+    assert_bf16_close(np_f(y), ref, atol_frac=2.0 ** -7, what=f"y H={hidden} I={inter} T={tokens}")
+    y2, h2 = moe_grouped(x, L, ids, wts, return_h=True)
+    assert torch.equal(y2, y) and torch.equal(h2, h)
+    x = x.clone()
+    x[tokens // 2, 1] = float("inf")
+    z = moe_grouped(x, L, ids, wts)
+    keep = torch.arange(tokens, device=dev) != tokens // 2
+    assert torch.equal(z[keep], y[keep])
+
+
 @pytest.mark.parametrize("n_exp,inter,tokens,alpha", [
     (8, 256, 4, torch.bfloat16), (8, 256, 16, torch.float32), (256, 512, 17, torch.float32),
     (256, 512, 33, torch.bfloat16), (40, 1024, 65, torch.bfloat16), (40, 1280, 20, torch.float32)])
