@@ -48,15 +48,40 @@ __device__ __forceinline__ bool decode_tile(const int32_t* __restrict__ offsets,
                                             int64_t tile, int nt, int& e, int& pos0, int& np) {
   const int lane = threadIdx.x & 63;
   int run = 0;  // tiles of the experts before this 64-expert slice
-  for (int base = 0; base < n_exp; base += 64) {
+  // The first 256 experts' offsets in one round trip (indices past the end read
+  // the last one: no tiles); a load per slice was a round trip each.
+  constexpr int kAhead = 4;
+  int a0[kAhead], a1[kAhead];
+#pragma unroll
+  for (int i = 0; i < kAhead; ++i) {
+    const int ee = 64 * i + lane;
+    a0[i] = offsets[ee < n_exp ? ee : n_exp];
+    a1[i] = offsets[ee + 1 < n_exp ? ee + 1 : n_exp];
+  }
+  // the slice of the tile, by the slices' totals (side by side, where a scan of
+  // one slice after the other is a chain of lane exchanges each)
+  int first = 0;
+  if (n_exp > 64) {
+    int total[kAhead - 1];
+#pragma unroll
+    for (int i = 0; i < kAhead - 1; ++i)
+      total[i] = static_cast<int>(group_sum<64>(static_cast<float>((a1[i] - a0[i] + nt - 1) / nt)));
+#pragma unroll
+    for (int i = 0; i < kAhead - 1; ++i)
+      if (first == 64 * i && 64 * (i + 1) < n_exp && tile >= run + total[i]) {
+        run += total[i];
+        first = 64 * (i + 1);
+      }
+  }
+  for (int base = first; base < n_exp; base += 64) {
     const int ee = base + lane;
-    int tiles = 0;
-    int o0 = 0, o1 = 0;
-    if (ee < n_exp) {
-      o0 = offsets[ee];
-      o1 = offsets[ee + 1];
-      tiles = (o1 - o0 + nt - 1) / nt;
+    int o0 = base == 0 ? a0[0] : base == 64 ? a0[1] : base == 128 ? a0[2] : a0[3];
+    int o1 = base == 0 ? a1[0] : base == 64 ? a1[1] : base == 128 ? a1[2] : a1[3];
+    if (base >= 64 * kAhead) {
+      o0 = offsets[ee < n_exp ? ee : n_exp];
+      o1 = offsets[ee + 1 < n_exp ? ee + 1 : n_exp];
     }
+    const int tiles = (o1 - o0 + nt - 1) / nt;
     int incl = tiles;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -356,272 +381,340 @@ __global__ __launch_bounds__(64 * KW) void k_grouped_down_ks(
 }
 
 // ---------------------------------------------------------------------------
-// Decode form, tile-resident: a workgroup stages its 16-pair tile's B operands
-// for all of K in LDS once (one sync), then each wave takes whole 16-row
-// blocks over all of K: a block's weights for the full K are loaded up front
-// (8 words per lane at K = 2048 ... per chunk of 16 words one uint4), so a
-// wave keeps all its weight bytes in flight at once and needs no cross-wave
-// reduction.  Same per-word arithmetic as the kernels above; each output is
-// one MFMA chain (fixed order).
+// Decode form (few pairs per expert): tiles of 16 pairs whose mx rows (two FP8
+// pieces, mx.h) lie in LDS for all of K, staged once; then each wave takes two
+// blocks of 16 rows over all of K, weights kAhead chunks of 16 words ahead in
+// registers, with no barrier and no reduction across waves.  The codes go in as
+// FP4: three instructions a word where the bf16 operands took twelve, and the
+// products need no spacing by hand.  The SwiGLU stage writes the tile's mx rows
+// of x itself (with every pair's sum), so it needs x alone, and h's like the
+// prefill form; both stages' operands are exact, so a row differs from its
+// float64 value by its bf16 rounding and little else.  Every load of a tile (x
+// or h, scales, sums, the first weights) is issued unconditionally up front, a
+// lane past the tile's end reading its last pair again: under a branch the
+// compiler moves a load next to its use and waits for it there, one round trip a
+// row (256 experts, 32 tokens x 8: the down stage 27 us that way).  Bound by the
+// weights' bytes and a few such round trips.  Hidden 2048: a block of 64 experts
+// (inter 768) 24 us at 4 tokens x 8 and 38 at 32 (30 and 41 with bf16 operands),
+// of 256 (inter 512) 53 at 32 and 66 at 64 (57 and 74).
+// NCH: chunks of 256 values of K (0: at run time, up to 16; the others unroll).
 // ---------------------------------------------------------------------------
-constexpr int kErWaves = 8;
-// K of the tile-resident forms, in 256-code chunks: the SwiGLU stage is built
-// for hidden 2048, the down stage for every intermediate up to 1024 (whole
-// rows of weights in registers, 2 NCH uint4 a lane); other sizes take the
-// K-split forms, whose 8 waves have nothing to split at such a K (256 experts
-// of intermediate 512: 57.3 against 16.4 us at 32 tokens, 120 against 33.2 us
-// at 509).
-constexpr int kErChunksUp = 8, kErMaxChunksDown = 4;
-constexpr int kErAhead = 2;  // weight chunks in flight per wave ahead of the MFMAs
+namespace gd {
+constexpr int kWaves = 8, kThreads = 64 * kWaves;
+constexpr int kMaxChunks = 16;
+// Weight chunks in flight ahead of the products.  (All of a wave's share at
+// once kept the tile's x loads waiting behind the other workgroups' weights.)
+constexpr int kAhead = 3, kRing = 4;
+constexpr int kRow = 272;  // bytes of a staged row of h: 256 and padding (banks)
 
-// SwiGLU: BPW up blocks (and the matching gate blocks) per wave; x' pairs of
-// the tile's tokens (x_pairs [T, K / 2] uint32, x_corr [T]) staged in LDS.
-template <int BPW, int ADT, int NCH, int QPB>
-__global__ __launch_bounds__(64 * kErWaves) void k_grouped_swiglu_er(
-    const uint32_t* __restrict__ x_pairs, const float* __restrict__ x_corr, int64_t topk,
-    const uint32_t* __restrict__ w, int64_t n_half, const void* __restrict__ alpha,
-    const int32_t* __restrict__ offsets, const int32_t* __restrict__ pair_ids, int n_exp,
-    uint16_t* __restrict__ hp, uint16_t* __restrict__ h, int64_t ldh) {
-  constexpr int NW = 16 * NCH;  // words of K
-  __shared__ u32x4v_t xs[NW][2][16];
-  __shared__ int32_t s_pid[16], s_tok[16];
-  __shared__ float s_c[16];
-  int e, pos0, np;
-  if (!decode_tile(offsets, n_exp, blockIdx.y, 16, e, pos0, np)) return;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int r16 = lane & 15, g = lane >> 4;
-  const int64_t nblk = n_half / 16;
-  const int64_t b0 = (static_cast<int64_t>(blockIdx.x) * kErWaves + wv) * BPW;  // first up block
-  const uint32_t* we = w + static_cast<int64_t>(e) * (2 * n_half) * NW;
-  // Issue order matters (memory counters complete in issue order): the pair
-  // ids, then the tile's x' pairs, then the weights, so that staging x' waits
-  // for nothing behind it and the weights stream while it happens.
-  if (tid < 16) {
-    const int p = tid < np ? pair_ids[pos0 + tid] : -1;
-    s_pid[tid] = p;
-    s_tok[tid] = p >= 0 ? static_cast<int>(p / topk) : -1;
-  }
-  __syncthreads();
-  // the tile's x' pairs: item = (col, word, half), 16-byte loads
-  constexpr int kItems = 16 * NW * 2, kPer = (kItems + 64 * kErWaves - 1) / (64 * kErWaves);
-  u32x4v_t sv[kPer];
+template <int NCH>
+struct Shared {
+  static constexpr int kSteps = 2 * (NCH ? NCH : kMaxChunks);
+  // step s, chunk c of pair p at (p * nsteps + s) * 16 + (c ^ p)
+  __align__(16) uint4 x[16 * kSteps * 16];
+  uint32_t scale[16][kSteps + 1];
+};
+
+// Rows r16 of the wave's two blocks from rp[j] (+ 4 g), nch chunks, against the
+// tile: acc[j][p] of piece p.
+template <int NCH>
+__device__ __forceinline__ void load(const uint32_t* const (&rp)[2], int c, uint4 (&w)[2]) {
 #pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    const int it = tid + 64 * kErWaves * k;
-    const int col = (it < kItems ? it : 0) / (NW * 2), rem = it % (NW * 2);
-    const int tk = s_tok[col];
-    sv[k] = u32x4v_t{0u, 0u, 0u, 0u};
-    if (it < kItems && tk >= 0)
-      sv[k] = *reinterpret_cast<const u32x4v_t*>(x_pairs + static_cast<int64_t>(tk) * (NW * 8) + rem * 4);
-  }
-  float cx = 0.f;
-  if (tid < 16 && s_tok[tid] >= 0) cx = x_corr[s_tok[tid]];
-  // weights of this wave's blocks, chunk by chunk, kErAhead chunks ahead of
-  // their use: with every wave's whole share requested at once (16 KB), the
-  // tile's x' loads queued behind the other workgroups' weight streams for
-  // ~6 us before the first MFMA could start; a short pipeline keeps the
-  // queues short, and the MFMAs run while the later chunks stream
-  const uint32_t* rp[2 * BPW];
+  for (int j = 0; j < 2; ++j) w[j] = *reinterpret_cast<const uint4*>(rp[j] + 16 * c);
+}
+
+__device__ __forceinline__ void chunk(const uint4 (&w)[2], const uint4* x, const uint32_t* scale, int g, int r16,
+                                      mx_f32x4_t (&acc)[2][2]) {
 #pragma unroll
-  for (int j = 0; j < 2 * BPW; ++j) {
-    int64_t blk = b0 + (j % BPW);
-    blk = blk < nblk ? blk : nblk - 1;
-    rp[j] = we + ((j / BPW) * n_half + blk * 16 + r16) * NW + 4 * g;
-  }
-  u32x4v_t wq[2 * BPW][NCH];
+  for (int s = 0; s < 2; ++s) {
+    const int sb = reinterpret_cast<const uint8_t*>(scale + s)[g];
+    const i32x8_t b0 = mx_operand(x[16 * s + (g ^ r16)], x[16 * s + ((4 + g) ^ r16)]);
+    const i32x8_t b1 = mx_operand(x[16 * s + ((8 + g) ^ r16)], x[16 * s + ((12 + g) ^ r16)]);
+    uint32_t a[2][4];
 #pragma unroll
-  for (int c = 0; c < kErAhead && c < NCH; ++c)
+    for (int j = 0; j < 2; ++j) mx_expand2(s ? make_uint2(w[j].z, w[j].w) : make_uint2(w[j].x, w[j].y), a[j]);
 #pragma unroll
-    for (int j = 0; j < 2 * BPW; ++j) wq[j][c] = *reinterpret_cast<const u32x4v_t*>(rp[j] + 16 * c);
-  MA_ISSUE_FENCE();
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    const int it = tid + 64 * kErWaves * k;
-    if (it < kItems) xs[(it % (NW * 2)) >> 1][it & 1][it / (NW * 2)] = sv[k];
-  }
-  if (tid < 16) s_c[tid] = cx;
-  __syncthreads();
-  // two accumulators per block (the two halves of each word), so a block's
-  // MFMAs are independent of each other
-  f32x4d_t acc[2 * BPW][2];
-#pragma unroll
-  for (int j = 0; j < 2 * BPW; ++j) acc[j][0] = acc[j][1] = f32x4d_t{0.f, 0.f, 0.f, 0.f};
-  const ExpandConsts kc;
-#pragma unroll
-  for (int c = 0; c < NCH; ++c) {
-    if (c + kErAhead < NCH) {
-#pragma unroll
-      for (int j = 0; j < 2 * BPW; ++j)
-        wq[j][c + kErAhead] = *reinterpret_cast<const u32x4v_t*>(rp[j] + 16 * (c + kErAhead));
-    }
-    MA_ISSUE_FENCE();
-#pragma unroll
-    for (int q0 = 0; q0 < 4; q0 += QPB) {  // QPB words per MFMA block
-      u32x4v_t av[QPB][2 * BPW][2], bv[QPB][2];
-#pragma unroll
-      for (int qi = 0; qi < QPB; ++qi) {
-#pragma unroll
-        for (int j = 0; j < 2 * BPW; ++j) {
-          uint32_t ex[8];
-          expand_word(wq[j][c][q0 + qi], ex, kc);
-          av[qi][j][0] = u32x4v_t{ex[0], ex[1], ex[2], ex[3]};
-          av[qi][j][1] = u32x4v_t{ex[4], ex[5], ex[6], ex[7]};
-        }
-        bv[qi][0] = xs[16 * c + 4 * g + q0 + qi][0][r16];
-        bv[qi][1] = xs[16 * c + 4 * g + q0 + qi][1][r16];
-      }
-      mfma_block_begin();
-#pragma unroll
-      for (int qi = 0; qi < QPB; ++qi)
-#pragma unroll
-        for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-          for (int j = 0; j < 2 * BPW; ++j) mfma_acc(acc[j][hf], av[qi][j][hf], bv[qi][hf]);
-      mfma_block_end();
-      keep_b(av, acc[0]);
-      keep_b(bv, acc[0]);
-    }
-  }
-  f32x4d_t accs[2 * BPW];
-#pragma unroll
-  for (int j = 0; j < 2 * BPW; ++j) accs[j] = acc[j][0] + acc[j][1];
-  // Epilogue: lane holds pair column r16, rows 4 g .. +3 of each block.
-  if (r16 >= np) return;
-  const float cc = s_c[r16];
-  const int pid = s_pid[r16];
-  const int64_t nwh = n_half / 16;
-#pragma unroll
-  for (int j = 0; j < BPW; ++j) {
-    const int64_t blk = b0 + j;
-    if (blk >= nblk) continue;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int64_t i = blk * 16 + 4 * g + r;
-      const float au = ld_t<ADT>(alpha, static_cast<int64_t>(e) * 2 * n_half + i);
-      const float ag = ld_t<ADT>(alpha, static_cast<int64_t>(e) * 2 * n_half + n_half + i);
-      const uint16_t hb = f32_to_bf16(swiglu_act(au * (accs[j][r] - cc), ag * (accs[BPW + j][r] - cc)));
-      if (hp) {
-        const int pos = static_cast<int>(i & 15), jj = pos & 7, hh = pos >> 3;
-        const float hv = bf16_to_f32(hb) * pair_scale(jj);  // exact: power-of-two scale
-        hp[((static_cast<int64_t>(pos0 + r16) * nwh + (i >> 4)) * 8 + jj) * 2 + hh] =
-            static_cast<uint16_t>(bf16_bits_exact(hv));
-      }
-      if (h) h[static_cast<int64_t>(pid) * ldh + i] = hb;
+    for (int j = 0; j < 2; ++j) {
+      acc[j][0] = mx_mfma_fp4(a[j], b0, acc[j][0], mx_piece_scale(0), sb);
+      acc[j][1] = mx_mfma_fp4(a[j], b1, acc[j][1], mx_piece_scale(1), sb);
     }
   }
 }
 
-// Down: BPW output blocks per wave; h's x' pairs of the tile (hp rows pos0 ..)
-// staged in LDS with each pair's correction.
-template <int BPW, int ADT, int NCH>
-__global__ __launch_bounds__(64 * kErWaves) void k_grouped_down_er(
-    const uint32_t* __restrict__ hp, const uint32_t* __restrict__ w, int64_t n_out,
-    const void* __restrict__ alpha, const int32_t* __restrict__ offsets, int n_exp,
-    uint16_t* __restrict__ out) {
-  constexpr int NW = 16 * NCH;  // words of K
-  __shared__ u32x4v_t xs[NW][2][16];
-  __shared__ float s_cw[16][NW];
-  __shared__ float s_c[16];
+template <int NCH>
+__device__ __forceinline__ void kloop(const uint32_t* const (&rp)[2], int nch, uint4 (&ring)[kRing][2],
+                                      const Shared<NCH>& sh, int g, int r16, mx_f32x4_t (&acc)[2][2]) {
+  const uint4* x = sh.x + r16 * (2 * nch) * 16;
+  const uint32_t* scale = sh.scale[r16];
+  if constexpr (NCH > 0) {
+#pragma unroll
+    for (int c = 0; c < NCH; ++c) {
+      if (c + kAhead < NCH) load<NCH>(rp, c + kAhead, ring[(c + kAhead) % kRing]);
+      MA_ISSUE_FENCE();
+      chunk(ring[c % kRing], x + 32 * c, scale + 2 * c, g, r16, acc);
+      mx_pin(acc[0][0], acc[0][1], acc[1][0], acc[1][1]);
+    }
+  } else {
+    for (int c0 = 0; c0 < nch; c0 += kRing) {
+#pragma unroll
+      for (int s = 0; s < kRing; ++s) {
+        const int c = c0 + s;
+        if (c >= nch) break;
+        load<NCH>(rp, c + kAhead < nch ? c + kAhead : nch - 1, ring[(s + kAhead) % kRing]);
+        MA_ISSUE_FENCE();
+        chunk(ring[s], x + 32 * c, scale + 2 * c, g, r16, acc);
+        mx_pin(acc[0][0], acc[0][1], acc[1][0], acc[1][1]);
+      }
+    }
+  }
+}
+}  // namespace gd
+
+// SwiGLU: 128 outputs (8 up blocks and the matching gate blocks, one of each a
+// wave) of a tile of 16 pairs.
+template <int ADT, int NCH>
+__global__ __launch_bounds__(gd::kThreads) void k_gd_swiglu(
+    const uint16_t* __restrict__ x, int64_t ldx, int64_t topk, const uint32_t* __restrict__ w, int64_t n_half,
+    int nch_arg, const void* __restrict__ alpha, const int32_t* __restrict__ offsets,
+    const int32_t* __restrict__ pair_ids, int n_exp, uint16_t* __restrict__ hp, uint32_t* __restrict__ hs,
+    float* __restrict__ hcorr, uint16_t* __restrict__ h, int64_t ldh) {
+  using namespace gd;
+  constexpr int MAXCH = NCH ? NCH : kMaxChunks;
+  constexpr int kPer = (16 * MAXCH + 63) / 64;  // words of a pair per lane
+  __shared__ Shared<NCH> sh;
+  __shared__ int32_t s_pid[16], s_tok[16];
+  __shared__ float s_c[16], s_sum[kWaves][16];
+  __shared__ uint32_t s_ex[kWaves][16], s_hsc[16];
   int e, pos0, np;
   if (!decode_tile(offsets, n_exp, blockIdx.y, 16, e, pos0, np)) return;
+  e = __builtin_amdgcn_readfirstlane(e);
+  pos0 = __builtin_amdgcn_readfirstlane(pos0);
+  np = __builtin_amdgcn_readfirstlane(np);
+  const int nch = NCH ? NCH : nch_arg, nwords = 16 * nch, nsteps = 2 * nch;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, g = lane >> 4;
-  const int64_t nblk = n_out / 16;
-  const int64_t b0 = (static_cast<int64_t>(blockIdx.x) * kErWaves + wv) * BPW;
-  const uint32_t* we = w + static_cast<int64_t>(e) * n_out * NW;
-  // stage: item = (col, word): both halves of the word and its correction;
-  // these loads go out before the weights' (memory counters complete in issue
-  // order), so staging does not wait for the weight stream
-  constexpr int kItems = 16 * NW, kPer = (kItems + 64 * kErWaves - 1) / (64 * kErWaves);
-  u32x4v_t sv[kPer][2];
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    const int it = tid + 64 * kErWaves * k;
-    const int col = it / NW, wd = it % NW;
-    sv[k][0] = sv[k][1] = u32x4v_t{0u, 0u, 0u, 0u};
-    if (it < kItems && col < np) {
-      const u32x4v_t* src = reinterpret_cast<const u32x4v_t*>(hp + (static_cast<int64_t>(pos0 + col) * NW + wd) * 8);
-      sv[k][0] = src[0];
-      sv[k][1] = src[1];
-    }
-  }
-  // weights of this wave's blocks for all of K (a pipeline as in the SwiGLU
-  // stage measured no faster here: K is only 3 chunks)
-  u32x4v_t wq[BPW][NCH];
-#pragma unroll
-  for (int j = 0; j < BPW; ++j) {
-    int64_t blk = b0 + j;
-    blk = blk < nblk ? blk : nblk - 1;
-    const uint32_t* rp = we + (blk * 16 + r16) * NW + 4 * g;
-#pragma unroll
-    for (int c = 0; c < NCH; ++c) wq[j][c] = *reinterpret_cast<const u32x4v_t*>(rp + 16 * c);
-  }
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    const int it = tid + 64 * kErWaves * k;
-    if (it >= kItems) continue;
-    const int col = it / NW, wd = it % NW;
-    xs[wd][0][col] = sv[k][0];
-    xs[wd][1][col] = sv[k][1];
-    const uint32_t pr[8] = {sv[k][0].x, sv[k][0].y, sv[k][0].z, sv[k][0].w,
-                            sv[k][1].x, sv[k][1].y, sv[k][1].z, sv[k][1].w};
-    s_cw[col][wd] = pairs_cst(pr);
+  const int n_rtiles = static_cast<int>(n_half / 128), rtile = static_cast<int>(blockIdx.x);
+  // Issue order matters (memory counters complete in issue order): the pair
+  // ids, then the tile's rows of x, then the weights, so that staging x waits
+  // for nothing behind it and the weights stream while it happens.
+  if (tid < np) {
+    const int p = pair_ids[pos0 + tid];
+    s_pid[tid] = p;
+    s_tok[tid] = p / static_cast<int>(topk);
   }
   __syncthreads();
-  if (tid < 16) {  // fixed order
-    float c = 0.f;
-    for (int wd = 0; wd < NW; ++wd) c += s_cw[tid][wd];
-    s_c[tid] = c;
-  }
-  f32x4d_t acc[BPW][2];  // per word half: a block's MFMAs are independent
+  uint4 xv[2][kPer][2];  // pairs wv and wv + 8
 #pragma unroll
-  for (int j = 0; j < BPW; ++j) acc[j][0] = acc[j][1] = f32x4d_t{0.f, 0.f, 0.f, 0.f};
-  const ExpandConsts kc;
+  for (int ci = 0; ci < 2; ++ci) {
+    const int col = wv + 8 * ci;
+    if (col < np) {
+      const uint4* src = reinterpret_cast<const uint4*>(x + s_tok[col] * ldx);
 #pragma unroll
-  for (int c = 0; c < NCH; ++c) {
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      u32x4v_t av[BPW][2], bv[2];
-#pragma unroll
-      for (int j = 0; j < BPW; ++j) {
-        uint32_t ex[8];
-        expand_word(wq[j][c][q], ex, kc);
-        av[j][0] = u32x4v_t{ex[0], ex[1], ex[2], ex[3]};
-        av[j][1] = u32x4v_t{ex[4], ex[5], ex[6], ex[7]};
+      for (int k = 0; k < kPer; ++k) {
+        const int wd = lane + 64 * k < nwords ? lane + 64 * k : nwords - 1;
+        xv[ci][k][0] = src[2 * wd];
+        xv[ci][k][1] = src[2 * wd + 1];
       }
-      bv[0] = xs[16 * c + 4 * g + q][0][r16];
-      bv[1] = xs[16 * c + 4 * g + q][1][r16];
-      mfma_block_begin();
-#pragma unroll
-      for (int hf = 0; hf < 2; ++hf)
-#pragma unroll
-        for (int j = 0; j < BPW; ++j) mfma_acc(acc[j][hf], av[j][hf], bv[hf]);
-      mfma_block_end();
-      keep_b(av, acc[0]);
-      keep_b(bv, acc[0]);
     }
   }
-  f32x4d_t accs[BPW];
+  MA_ISSUE_FENCE();
+  const int64_t blk = static_cast<int64_t>(rtile) * kWaves + wv;
+  const uint32_t* we = w + static_cast<int64_t>(e) * (2 * n_half) * nwords;
+  const uint32_t* rp[2] = {we + (blk * 16 + r16) * nwords + 4 * g, we + (n_half + blk * 16 + r16) * nwords + 4 * g};
+  uint4 ring[kRing][2];
 #pragma unroll
-  for (int j = 0; j < BPW; ++j) accs[j] = acc[j][0] + acc[j][1];
-  __syncthreads();  // s_c
-  if (r16 >= np) return;
+  for (int c = 0; c < kAhead; ++c)
+    if (NCH == 0 || c < NCH) load<NCH>(rp, c < nch ? c : nch - 1, ring[c]);
+  MA_ISSUE_FENCE();
+#pragma unroll
+  for (int ci = 0; ci < 2; ++ci) {
+    const int col = wv + 8 * ci;
+    if (col >= np) continue;  // (a column past np keeps what is there: its products are dropped)
+    float sum = 0.f;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int wd = lane + 64 * k;
+      if (wd >= nwords) break;  // a word pair's two lanes together
+      const uint4 a = xv[ci][k][0], b = xv[ci][k][1];
+      const uint32_t u[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      float v[16];
+      uint32_t ex = 0;
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        v[2 * q] = __uint_as_float(u[q] << 16);
+        v[2 * q + 1] = __uint_as_float(u[q] & 0xffff0000u);
+        sum += v[2 * q];
+        sum += v[2 * q + 1];
+        ex = mx_exponent(mx_exponent(ex, v[2 * q]), v[2 * q + 1]);
+      }
+      const uint32_t eo = __shfl_xor(ex, 1, 64);
+      ex = ex > eo ? ex : eo;
+      uint4 out[2];
+      mx_word<2>(v, mx_factor(ex), out);
+      const int step = wd / 16 * 2 + (wd >> 1 & 1), pos = (wd >> 2 & 3) * 2 + (wd & 1);
+#pragma unroll
+      for (int p = 0; p < 2; ++p) sh.x[(col * nsteps + step) * 16 + ((8 * p + pos) ^ col)] = out[p];
+      if ((wd & 1) == 0)
+        reinterpret_cast<uint8_t*>(&sh.scale[col][step])[pos / 2] = static_cast<uint8_t>(mx_scale_byte(ex));
+    }
+    sum = group_sum<64>(sum);
+    if (lane == 0) s_c[col] = sum;
+  }
+  __syncthreads();
+  mx_f32x4_t acc[2][2];  // up, gate by piece
+#pragma unroll
+  for (int j = 0; j < 2; ++j) acc[j][0] = acc[j][1] = mx_f32x4_t{0.f, 0.f, 0.f, 0.f};
+  kloop<NCH>(rp, nch, ring, sh, g, r16, acc);
+  // Epilogue: lane holds pair r16, outputs i0 + r of its 16-output word (word wv
+  // of the tile's 8).  Two waves' words share a scale block, so the exponents
+  // meet in LDS first; then as the prefill form: h's bytes staged as [pair][two
+  // half steps], out in 16-byte pieces.
+  const int64_t i0 = blk * 16 + 4 * g;
   const float cc = s_c[r16];
+  float hv[4], hsum = 0.f;
+  uint32_t ex = 0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float au = ld_t<ADT>(alpha, static_cast<int64_t>(e) * 2 * n_half + i0 + r);
+    const float ag = ld_t<ADT>(alpha, static_cast<int64_t>(e) * 2 * n_half + n_half + i0 + r);
+    const uint16_t hb = f32_to_bf16(
+        swiglu_act(au * (acc[0][0][r] + acc[0][1][r] - cc), ag * (acc[1][0][r] + acc[1][1][r] - cc)));
+    hv[r] = bf16_to_f32(hb);
+    hsum += hv[r];
+    ex = mx_exponent(ex, hv[r]);
+    if (h && r16 < np) h[static_cast<int64_t>(s_pid[r16]) * ldh + i0 + r] = hb;
+  }
+  uint32_t eo = __shfl_xor(ex, 16, 64);
+  ex = ex > eo ? ex : eo;
+  eo = __shfl_xor(ex, 32, 64);
+  ex = ex > eo ? ex : eo;
+  hsum += __shfl_xor(hsum, 16, 64);
+  hsum += __shfl_xor(hsum, 32, 64);
+  if (g == 0) {
+    s_ex[wv][r16] = ex;
+    s_sum[wv][r16] = hsum;
+  }
+  __syncthreads();  // (and every wave is done with the tile's rows)
+  eo = s_ex[wv ^ 1][r16];
+  ex = ex > eo ? ex : eo;
+  const int b = wv / 2;  // block of 32 outputs: step b & 1, half b / 2 of the tile's part
+  uint8_t* hst = reinterpret_cast<uint8_t*>(sh.x);
+  const float f = mx_factor(ex);
+  float v[4] = {hv[0] * f, hv[2] * f, hv[1] * f, hv[3] * f};
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const uint32_t w4 = mx_piece4(v);
+    uint16_t* dst =
+        reinterpret_cast<uint16_t*>(hst + r16 * kRow + 128 * (b & 1) + 64 * p + 32 * (b / 2) + 16 * (wv & 1) + 2 * g);
+    dst[0] = static_cast<uint16_t>(w4);
+    dst[4] = static_cast<uint16_t>(w4 >> 16);
+  }
+  if (g == 0 && (wv & 1) == 0)
+    reinterpret_cast<uint8_t*>(s_hsc + r16)[(b & 1) * 2 + b / 2] = static_cast<uint8_t>(mx_scale_byte(ex));
+  __syncthreads();
+  if (tid < np) {
+    float c = 0.f;
+#pragma unroll
+    for (int k = 0; k < kWaves; ++k) c += s_sum[k][tid];
+    hcorr[static_cast<int64_t>(pos0 + tid) * n_rtiles + rtile] = c;
+  }
+  if (tid < 2 * np) {  // the scale bytes of the tile's two blocks of each step
+    const int col = tid >> 1, st = tid & 1;
+    reinterpret_cast<uint16_t*>(hs + static_cast<int64_t>(pos0 + col) * n_rtiles + (rtile & ~1) + st)[rtile & 1] =
+        reinterpret_cast<const uint16_t*>(s_hsc + col)[st];
+  }
+  if (tid < 16 * np) {
+    const int col = tid / 16, part = tid % 16;
+    *reinterpret_cast<uint4*>(hp + (static_cast<int64_t>(pos0 + col) * n_rtiles + (rtile & ~1) + part / 8) * kMxStep +
+                              64 * (part / 4 & 1) + 32 * (rtile & 1) + 8 * (part & 3)) =
+        *reinterpret_cast<const uint4*>(hst + col * kRow + part * 16);
+  }
+}
+
+// Down: 256 output rows (two blocks a wave) of a tile of 16 pairs, whose mx rows
+// of h, scale words and correction parts the SwiGLU stage wrote.
+template <int ADT, int NCH>
+__global__ __launch_bounds__(gd::kThreads) void k_gd_down(const uint32_t* __restrict__ hp,
+                                                          const uint32_t* __restrict__ hs,
+                                                          const float* __restrict__ hcorr,
+                                                          const uint32_t* __restrict__ w, int64_t n_out, int nch_arg,
+                                                          const void* __restrict__ alpha,
+                                                          const int32_t* __restrict__ offsets, int n_exp,
+                                                          uint16_t* __restrict__ out) {
+  using namespace gd;
+  constexpr int MAXCH = NCH ? NCH : kMaxChunks;
+  constexpr int kPer = (2 * MAXCH * 16 + 63) / 64;  // 16-byte chunks of a pair per lane
+  __shared__ Shared<NCH> sh;
+  __shared__ float s_cp[16][2 * MAXCH + 1];
+  int e, pos0, np;
+  if (!decode_tile(offsets, n_exp, blockIdx.y, 16, e, pos0, np)) return;
+  e = __builtin_amdgcn_readfirstlane(e);
+  pos0 = __builtin_amdgcn_readfirstlane(pos0);
+  np = __builtin_amdgcn_readfirstlane(np);
+  const int nch = NCH ? NCH : nch_arg, nwk = 16 * nch, nsteps = 2 * nch;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, g = lane >> 4;
+  // the rows' loads go out before the weights' (memory counters complete in
+  // issue order), so staging does not wait for the weight stream
+  uint4 hv[2][kPer];  // pairs wv and wv + 8 (past np: the last one's, not stored)
+#pragma unroll
+  for (int ci = 0; ci < 2; ++ci) {
+    const int col = wv + 8 * ci < np ? wv + 8 * ci : np - 1;
+    const uint4* src = reinterpret_cast<const uint4*>(hp) + static_cast<int64_t>(pos0 + col) * nsteps * 16;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) hv[ci][k] = src[lane + 64 * k < nsteps * 16 ? lane + 64 * k : 0];
+  }
+  uint32_t sw = 0;
+  float cp = 0.f;
+  const int sc = tid / nsteps, ss = tid % nsteps;  // 16 nsteps <= 512
+  if (sc < np) {
+    sw = hs[static_cast<int64_t>(pos0 + sc) * nsteps + ss];
+    cp = hcorr[static_cast<int64_t>(pos0 + sc) * nsteps + ss];
+  }
+  MA_ISSUE_FENCE();
+  const uint32_t* we = w + static_cast<int64_t>(e) * n_out * nwk;
+  const int64_t n0 = (static_cast<int64_t>(blockIdx.x) * kWaves + wv) * 32;  // n_out % 256 == 0
+  const uint32_t* rp[2] = {we + (n0 + r16) * nwk + 4 * g, we + (n0 + 16 + r16) * nwk + 4 * g};
+  uint4 ring[kRing][2];
+#pragma unroll
+  for (int c = 0; c < kAhead; ++c)
+    if (NCH == 0 || c < NCH) load<NCH>(rp, c < nch ? c : nch - 1, ring[c]);
+  MA_ISSUE_FENCE();
+#pragma unroll
+  for (int ci = 0; ci < 2; ++ci) {
+    const int col = wv + 8 * ci;
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) {
+      const int i = lane + 64 * k;
+      if (col < np && i < nsteps * 16) sh.x[(col * nsteps + i / 16) * 16 + (i % 16 ^ col)] = hv[ci][k];
+    }
+  }
+  if (sc < np) {
+    sh.scale[sc][ss] = sw;
+    s_cp[sc][ss] = cp;
+  }
+  __syncthreads();
+  mx_f32x4_t acc[2][2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) acc[j][0] = acc[j][1] = mx_f32x4_t{0.f, 0.f, 0.f, 0.f};
+  kloop<NCH>(rp, nch, ring, sh, g, r16, acc);
+  if (r16 >= np) return;
+  float cc = 0.f;  // the correction parts in order
+  for (int k = 0; k < nsteps; ++k) cc += s_cp[r16][k];
   uint16_t* orow = out + static_cast<int64_t>(pos0 + r16) * n_out;
 #pragma unroll
-  for (int j = 0; j < BPW; ++j) {
-    const int64_t blk = b0 + j;
-    if (blk >= nblk) continue;
-    const int64_t n0 = blk * 16 + 4 * g;
+  for (int j = 0; j < 2; ++j) {
+    const int64_t n = n0 + 16 * j + 4 * g;
     float o[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) o[r] = ld_t<ADT>(alpha, static_cast<int64_t>(e) * n_out + n0 + r) * (accs[j][r] - cc);
+    for (int r = 0; r < 4; ++r)
+      o[r] = ld_t<ADT>(alpha, static_cast<int64_t>(e) * n_out + n + r) * (acc[j][0][r] + acc[j][1][r] - cc);
     uint2 rr;
     rr.x = pack_bf16x2_rn(o[0], o[1]);
     rr.y = pack_bf16x2_rn(o[2], o[3]);
-    *reinterpret_cast<uint2*>(orow + n0) = rr;
+    *reinterpret_cast<uint2*>(orow + n) = rr;
   }
 }
 
@@ -767,9 +860,10 @@ __device__ __forceinline__ bool gp_tile(const int32_t* __restrict__ offsets, int
                                         int& rtile) {
   const int lane = threadIdx.x & 63;
   int m = 0;  // pair tiles of every expert
+#pragma unroll 4
   for (int base = 0; base < n_exp; base += 64) {
     const int ee = base + lane;
-    m += ee < n_exp ? (offsets[ee + 1] - offsets[ee] + TOK - 1) / TOK : 0;
+    m += (offsets[ee + 1 < n_exp ? ee + 1 : n_exp] - offsets[ee < n_exp ? ee : n_exp] + TOK - 1) / TOK;
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) m += __shfl_xor(m, off, 64);
@@ -1174,8 +1268,11 @@ __global__ __launch_bounds__(gp::Tile<TOK>::kThreads) __attribute__((amdgpu_wave
 
 using namespace ma;
 
-// Up to this many pairs per expert on average (decode batches) the K-split
-// kernels run; above it (prefill) the LDS-staged tiles of up to 64 pairs.
+// Up to this many pairs per expert on average (decode batches) 16-pair tiles
+// run, above it (prefill) tiles of 32 and 64 pairs: at 16 an expert (256
+// experts, inter 512, 509 tokens x 8) 103 us a block against 104, at 16 of 64
+// experts (128 tokens) 52 against 53, at 1 of 256 53
+// against 71.
 constexpr int64_t kKsMaxPairsPerExpert = 16;
 // Up to this many the prefill form's tiles hold 32 pairs instead of 64 (64
 // experts: at 64 pairs an expert 94 against 97 us a block, at 96 104 against
@@ -1185,18 +1282,18 @@ constexpr int64_t kSmallTilePairsPerExpert = 48;
 static size_t align256(size_t b) { return (b + 255) & ~static_cast<size_t>(255); }
 
 // Workspace of one call: h [P, inter] in 16 bits a value (pairs, or mx rows),
-// per-pair down outputs [P, hidden] bf16; in the prefill form also the mx rows
-// of the tokens (2 bytes a value), their sums and scale words, and h's scale
-// words and the SwiGLU tiles' correction parts [P, inter / 128].
+// per-pair down outputs [P, hidden] bf16, h's scale words and the SwiGLU tiles'
+// correction parts [P, inter / 128]; in the prefill form also the mx rows of the
+// tokens (2 bytes a value), their sums and scale words.
 static bool grouped_prefill_form(int64_t n_pairs, int64_t n_experts) {
   return n_pairs > kKsMaxPairsPerExpert * n_experts;
 }
 static size_t grouped_bytes(int64_t n_pairs, int64_t tokens, int64_t inter, int64_t hidden, bool prefill) {
-  size_t b = align256(static_cast<size_t>(n_pairs) * inter * 2) + align256(static_cast<size_t>(n_pairs) * hidden * 2);
+  size_t b = align256(static_cast<size_t>(n_pairs) * inter * 2) + align256(static_cast<size_t>(n_pairs) * hidden * 2) +
+             2 * align256(static_cast<size_t>(n_pairs) * (inter / kMxStep) * 4);
   if (prefill)
     b += align256(static_cast<size_t>(tokens) * hidden * 2) + align256(static_cast<size_t>(tokens) * 8) +
-         align256(static_cast<size_t>(tokens) * (hidden / kMxStep) * 4) +
-         2 * align256(static_cast<size_t>(n_pairs) * cdiv(inter, gp::kRows / 2) * 4);
+         align256(static_cast<size_t>(tokens) * (hidden / kMxStep) * 4);
   return b;
 }
 
@@ -1239,23 +1336,34 @@ static int grouped_launch(const void* x, int64_t ldx, const uint32_t* x_pairs, c
   const auto* xb = static_cast<const uint16_t*>(x);
   auto* hb = static_cast<uint16_t*>(h_out);
   if (!grouped_prefill_form(n_pairs, n_experts)) {
-    // decode: 16-pair tiles, K split over the waves of a workgroup
+    // decode: 16-pair tiles
     const unsigned max_tiles = static_cast<unsigned>(n_pairs / 16 + n_experts);
-    dim3 g1(static_cast<unsigned>(cdiv(inter, 32)), max_tiles);
-    dim3 g2(static_cast<unsigned>(cdiv(hidden, 64)), max_tiles);
-    // tile-resident forms: 16 rows (up + gate) / 32 rows per wave
-    dim3 ge1(static_cast<unsigned>(cdiv(inter, 16 * kErWaves)), max_tiles);
-    dim3 ge2(static_cast<unsigned>(cdiv(hidden, 32 * kErWaves)), max_tiles);
-#define MA_GROUPED_DOWN(ADT, NCH)                                                                \
-  hipLaunchKernelGGL((k_grouped_down_er<2, ADT, NCH>), ge2, dim3(64 * kErWaves), 0, s,           \
-                     reinterpret_cast<const uint32_t*>(hp), down, hidden, down_alpha, offsets,   \
-                     ne, out);
+    if (hidden <= 256 * gd::kMaxChunks && inter <= 256 * gd::kMaxChunks) {
+      const int64_t hsteps = inter / kMxStep;
+      const int uch = static_cast<int>(hidden / 256), dch = static_cast<int>(inter / 256);
+      uint32_t* hs = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(out) +
+                                                 align256(static_cast<size_t>(n_pairs) * hidden * 2));
+      float* hcorr = reinterpret_cast<float*>(reinterpret_cast<char*>(hs) +
+                                              align256(static_cast<size_t>(n_pairs) * hsteps * 4));
+      const dim3 g1(static_cast<unsigned>(hsteps), max_tiles), g2(static_cast<unsigned>(hidden / 256), max_tiles);
+#define MA_GD_UP(ADT, NCH)                                                                                           \
+  hipLaunchKernelGGL((k_gd_swiglu<ADT, NCH>), g1, dim3(gd::kThreads), 0, s, xb, ldx, top_k, up_gate, inter, uch,      \
+                     up_gate_alpha, offsets, pair_ids, ne, hp, hs, hcorr, hb, ldh)
+#define MA_GD_DOWN(ADT, NCH)                                                                                         \
+  hipLaunchKernelGGL((k_gd_down<ADT, NCH>), g2, dim3(gd::kThreads), 0, s, reinterpret_cast<const uint32_t*>(hp), hs, \
+                     hcorr, down, hidden, dch, down_alpha, offsets, ne, out)
+#define MA_GD(ADT)                                                                            \
+  if (uch == 8) MA_GD_UP(ADT, 8); else MA_GD_UP(ADT, 0);                                      \
+  if (dch == 2) MA_GD_DOWN(ADT, 2); else if (dch == 3) MA_GD_DOWN(ADT, 3); else MA_GD_DOWN(ADT, 0);
+      if (alpha_dtype == MA_BF16) { MA_GD(MA_BF16) } else { MA_GD(MA_F32) }
+#undef MA_GD
+#undef MA_GD_DOWN
+#undef MA_GD_UP
+    } else {
+      // rows too long for a tile in LDS: K split over the waves of a workgroup
+      const dim3 g1(static_cast<unsigned>(cdiv(inter, 32)), max_tiles), g2(static_cast<unsigned>(cdiv(hidden, 64)), max_tiles);
 #define MA_GROUPED_KS(ADT)                                                                       \
-  if (x_pairs && hidden == 16 * 16 * kErChunksUp)                                                \
-    hipLaunchKernelGGL((k_grouped_swiglu_er<1, ADT, kErChunksUp, 1>), ge1, dim3(64 * kErWaves),  \
-                       0, s, x_pairs, x_corr, top_k, up_gate, inter, up_gate_alpha, offsets,     \
-                       pair_ids, ne, hp, hb, ldh);                                               \
-  else if (x_pairs)                                                                              \
+  if (x_pairs)                                                                                   \
     hipLaunchKernelGGL((k_grouped_swiglu_ks<2, ADT, 8, true>), g1, dim3(512), 0, s, xb, ldx,     \
                        x_pairs, x_corr, top_k, up_gate, inter, hidden / 16, up_gate_alpha,      \
                        offsets, pair_ids, ne, hp, hb, ldh);                                      \
@@ -1263,19 +1371,12 @@ static int grouped_launch(const void* x, int64_t ldx, const uint32_t* x_pairs, c
     hipLaunchKernelGGL((k_grouped_swiglu_ks<2, ADT, 8, false>), g1, dim3(512), 0, s, xb, ldx,    \
                        x_pairs, x_corr, top_k, up_gate, inter, hidden / 16, up_gate_alpha,      \
                        offsets, pair_ids, ne, hp, hb, ldh);                                      \
-  switch (inter / 256) {                                                                         \
-    case 1: MA_GROUPED_DOWN(ADT, 1) break;                                                       \
-    case 2: MA_GROUPED_DOWN(ADT, 2) break;                                                       \
-    case 3: MA_GROUPED_DOWN(ADT, 3) break;                                                       \
-    case kErMaxChunksDown: MA_GROUPED_DOWN(ADT, kErMaxChunksDown) break;                         \
-    default:                                                                                     \
-      hipLaunchKernelGGL((k_grouped_down_ks<4, ADT, 8, 2>), g2, dim3(512), 0, s,                 \
-                         reinterpret_cast<const uint32_t*>(hp), down, hidden, inter / 16,        \
-                         down_alpha, offsets, ne, out);                                          \
-  }
-    if (alpha_dtype == MA_BF16) { MA_GROUPED_KS(MA_BF16) } else { MA_GROUPED_KS(MA_F32) }
+  hipLaunchKernelGGL((k_grouped_down_ks<4, ADT, 8, 2>), g2, dim3(512), 0, s,                     \
+                     reinterpret_cast<const uint32_t*>(hp), down, hidden, inter / 16,            \
+                     down_alpha, offsets, ne, out);
+      if (alpha_dtype == MA_BF16) { MA_GROUPED_KS(MA_BF16) } else { MA_GROUPED_KS(MA_F32) }
 #undef MA_GROUPED_KS
-#undef MA_GROUPED_DOWN
+    }
   } else {
     // prefill: the tokens' mx rows once (x_pairs are the decode form's), then
     // tiles of 128 pairs x 256 weight rows.  The tiles' copy sources are

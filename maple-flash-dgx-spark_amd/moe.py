@@ -215,8 +215,6 @@ def moe_fused(x: torch.Tensor, layer: MoELayer, top_k: int, residual: torch.Tens
 
 
 ROUTE_MAX_TOKENS = 1024
-# Pairs per expert, on average, up to which ma_moe_grouped takes its decode form.
-GROUPED_DECODE_PAIRS = 16
 
 
 def route_supported(layer: MoELayer, top_k: int, x: torch.Tensor) -> bool:
@@ -376,21 +374,10 @@ def moe_block(x: torch.Tensor, layer: MoELayer, top_k: int, residual: torch.Tens
         y, ids, wts = moe_fused(xf, layer, top_k, residual, prefetch=prefetch)
         return y.reshape(x.shape), ids, wts
     res = None if residual is None else residual.reshape(-1, hidden)
-    if plan == "grouped":
-        # Decode batches: the top-k launch also writes the x' pairs that the tile-resident SwiGLU reads.  (Up to
-        # 16 tokens the router alone would be one launch instead of two, but the SwiGLU that expands x itself
-        # costs more: a block of 64 experts takes 35.4 against 37.4 us at 4 tokens and 44.9 against 53.7 at 16,
-        # of 256 experts 41.6 against 63.6 and 51.7 against 85.8; at 32 tokens 39.3 against 49.6 us.)  The
-        # prefill form reads x in another layout, which its own launch writes.
-        xf = xf.contiguous()
-        if xf.shape[0] * top_k > GROUPED_DECODE_PAIRS * layer.n_experts:
-            ids, wts = router_topk(xf, layer.gate_weight, top_k, bias=layer.router_bias)
-            xp = None
-        else:
-            ids, wts, xp = router_topk(xf, layer.gate_weight, top_k, bias=layer.router_bias, pairs=True)
-        y = moe_grouped(xf, layer, ids, wts, res, x_pairs=xp)
-        return y.reshape(x.shape), ids, wts
     ids, wts = router_topk(xf, layer.gate_weight, top_k, bias=layer.router_bias)
+    if plan == "grouped":
+        y = moe_grouped(xf, layer, ids, wts, res)
+        return y.reshape(x.shape), ids, wts
     h = ternary_expert_swiglu(xf, layer.up_gate_packed, layer.up_gate_alpha, ids)
     y = ternary_expert_down_sum(h, layer.down_packed, layer.down_alpha, ids, wts, residual=res,
                                 round_slots=True)
@@ -408,9 +395,8 @@ def moe_layer(hidden: torch.Tensor, layer: MoELayer, top_k: int, norm_weight: to
     tokens = hidden.shape[0]
     if (tokens >= GROUPED_MIN_TOKENS and route_supported(layer, top_k, hidden)
             and hidden.shape[-1] % 256 == 0 and layer.inter % 256 == 0):
-        h, xn, ids, wts, d, xp = moe_route(hidden, layer, top_k, norm_weight, eps, add=add,
-                                           pairs=True)
-        return moe_grouped(xn, layer, ids, wts, h, dispatch=d, x_pairs=xp, combine=not defer_combine), ids
+        h, xn, ids, wts, d = moe_route(hidden, layer, top_k, norm_weight, eps, add=add)
+        return moe_grouped(xn, layer, ids, wts, h, dispatch=d, combine=not defer_combine), ids
     if add is not None:
         h, xn = add_rms_norm(hidden, add, norm_weight, eps)
     else:

@@ -169,13 +169,47 @@ def test_moe_grouped_prefill_tiles_edges(dev, hidden, n_exp, inter, k, tokens, a
     assert torch.equal(z[keep], y[keep])
 
 
+@pytest.mark.parametrize("hidden,n_exp,inter,k,tokens,alpha", [
+    (256, 4, 256, 2, 9, torch.bfloat16),      # one chunk of K in both stages
+    (4096, 3, 256, 2, 17, torch.float32),     # the longest rows a tile holds
+    (512, 2, 4096, 1, 31, torch.bfloat16),    # the widest h; a full and a ragged tile
+    (2048, 8, 768, 8, 16, torch.bfloat16),    # 16 pairs an expert: one whole tile each
+    (768, 20, 512, 3, 33, torch.float32),
+    (4352, 2, 256, 2, 8, torch.bfloat16)])    # past a tile: K split over the waves
+def test_moe_grouped_decode_tiles_edges(dev, hidden, n_exp, inter, k, tokens, alpha):
+    """The decode form at the edges of its 16-pair tiles, over values of very
+    different size and rows with a stride: h and y against the oracle on the
+    kernel's own routing, the same bits on a second run, and a token with an
+    infinity leaves the others alone."""
+    L = synthetic.make_moe_layer(hidden, n_exp, inter, seed=17, device=dev)
+    L.up_gate_alpha, L.down_alpha = L.up_gate_alpha.to(alpha), L.down_alpha.to(alpha)
+    assert tokens * k <= 16 * n_exp  # the decode form
+    rng = np.random.default_rng(tokens)
+    x = synthetic.randn_bf16((tokens, hidden + 8), 650 + tokens, dev)[:, :hidden]
+    x.copy_((x.double() * torch.from_numpy(2.0 ** rng.integers(-6, 3, size=x.shape)).to(dev)).to(torch.bfloat16))
+    ids, wts = router_topk(x, L.gate_weight, k)
+    y, h = moe_grouped(x, L, ids, wts, return_h=True)
+    ref, href = ok.moe_experts(np_f(x), ids.cpu().numpy(), wts.cpu().numpy(), *_oracle_inputs(L))
+    # a value next to the middle of two bf16 numbers may round to either: one
+    # ulp, 2^-7 of a value just above a power of two, so up to 2^-8 of the scale
+    # over the relative 2^-8
+    assert_bf16_close(np_f(h), href, atol_frac=2.0 ** -8, what=f"h H={hidden} I={inter} T={tokens}")
+    assert_bf16_close(np_f(y), ref, atol_frac=2.0 ** -7, what=f"y H={hidden} I={inter} T={tokens}")
+    y2, h2 = moe_grouped(x, L, ids, wts, return_h=True)
+    assert torch.equal(y2, y) and torch.equal(h2, h)
+    x = x.clone()
+    x[tokens // 2, 1] = float("inf")
+    z = moe_grouped(x, L, ids, wts)
+    keep = torch.arange(tokens, device=dev) != tokens // 2
+    assert torch.equal(z[keep], y[keep])
+
+
 @pytest.mark.parametrize("n_exp,inter,tokens,alpha", [
     (8, 256, 4, torch.bfloat16), (8, 256, 16, torch.float32), (256, 512, 17, torch.float32),
     (256, 512, 33, torch.bfloat16), (40, 1024, 65, torch.bfloat16), (40, 1280, 20, torch.float32)])
 def test_moe_block_decode_batches_other_shapes(dev, n_exp, inter, tokens, alpha):
-    """Decode batches of the MoE block (the top-k launch also writes x') at every
-    K the tile-resident down stage is built for (256, 512, 1024) and one it is
-    not (1280), rows with a stride included."""
+    """Decode batches of the MoE block at several K of the down stage, rows with a
+    stride included."""
     L = synthetic.make_moe_layer(H, n_exp, inter, seed=21, device=dev)
     L.up_gate_alpha, L.down_alpha = L.up_gate_alpha.to(alpha), L.down_alpha.to(alpha)
     assert tokens * K <= 16 * n_exp  # the decode form
