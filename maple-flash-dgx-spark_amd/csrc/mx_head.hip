@@ -114,10 +114,76 @@ struct MhRaw {
   }
 };
 
+// The FP8 operand of four packed words.
+__device__ __forceinline__ i32x8_t mh_expand(uint4 w) {
+  return i32x8_t{static_cast<int>(w.x & 0x0F0F0F0Fu), static_cast<int>((w.x >> 4) & 0x0F0F0F0Fu),
+                 static_cast<int>(w.y & 0x0F0F0F0Fu), static_cast<int>((w.y >> 4) & 0x0F0F0F0Fu),
+                 static_cast<int>(w.z & 0x0F0F0F0Fu), static_cast<int>((w.z >> 4) & 0x0F0F0F0Fu),
+                 static_cast<int>(w.w & 0x0F0F0F0Fu), static_cast<int>((w.w >> 4) & 0x0F0F0F0Fu)};
+}
+
+// out += sum_g b X for MB x NB blocks of 32 tokens from t0 and the lane's rows:
+// n_groups % 16 == 0; lane half h holds groups 8 h ..+7 of each 16 on both sides.
+template <int MB, int NB>
+__device__ __forceinline__ void mh_bias(const uint16_t* x3, int64_t t0, const uint16_t* biases, const int64_t (&row)[NB],
+                                        int64_t n_groups, f32x16_t (&out)[MB][NB]) {
+  const int lane = threadIdx.x & 63, r32 = lane & 31, h = lane >> 5;
+  for (int64_t g0 = 8 * h; g0 < n_groups; g0 += 16) {
+    uint4 b[NB], xp[MB][3];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) b[nb] = *reinterpret_cast<const uint4*>(biases + row[nb] * n_groups + g0);
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        xp[mb][i] = *reinterpret_cast<const uint4*>(x3 + (3 * (t0 + mb * 32 + r32) + i) * n_groups + g0);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+          out[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mh_bf16x8_t, xp[mb][i]),
+                                                                __builtin_bit_cast(mh_bf16x8_t, b[nb]), out[mb][nb], 0,
+                                                                0, 0);
+  }
+}
+
+// Rows 2j and 2j + 1 of a lane pair's two columns: the even lane stores the
+// first row's two values, the odd lane the second's.
+template <int MB, int NB>
+__device__ __forceinline__ void mh_store(const f32x16_t (&out)[MB][NB], int64_t t0, int64_t n0, int64_t batch,
+                                         int64_t n_out, uint16_t* y, int64_t ldy) {
+  const int lane = threadIdx.x & 63, r32 = lane & 31, h = lane >> 5;
+  const bool packed = (ldy % 2) == 0;
+#pragma unroll
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const float a = out[mb][nb][2 * j], b = out[mb][nb][2 * j + 1];
+        const float o = __shfl_xor((lane & 1) ? a : b, 1, 64);
+        const int i = 2 * j + (lane & 1);
+        const int64_t t = t0 + mb * 32 + 8 * (i / 4) + 4 * h + i % 4;
+        const int64_t n = n0 + 32 * nb + (r32 & ~1);
+        const float v0 = (lane & 1) ? o : a, v1 = (lane & 1) ? b : o;
+        if (t < batch && n < n_out) {
+          uint16_t* dst = y + t * ldy + n;
+          if (packed && n + 1 < n_out) {
+            *reinterpret_cast<uint32_t*>(dst) = pack_bf16x2_rn(v0, v1);
+          } else {
+            dst[0] = f32_to_bf16(v0);
+            if (n + 1 < n_out) dst[1] = f32_to_bf16(v1);
+          }
+        }
+      }
+}
+
 // Bound by the table's bytes up to 64 tokens (151,936 x 2048 in groups of 64:
-// 40 us at 24 tokens for 175 MB, 89 with both launches as bf16 MFMAs), above
-// by the matrix instructions and the folds between them (256 tokens in groups
-// of 128: 203 us, 350 as bf16; the matrix units work 40 % of the time).
+// 57 us both launches at 24 tokens for 175 MB, 90 as bf16 MFMAs), above by the
+// matrix instructions and the folds between them (k_mx_head_ring, and this form
+// where the bias half cannot go to the matrix units).
 //
 // Tiles of 32 MB WT tokens x 32 NB WN table rows, KS groups of 64 per stage;
 // BM: the bias half on the matrix units.  Per stage:
@@ -252,11 +318,7 @@ struct MxHead {
       if (p == 0 && u % MB == 0) {
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) {
-          const uint4 w = r.w[nb][(u / MB) * GPR + g2];
-          bv[g2][nb] = i32x8_t{static_cast<int>(w.x & 0x0F0F0F0Fu), static_cast<int>((w.x >> 4) & 0x0F0F0F0Fu),
-                               static_cast<int>(w.y & 0x0F0F0F0Fu), static_cast<int>((w.y >> 4) & 0x0F0F0F0Fu),
-                               static_cast<int>(w.z & 0x0F0F0F0Fu), static_cast<int>((w.z >> 4) & 0x0F0F0F0Fu),
-                               static_cast<int>(w.w & 0x0F0F0F0Fu), static_cast<int>((w.w >> 4) & 0x0F0F0F0Fu)};
+          bv[g2][nb] = mh_expand(r.w[nb][(u / MB) * GPR + g2]);
         }
       }
       i32x8_t an = av;  // the next operand's reads go out ahead of these products
@@ -327,29 +389,8 @@ struct MxHead {
     Regs nx;
     load(nx, wp, row, scales, biases, n_groups, 0);
     dma(d, 0, ba);
-    if constexpr (BM) {  // n_groups % 16 == 0; lane half h holds groups 8 h ..+7 of each 16 on both sides
-      for (int64_t g0 = 8 * h; g0 < n_groups; g0 += 16) {
-        uint4 bb4[NB], xa4[MB][3];
-#pragma unroll
-        for (int nb = 0; nb < NB; ++nb)
-          bb4[nb] = *reinterpret_cast<const uint4*>(static_cast<const uint16_t*>(biases) + row[nb] * n_groups + g0);
-#pragma unroll
-        for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-          for (int i = 0; i < 3; ++i)
-            xa4[mb][i] = *reinterpret_cast<const uint4*>(
-                x3 + (3 * (t0 + (wt * MB + mb) * 32 + r32) + i) * n_groups + g0);
-#pragma unroll
-        for (int i = 0; i < 3; ++i)
-#pragma unroll
-          for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-            for (int nb = 0; nb < NB; ++nb)
-              out[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(mh_bf16x8_t, xa4[mb][i]),
-                                                                    __builtin_bit_cast(mh_bf16x8_t, bb4[nb]),
-                                                                    out[mb][nb], 0, 0, 0);
-      }
-    }
+    if constexpr (BM)
+      mh_bias<MB, NB>(x3, t0 + wt * MB * 32, static_cast<const uint16_t*>(biases), row, n_groups, out);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
     auto step = [&](int64_t st, const Buf& cur, const Buf& nxt) {
@@ -373,31 +414,7 @@ struct MxHead {
       step(st, ba, bb);
       if (st + 1 < nst) step(st + 1, bb, ba);
     }
-    // rows 2j and 2j + 1 of a lane pair's two columns: the even lane stores
-    // the first row's two values, the odd lane the second's
-    const bool packed = (ldy % 2) == 0;
-#pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-      for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const float a = out[mb][nb][2 * j], b = out[mb][nb][2 * j + 1];
-          const float o = __shfl_xor((lane & 1) ? a : b, 1, 64);
-          const int i = 2 * j + (lane & 1);
-          const int64_t t = t0 + (wt * MB + mb) * 32 + 8 * (i / 4) + 4 * h + i % 4;
-          const int64_t n = n0 + 32 * nb + (r32 & ~1);
-          const float v0 = (lane & 1) ? o : a, v1 = (lane & 1) ? b : o;
-          if (t < batch && n < n_out) {
-            uint16_t* dst = y + t * ldy + n;
-            if (packed && n + 1 < n_out) {
-              *reinterpret_cast<uint32_t*>(dst) = pack_bf16x2_rn(v0, v1);
-            } else {
-              dst[0] = f32_to_bf16(v0);
-              if (n + 1 < n_out) dst[1] = f32_to_bf16(v1);
-            }
-          }
-        }
+    mh_store<MB, NB>(out, t0 + wt * MB * 32, n0, batch, n_out, y, ldy);
   }
 };
 
@@ -415,6 +432,247 @@ __global__ __launch_bounds__(64 * WT * WN) __attribute__((amdgpu_waves_per_eu(WP
   __shared__ __align__(16) float ga[H::kSums * H::kTok], gb[H::kSums * H::kTok];
   H::run(xq, xs, xg, x3, batch, rows, w, n_out, nwords, scales, biases, y, ldy, n_ttiles, n_tiles,
          typename H::Buf{xa, sa, ga}, typename H::Buf{xb, sb, gb});
+}
+
+// The tile of many tokens, 128 x 256 table rows on 8 waves (2 along the tokens,
+// 64 x 64 each): everything a stage of 128 values of K needs -- x rows, table
+// words, row scales, scale bytes -- comes by the LDS DMA two stages ahead, into
+// three buffers (156 KB: one workgroup a CU).  A stage multiplies for about 1 us
+// and its copies take 1 to 2; with one stage ahead the waves waited for them at
+// every barrier.  bf16 scales and biases, the bias half on the matrix units.
+// Both launches, 151,936 x 2048 in groups of 128 (64): 182 us at 256 tokens
+// (201), 350 (551) as bf16 MFMAs, 203 in MxHead's tile of the same size, 194
+// with a unit's fold in one piece; 104 (122) at 96, 124 in MxHead's tile.  The
+// matrix units work 51 % of the time; the vector unit's 9 instructions a product
+// hide behind them in part, and 4.6 tiles a CU leave the last round half empty.
+template <int GW>
+struct MxRing {
+  static constexpr int MB = 2, NB = 2, WT = 2, WN = 4;
+  static constexpr int kTok = 128, kRows = 256, kThreads = 512, KS = 2, NBUF = 3;
+  static constexpr int kSums = KS * mh::kGroupWords / GW, GPR = GW / mh::kGroupWords;
+  static constexpr int kCh = mh::kGroupChunks * KS;  // of a token per stage
+  // dwords of a buffer: x rows, table words, then each wave's own scale bytes
+  // (64 words, all tokens) and row scales (64 rows)
+  static constexpr int kX = kTok * kCh * 4, kW = kRows * 16, kS = 8 * 64, kBuf = kX + kW + 2 * kS;
+  static constexpr int kCopies = 4 + 2 + 1 + 1;  // per wave and stage
+
+  const uint4* xq;
+  int64_t ld, rows;
+  const uint8_t* xs;
+  const uint32_t* w;
+  uint32_t woff[2];  // this thread's table copies
+  const uint16_t* sc;  // scales of the lane's row of the wave's 64
+
+  // x: token p's chunk c at slot p kCh + (c ^ p % 16); table row r's chunk c (4
+  // words) at slot 4 r + (c ^ r / 4 % 4): a wave's reads of one chunk fall on
+  // different banks
+  __device__ __forceinline__ void copy(int64_t st, uint32_t* buf) const {
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int PER = kThreads / kCh;
+    const int p0 = tid / kCh;
+#pragma unroll
+    for (int i = 0; i < kTok / PER; ++i) {
+      const int c = (tid % kCh) ^ ((p0 + PER * i) % 16);
+      const uint4* base = xq + PER * i * ld + st * kCh;  // the same in every lane
+      __builtin_amdgcn_global_load_lds(base + static_cast<uint32_t>(p0 * static_cast<int>(ld) + c),
+                                       (mh_lds_t)(buf + 4 * (64 * wv + kThreads * i)), 16, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_global_load_lds(w + st * 16 + woff[i], (mh_lds_t)(buf + kX + 4 * (64 * wv + kThreads * i)), 16, 0,
+                                       0);
+    __builtin_amdgcn_global_load_lds(
+        reinterpret_cast<const uint32_t*>(xs + (st * KS + (lane >> 5)) * rows) + (lane & 31),
+        (mh_lds_t)(buf + kX + kW + 64 * wv), 4, 0, 0);
+    // the word that holds the stage's scales (n_groups is even)
+    __builtin_amdgcn_global_load_lds(reinterpret_cast<const uint32_t*>(sc + (st * kSums & ~int64_t{1})),
+                                     (mh_lds_t)(buf + kX + kW + kS + 64 * wv), 4, 0, 0);
+  }
+
+  // A stage's products, each unit's (an RTN group of a token block) followed by
+  // a part of the unit before's fold: the vector unit folds while the matrix
+  // unit multiplies (folding a unit in one piece, the two took turns).  acc[1]
+  // and sp (its scales) carry the last unit over to the next stage.
+  template <typename F>
+  static __device__ __forceinline__ void multiply(const uint32_t* buf, int64_t st, int wv, f32x16_t (&out)[MB][NB],
+                                                  f32x16_t (&acc)[2][NB], float (&sp)[NB], F&& send) {
+    const int lane = threadIdx.x & 63, r32 = lane & 31, h = lane >> 5, wt = wv % WT, wn = wv / WT;
+    const char* const b8 = reinterpret_cast<const char*>(buf);
+    uint32_t off[MB];
+#pragma unroll
+    for (int mb = 0; mb < MB; ++mb) {
+      const int p = (wt * MB + mb) * 32 + r32;
+      off[mb] = static_cast<uint32_t>(p * kCh + ((2 * h) ^ (p % 16))) * 16;
+      asm volatile("" : "+v"(off[mb]));  // recomputed per stage: hoisted, every read's address takes a register
+    }
+    uint4 w[KS][NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      const int r = wn * 64 + 32 * nb + r32;
+#pragma unroll
+      for (int gi = 0; gi < KS; ++gi)
+        w[gi][nb] = *reinterpret_cast<const uint4*>(buf + kX + 4 * (4 * r + ((2 * gi + h) ^ (r / 4 % 4))));
+    }
+    uint32_t sw[NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) sw[nb] = buf[kX + kW + kS + 64 * wv + 32 * nb + r32];
+    constexpr int U = kSums * MB;
+    const uint8_t* const s8 = reinterpret_cast<const uint8_t*>(buf + kX + kW + 64 * wv);
+    auto scale = [&](int u, int g2) {
+      return static_cast<int>(s8[((u / MB) * GPR + g2) * kTok + (wt * MB + u % MB) * 32 + r32]);
+    };
+    auto read = [&](int j) {  // piece j % 2 of group j / 2 % GPR of unit j / 2 / GPR
+      const int u = j / 2 / GPR;
+      const uint32_t c = (((u / MB) * GPR + j / 2 % GPR) * 8 + (j % 2) * 4) * 16;
+      return mx_operand(*reinterpret_cast<const uint4*>(b8 + (off[u % MB] ^ c)),
+                        *reinterpret_cast<const uint4*>(b8 + (off[u % MB] ^ (c + 16))));
+    };
+    i32x8_t bv[GPR][NB];
+    float s[kSums][NB];
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) {
+      if constexpr (kSums == 2) {
+        s[0][nb] = __uint_as_float(sw[nb] << 16);
+        s[kSums - 1][nb] = __uint_as_float(sw[nb] & 0xffff0000u);
+      } else {
+        s[0][nb] = __uint_as_float((st & 1) ? (sw[nb] & 0xffff0000u) : (sw[nb] << 16));
+      }
+    }
+    // part q of kParts of the fold of the unit before unit u
+    constexpr int kParts = 2 * GPR * NB, kPer = 16 * NB / kParts;
+    auto fold = [&](int u, int q) {
+      const int up = u == 0 ? U - 1 : u - 1, mb = up % MB, nb = q * kPer / 16;
+      const float f = u == 0 ? sp[nb] : s[up / MB][nb];
+#pragma unroll
+      for (int i = 0; i < kPer; ++i) {
+        const int e = q * kPer % 16 + i;
+        out[mb][nb][e] = __builtin_fmaf(f, acc[up & 1][nb][e], out[mb][nb][e]);
+      }
+    };
+    int sa = scale(0, 0);
+    i32x8_t av = read(0);
+#pragma unroll
+    for (int j = 0; j < 2 * GPR * U; ++j) {
+      const int u = j / 2 / GPR, g2 = j / 2 % GPR, p = j % 2;
+      if (p == 0 && u % MB == 0) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) bv[g2][nb] = mh_expand(w[(u / MB) * GPR + g2][nb]);
+      }
+      i32x8_t an = av;  // the next operand's reads go out ahead of these products
+      int sn = sa;
+      if (j + 1 < 2 * GPR * U) {
+        an = read(j + 1);
+        if (p == 1) sn = scale((j + 1) / 2 / GPR, (j + 1) / 2 % GPR);
+      }
+      MA_ISSUE_FENCE();
+#pragma unroll
+      for (int nb = 0; nb < NB; ++nb) {
+        if (g2 == 0 && p == 0) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) acc[u & 1][nb][i] = 0.f;
+        }
+        acc[u & 1][nb] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(av, bv[g2][nb], acc[u & 1][nb], 0, 0, 0, sa, 0,
+                                                                         136 - 4 * p);
+        asm volatile("" : "+v"(acc[u & 1][nb])::"memory");  // one operand's reads at a time (mx_pin)
+        fold(u, (g2 * 2 + p) * NB + nb);
+        MA_ISSUE_FENCE();
+      }
+      if (j == 0) {
+        MA_ISSUE_FENCE();
+        send();
+        MA_ISSUE_FENCE();
+      }
+      av = an;
+      sa = sn;
+    }
+#pragma unroll
+    for (int nb = 0; nb < NB; ++nb) sp[nb] = s[kSums - 1][nb];
+  }
+
+  // As MxTile::step (mx_gemm.hip): wait for stage st's copies, meet, send a
+  // later stage's into the buffer just freed, multiply.
+  template <bool TAIL>
+  __device__ __forceinline__ void step(int64_t st, int64_t nst, const uint32_t* cur, uint32_t* prev, int wv,
+                                       f32x16_t (&out)[MB][NB], f32x16_t (&acc)[2][NB], float (&sp)[NB]) const {
+    if (!TAIL || st + NBUF - 1 < nst) __builtin_amdgcn_s_waitcnt(mh_vmcnt((NBUF - 2) * kCopies));
+    else __builtin_amdgcn_s_waitcnt(mh_vmcnt(0));
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    multiply(cur, st, wv, out, acc, sp, [&]() {
+      if (!TAIL || st + NBUF - 1 < nst) copy(st + NBUF - 1, prev);
+    });
+    MA_ISSUE_FENCE();
+  }
+};
+
+template <int GW>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_mx_head_ring(
+    const uint4* __restrict__ xq, const uint8_t* __restrict__ xs, const uint16_t* __restrict__ x3, int64_t batch,
+    int64_t rows, const uint32_t* __restrict__ w, int64_t n_out, int64_t nwords, const uint16_t* __restrict__ scales,
+    const uint16_t* __restrict__ biases, uint16_t* __restrict__ y, int64_t ldy, int n_ttiles, int n_tiles) {
+  using R = MxRing<GW>;
+  __shared__ __align__(16) uint32_t b0[R::kBuf], b1[R::kBuf], b2[R::kBuf];
+  const int per = (n_tiles + kXcds - 1) / kXcds;
+  const int local = static_cast<int>(blockIdx.x) / kXcds;
+  const int idx = (static_cast<int>(blockIdx.x) % kXcds) * per + local;
+  if (local >= per || idx >= n_tiles) return;
+  const int tid = threadIdx.x, lane = tid & 63, r32 = lane & 31, h = lane >> 5;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wt = wv % R::WT, wn = wv / R::WT;
+  const int64_t t0 = static_cast<int64_t>(idx % n_ttiles) * R::kTok;
+  const int64_t r0 = static_cast<int64_t>(idx / n_ttiles) * R::kRows, n0 = r0 + 64 * wn;
+  const int64_t nst = nwords / 16, n_groups = nwords / GW;
+  const int64_t ld = nwords / mh::kGroupWords * mh::kGroupChunks;
+  R t{xq + t0 * ld, ld, rows, xs + t0, w + r0 * nwords, {0u, 0u}, nullptr};
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    const int r = (tid + 512 * i) / 4, c = (tid % 4) ^ (r / 4 % 4);
+    const int rc = r0 + r < n_out ? r : static_cast<int>(n_out - 1 - r0);  // past n_out: its last row
+    t.woff[i] = static_cast<uint32_t>(rc * nwords + 4 * c);
+  }
+  t.sc = scales + (n0 + lane < n_out ? n0 + lane : n_out - 1) * n_groups;
+  f32x16_t out[R::MB][R::NB];
+#pragma unroll
+  for (int mb = 0; mb < R::MB; ++mb)
+#pragma unroll
+    for (int nb = 0; nb < R::NB; ++nb)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) out[mb][nb][i] = 0.f;
+  int64_t row[R::NB];
+#pragma unroll
+  for (int nb = 0; nb < R::NB; ++nb) row[nb] = n0 + 32 * nb + r32 < n_out ? n0 + 32 * nb + r32 : n_out - 1;
+  mh_bias<R::MB, R::NB>(x3, t0 + wt * 64, biases, row, n_groups, out);
+  MA_ISSUE_FENCE();
+  t.copy(0, b0);
+  MA_ISSUE_FENCE();
+  t.copy(1, b1);  // nst is even
+  MA_ISSUE_FENCE();
+  // (no unit before the first: its fold adds 0 x 0)
+  f32x16_t acc[2][R::NB];
+  float sp[R::NB];
+#pragma unroll
+  for (int nb = 0; nb < R::NB; ++nb) {
+    sp[nb] = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[1][nb][i] = 0.f;
+  }
+  int64_t st = 0;
+  for (; st + 5 <= nst; st += 3) {
+    t.template step<false>(st, nst, b0, b2, wv, out, acc, sp);
+    t.template step<false>(st + 1, nst, b1, b0, wv, out, acc, sp);
+    t.template step<false>(st + 2, nst, b2, b1, wv, out, acc, sp);
+  }
+  if (st < nst) t.template step<true>(st, nst, b0, b2, wv, out, acc, sp);
+  if (st + 1 < nst) t.template step<true>(st + 1, nst, b1, b0, wv, out, acc, sp);
+  if (st + 2 < nst) t.template step<true>(st + 2, nst, b2, b1, wv, out, acc, sp);
+  if (st + 3 < nst) t.template step<true>(st + 3, nst, b0, b2, wv, out, acc, sp);
+#pragma unroll
+  for (int nb = 0; nb < R::NB; ++nb)
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      out[R::MB - 1][nb][i] = __builtin_fmaf(sp[nb], acc[1][nb][i], out[R::MB - 1][nb][i]);
+  mh_store<R::MB, R::NB>(out, t0 + wt * 64, n0, batch, n_out, y, ldy);
 }
 
 static int64_t mx_head_rows(int64_t batch) { return cdiv(batch, mh::kPad) * mh::kPad; }
@@ -449,30 +707,49 @@ int launch_rtn4_mx(const uint16_t* x, int64_t batch, int64_t ldx, const uint32_t
                        static_cast<int>(tiles));                                                                     \
   } while (0)
 // Tile by batch: 32 or 64 tokens x 128 rows while the table's bytes are the
-// bound (151,936 rows, groups of 64: 57 us at 24 tokens, 74 at 64); 128 tokens
-// x 128 rows up to one such token tile (118 us at 128 tokens in groups of 128,
-// 127 with 256 rows), x 256 rows above (203 against 217 at 256: half the x
-// rows' traffic).
-#define MA_MH_T(GW, SDT, BM)                  \
-  if (batch <= 32)                            \
-    MA_MH(1, 1, 1, 4, 4, GW, SDT, BM, 3);     \
-  else if (batch <= 64)                       \
-    MA_MH(2, 1, 1, 4, 2, GW, SDT, BM, 3);     \
-  else if (batch <= 128)                      \
-    MA_MH(2, 2, 2, 2, 2, GW, SDT, BM, 2);     \
-  else                                        \
-    MA_MH(2, 2, 2, 4, 2, GW, SDT, BM, 2);
-#define MA_MH_G(SDT, BM) \
-  if (group == 64) { MA_MH_T(8, SDT, BM) } else { MA_MH_T(16, SDT, BM) }
+// bound (151,936 rows, groups of 64: 57 us at 24 tokens, 75 at 64); past 64 the
+// ring's 128 x 256 (at 128 tokens in groups of 128 114 us, 118 in a tile of 128
+// x 128, 127 with the ring's size and two buffers).  The ring needs the bias
+// half's product, whole steps of 16 bf16 groups; without it 128 x 128 rows up to
+// one such token tile, x 256 above (203 against 217 at 256: half the x rows'
+// traffic).
+#define MA_MH_S(GW, SDT, BM)              \
+  if (batch <= 32)                        \
+    MA_MH(1, 1, 1, 4, 4, GW, SDT, BM, 3); \
+  else                                    \
+    MA_MH(2, 1, 1, 4, 2, GW, SDT, BM, 3);
+#define MA_MH_T(GW, SDT)                     \
+  if (batch <= 64) {                         \
+    MA_MH_S(GW, SDT, false)                  \
+  } else if (batch <= 128)                   \
+    MA_MH(2, 2, 2, 2, 2, GW, SDT, false, 2); \
+  else                                       \
+    MA_MH(2, 2, 2, 4, 2, GW, SDT, false, 2);
+#define MA_MR(G64)                                                                                                     \
+  const int64_t tt = cdiv(batch, 128), tiles = tt * cdiv(n_out, 256);                                                \
+  auto* const kernel = (G64) ? &k_mx_head_ring<8> : &k_mx_head_ring<16>;                                             \
+  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(cdiv(tiles, kXcds) * kXcds)), dim3(512), 0, s, xq, xs, x3,    \
+                     batch, rows, w, n_out, nwords, static_cast<const uint16_t*>(scales),                            \
+                     static_cast<const uint16_t*>(biases), y, ldy, static_cast<int>(tt), static_cast<int>(tiles));
+#define MA_MH_G(SDT) \
+  if (group == 64) { MA_MH_T(8, SDT) } else { MA_MH_T(16, SDT) }
   if (s_dt == MA_F32) {
-    MA_MH_G(MA_F32, false)
+    MA_MH_G(MA_F32)
   } else if (nwords / gw % 16 == 0) {
-    MA_MH_G(MA_BF16, true)
+    if (batch > 64) {
+      MA_MR(group == 64)
+    } else if (group == 64) {
+      MA_MH_S(8, MA_BF16, true)
+    } else {
+      MA_MH_S(16, MA_BF16, true)
+    }
   } else {
-    MA_MH_G(MA_BF16, false)
+    MA_MH_G(MA_BF16)
   }
 #undef MA_MH_G
+#undef MA_MR
 #undef MA_MH_T
+#undef MA_MH_S
 #undef MA_MH
   return check_launch("rtn4_gemv (mx)");
 }
