@@ -14,7 +14,7 @@ constexpr int kRows = 128;     // weight rows per tile, 64 a wave
 constexpr int kWords = 8;      // packed words per step
 }  // namespace mx
 
-constexpr int kMxTok = 64;  // tokens per tile; the workspace's rows are padded to it
+constexpr int kMxTok = 64;  // tokens of the larger tile; the workspace's rows are padded to it
 
 // One token per workgroup: x (times w_rms) as an mx row of NP pieces, xs[t *
 // s_row + step * s_step] its scale bytes, xc[t] = (sum x_hat, RMS factor) with the sums in a
@@ -99,12 +99,15 @@ constexpr int mx_vmcnt(int n) { return (n & 0xF) | (0x7 << 4) | ((n >> 4) << 14)
 // step's copies come mostly from memory that another XCD wrote: a call of 64
 // tokens at K = 2048 took 20 us with one step ahead, 16.7 with two).  The
 // operands need two ANDs and a shift a word, so a tile is bound by the matrix
-// instructions and the steps' fixed parts: 2048 tokens x 2048 -> 2560 take 32.7
-// us (208 as bf16 MFMAs of 16-row tiles, which read each token's operands 160
-// times), 55.5 with the RMSNorm (149), 777 x 2048 -> 2048 18.7 (68).
+// instructions and the steps' fixed parts: both launches for 2048 tokens x 2048
+// -> 2560 take 32.3 us (208 as bf16 MFMAs of 16-row tiles, which read each
+// token's operands 160 times), 49.3 with the RMSNorm (149), 777 x 2048 -> 2048
+// 16.9 (68).
 template <int NP, int TOK, int NBUF>
 struct MxTile {
-  static_assert(TOK == 64, "a wave's lanes copy the tile's scale words");
+  // (a wave's lanes copy 64 scale words; those past a tile of 32 tokens are the
+  // next tokens' or, past the last step's rows, the sums that follow them)
+  static_assert(TOK == 64 || TOK == 32, "tokens");
   static constexpr int kNb = TOK / 32, kCh = 8 * NP;
   static constexpr int kXDwords = TOK * kCh * 4, kWDwords = mx::kRows * mx::kWords;
   static constexpr int kBuf = kXDwords + kWDwords + 4 * 64;  // one step: rows, weights, each wave's scale words
@@ -305,25 +308,48 @@ int launch_tgemm_mx(const uint16_t* x, int64_t batch, int64_t ldx, const uint32_
   uint32_t* xs = reinterpret_cast<uint32_t*>(xq + rows * nwords * np);
   float2* xc = reinterpret_cast<float2*>(xs + rows * nsteps);
   const int64_t n_rtiles = cdiv(n_out, mx::kRows);
-  const int64_t n_tiles = n_rtiles * cdiv(batch, kMxTok);
-  const dim3 grid(static_cast<unsigned>(cdiv(n_tiles, kXcds) * kXcds));
-#define MA_MX(NP, NBUF, ADT)                                                                                     \
-  hipLaunchKernelGGL((k_mx_gemm<NP, kMxTok, NBUF, ADT>), grid, dim3(mx::kThreads), 0, s, xq, xs, xc, batch, rows, w, n_out, \
-                     nwords, alpha, y, ldy, static_cast<int>(n_rtiles), static_cast<int>(n_tiles))
+  const int64_t n64 = n_rtiles * cdiv(batch, 64), n32 = n_rtiles * cdiv(batch, 32);
+#define MA_MX1(NP, TOK, NBUF, ADT)                                                                                   \
+  hipLaunchKernelGGL((k_mx_gemm<NP, TOK, NBUF, ADT>),                                                                \
+                     dim3(static_cast<unsigned>(cdiv(TOK == 64 ? n64 : n32, kXcds) * kXcds)), dim3(mx::kThreads), 0, \
+                     s, xq, xs, xc, batch, rows, w, n_out, nwords, alpha, y, ldy, static_cast<int>(n_rtiles),        \
+                     static_cast<int>(TOK == 64 ? n64 : n32))
+#define MA_MX(NP, TOK, NBUF) \
+  if (alpha_dt == MA_F32) MA_MX1(NP, TOK, NBUF, MA_F32); else MA_MX1(NP, TOK, NBUF, MA_BF16)
+  // Tiles of 32 tokens instead of 64 take about 0.6 of the time each and more of
+  // them fit on a CU, so they win wherever that saves a pass over the chip or
+  // spreads a small call over more of it.
   if (rms_w) {
     hipLaunchKernelGGL((k_mx_prep<4, false>), dim3(static_cast<unsigned>(batch)), dim3(128), 0, s, x, ldx, nwords, rms_w,
                        rms_dt, rms_eps, int64_t{1}, rows, xq, xs, xc, cb);
-    if (alpha_dt == MA_F32) MA_MX(4, 2, MA_F32); else MA_MX(4, 2, MA_BF16);
+    // 32 tokens with three buffers (two a CU) in one pass, with two buffers (three
+    // a CU) as long as that takes no more passes than 64 tokens (two a CU).  K =
+    // 2048, us: 256 x 2560 16.6 / 18.4 / 24.3 in that order, 777 x 2560 25.3 / 26.0
+    // / 36.2, 1024 x 2560 34.2 / 30.2 / 36.3, 1344 x 2560 41.5 / 41.1 / 39.2, 2048
+    // x 2560 52.4 / 49.3 / 54.7, 1536 x 5120 69.1 / 67.7 / 65.9, 2048 x 5120 86.4 /
+    // 84.1 / 79.2; at K = 4096 alike (1024 x 2560 - / 49.0 / 58.9, 2048 x 5120 - /
+    // 151 / 141).
+    if (n32 <= 512) {
+      MA_MX(4, 32, 3);
+    } else if (cdiv(n32, 768) <= cdiv(n64, 512)) {
+      MA_MX(4, 32, 2);
+    } else {
+      MA_MX(4, 64, 2);
+    }
   } else {
     hipLaunchKernelGGL((k_mx_prep<2, false>), dim3(static_cast<unsigned>(batch)), dim3(128), 0, s, x, ldx, nwords,
                        nullptr, 0, 0.f, int64_t{1}, rows, xq, xs, xc, CombineIn{});
-    // up to two workgroups a CU, three buffers; with more, two (three fit on a CU: one pass over 768 tiles)
-    if (n_tiles <= 512) {
-      if (alpha_dt == MA_F32) MA_MX(2, 3, MA_F32); else MA_MX(2, 3, MA_BF16);
+    // 32 tokens with three buffers (four a CU) in one pass, else 64 with two
+    // (three a CU).  K = 2048, us: 128 x 2560 12.8 / 16.4, 777 x 2048 16.9 / 19.3,
+    // 777 x 5120 26.4 / 30.3, 1536 x 2560 26.5 / 25.8, 2048 x 2048 27.7 / 28.5, past
+    // it 1664 x 2560 31.7 / 30.4, 2048 x 5120 55.6 / 49.9.
+    if (n32 <= 1024) {
+      MA_MX(2, 32, 3);
     } else {
-      if (alpha_dt == MA_F32) MA_MX(2, 2, MA_F32); else MA_MX(2, 2, MA_BF16);
+      MA_MX(2, 64, 2);
     }
   }
+#undef MA_MX1
 #undef MA_MX
   return check_launch("ternary_gemv (mx)");
 }

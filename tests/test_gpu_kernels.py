@@ -364,10 +364,12 @@ def test_gemv_two_launch_small_workspace_raises(dev):
 @pytest.mark.parametrize("tokens,n_out,k_in,rms,alpha", [
     (64, 5120, 256, None, torch.bfloat16),         # the fewest tokens, one pass over the step buffers
     (65, 5129, 768, None, torch.float32),          # ragged tokens and rows, odd row count, 6 steps
-    (513, 2056, 2048, None, torch.bfloat16),       # two buffers (over 512 tiles would be; here three)
-    (2049, 2050, 256, None, torch.float32),        # over 512 tiles
+    (513, 2056, 2048, None, torch.bfloat16),       # 17 tiles of 32 tokens, the last of one
+    (2049, 2050, 256, None, torch.float32),        # tiles of 64 tokens (over 1024 of 32)
     (129, 4600, 512, torch.float32, torch.bfloat16),
     (290, 2056, 1280, torch.bfloat16, torch.float32),  # 10 steps
+    (545, 5113, 256, torch.float32, torch.bfloat16),   # with the RMSNorm: two buffers, 720 tiles of 32 tokens
+    (705, 5120, 512, torch.bfloat16, torch.float32),   # 480 tiles of 64 (920 of 32 would take a second pass)
 ])
 def test_gemv_mx_vs_oracle(dev, tokens, n_out, k_in, rms, alpha):
     """Projections of many tokens (ma_ternary_gemv_ws's scaled 8-bit form) at the
