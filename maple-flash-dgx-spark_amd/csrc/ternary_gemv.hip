@@ -118,13 +118,14 @@ constexpr int64_t kXpMinBatch = 17;
 constexpr int64_t kMxMinBatch = 64;
 
 // Where that form is the faster one: the others cost in proportion to tokens x
-// rows, this one about 17 us (24 with the RMSNorm) up to 512 tokens at K = 2048.
-// They cross near 5 x 2^16 outputs (128 tokens of 2560 rows 18.1 against 16.5
-// us, 128 of 2048 12.8 against 16.7, 512 of 1024 24.5 against 17.3) and with
-// the RMSNorm near 9 x 2^16 (256 of 2560 26.7 against 23.9, 96 of 5120 21.4
-// against 23.3, 512 of 1024 26.6 against 25.1); at K = 768 and 4096 alike.
-static bool mx_faster(int64_t batch, int64_t n_out, bool rms) {
-  return batch >= kMxMinBatch && batch * n_out >= (rms ? 9 : 5) * int64_t{65536};
+// rows, this one about 13 us (16 with the RMSNorm) up to 256 tokens of 2560 rows
+// at K = 2048.  They cross near 4 x 2^16 outputs, us: 128 tokens of 2048 rows
+// 12.7 against 12.6 (with the RMSNorm 14.1 against 16.4), 112 of 2560 17.0
+// against 12.5 (17.0, 16.2), 288 of 1024 16.9 against 13.1 (19.2, 17.6), 512 of
+// 1024 with the RMSNorm 25.9 against 17.8; at K = 768 and 4096 alike (112 of 2560
+// 8.8 against 8.4 and 23.8 against 19.4).
+static bool mx_faster(int64_t batch, int64_t n_out) {
+  return batch >= kMxMinBatch && batch * n_out > int64_t{4} * 65536;
 }
 
 static bool mfma_ok(const void* x, int x_dtype, int64_t batch, int64_t ldx, const uint32_t* packed,
@@ -186,7 +187,7 @@ extern "C" int ma_ternary_gemv_ws(const void* x, int x_dtype, int64_t batch, int
   const bool mfma = mfma_ok(x, x_dtype, batch, ldx, packed, nwords, packed_kn, alpha_dtype, rms_weight,
                             rms_dtype, y);
   // (a workspace of less than the query's bytes still takes the forms that need less)
-  if (mfma && mx_faster(batch, n_out, rms_weight != nullptr) && workspace && !(reinterpret_cast<uintptr_t>(workspace) & 255) &&
+  if (mfma && mx_faster(batch, n_out) && workspace && !(reinterpret_cast<uintptr_t>(workspace) & 255) &&
       workspace_bytes >= tgemm_mx_bytes(batch, nwords, rms_weight != nullptr))
     return launch_tgemm_mx(static_cast<const uint16_t*>(x), batch, ldx, packed, n_out, nwords, row_alpha,
                            alpha_dtype, rms_weight, rms_dtype, rms_eps, static_cast<uint16_t*>(y), ldy, workspace,
@@ -239,7 +240,7 @@ extern "C" int ma_ternary_gemv_combine_ws(const void* slot_out, const int32_t* i
   const CombineIn cb{static_cast<const uint16_t*>(slot_out), inverse, topk_weight,
                      static_cast<int>(top_k), static_cast<const uint16_t*>(residual),
                      static_cast<uint16_t*>(x_out)};
-  if (mx_faster(batch, n_out, true) && workspace_bytes >= tgemm_mx_bytes(batch, nwords, true))
+  if (mx_faster(batch, n_out) && workspace_bytes >= tgemm_mx_bytes(batch, nwords, true))
     return launch_tgemm_mx(static_cast<const uint16_t*>(x_out), batch, nwords * 16, packed, n_out, nwords, row_alpha,
                            alpha_dtype, rms_weight, rms_dtype, rms_eps, static_cast<uint16_t*>(y), ldy, workspace,
                            static_cast<hipStream_t>(stream), cb);
