@@ -20,16 +20,25 @@ constexpr int kMxTok = 64;  // tokens of the larger tile; the workspace's rows a
 // s_row + step * s_step] its scale bytes, xc[t] = (sum x_hat, RMS factor) with the sums in a
 // fixed order.  Two pieces hold bf16 x; the RMS-folded product is float32 and
 // takes four, which is no less than the two bf16 numbers of the smaller
-// batches' operands (relative 2^-19 against 2^-17).  Latency: about
-// 5 us for 2048 x 2048 with two pieces and 8 with four (16 MB written).  With a MoE combine in front (cb.slot_out
+// batches' operands (relative 2^-19 against 2^-17).  Latency: about 5 us for 2048
+// x 2048 with two pieces and 8 with four (16 MB written).  XCD x takes the
+// tokens of its eighth, whose tiles it multiplies too (k_mx_gemm), and a step's
+// scale word is one store: with tokens dealt to the XCDs in turn and a byte a
+// block, a line of scale words was written by all eight (both launches for 2048
+// tokens at K = 2048: 27.2 -> 23.9 us to 2048 rows, with the RMSNorm 48.7 -> 45.1
+// to 2560 and 31.5 -> 26.1 to 1024).  (WIDE rows are gathered
+// by expert from every XCD: in order.)  With a MoE combine in front (cb.slot_out
 // set, NP 4) the rows are combined first instead of read from x.
 template <int NP, bool WIDE>
 __global__ __launch_bounds__(128) void k_mx_prep(const uint16_t* __restrict__ x, int64_t ldx, int64_t nwords,
                                                  const void* __restrict__ rms_w, int rms_dt, float rms_eps,
                                                  int64_t s_row, int64_t s_step, uint4* __restrict__ xq,
-                                                 uint32_t* __restrict__ xs, float2* __restrict__ xc, CombineIn cb) {
+                                                 uint32_t* __restrict__ xs, float2* __restrict__ xc, int64_t tokens,
+                                                 CombineIn cb) {
   __shared__ float red_c[2], red_s[2];
-  const int64_t t = blockIdx.x;
+  const int64_t t = WIDE ? static_cast<int64_t>(blockIdx.x)
+                         : static_cast<int64_t>(blockIdx.x % kXcds) * (gridDim.x / kXcds) + blockIdx.x / kXcds;
+  if (t >= tokens) return;
   const int tid = threadIdx.x;
   const int64_t nsteps = nwords / mx::kWords;
   float c = 0.f, ss = 0.f;
@@ -75,8 +84,12 @@ __global__ __launch_bounds__(128) void k_mx_prep(const uint16_t* __restrict__ x,
     uint4* dst = xq + (t * nsteps + step) * (8 * NP) + pos;
 #pragma unroll
     for (int p = 0; p < NP; ++p) dst[8 * p] = out[p];
-    if ((wd & 1) == 0)
-      reinterpret_cast<uint8_t*>(xs + t * s_row + step * s_step)[pos / 2] = static_cast<uint8_t>(mx_scale_byte(e));
+    // the step's scale word: its first lane takes the other blocks' bytes
+    constexpr int kStepBit = WIDE ? 4 : 2;
+    uint32_t sw = mx_scale_byte(e) << (8 * (pos / 2));
+    sw |= __shfl_xor(sw, kStepBit, 64);
+    sw |= __shfl_xor(sw, 2 * kStepBit, 64);
+    if (pos == 0) xs[t * s_row + step * s_step] = sw;
   }
   c = group_sum<64>(c);
   ss = group_sum<64>(ss);
@@ -100,9 +113,9 @@ constexpr int mx_vmcnt(int n) { return (n & 0xF) | (0x7 << 4) | ((n >> 4) << 14)
 // tokens at K = 2048 took 20 us with one step ahead, 16.7 with two).  The
 // operands need two ANDs and a shift a word, so a tile is bound by the matrix
 // instructions and the steps' fixed parts: both launches for 2048 tokens x 2048
-// -> 2560 take 32.3 us (208 as bf16 MFMAs of 16-row tiles, which read each
-// token's operands 160 times), 49.3 with the RMSNorm (149), 777 x 2048 -> 2048
-// 16.9 (68).
+// -> 2560 take 28.4 us (208 as bf16 MFMAs of 16-row tiles, which read each
+// token's operands 160 times), 45.1 with the RMSNorm (149), 777 x 2048 -> 2048
+// 16.1 (68).
 template <int NP, int TOK, int NBUF>
 struct MxTile {
   // (a wave's lanes copy 64 scale words; those past a tile of 32 tokens are the
@@ -284,7 +297,8 @@ __global__ __launch_bounds__(mx::kThreads) __attribute__((amdgpu_waves_per_eu(2,
 void launch_mx_prep_wide(const uint16_t* x, int64_t ldx, int64_t tokens, int64_t nwords, uint32_t* xq, uint32_t* xs,
                          float2* xc, hipStream_t s) {
   hipLaunchKernelGGL((k_mx_prep<2, true>), dim3(static_cast<unsigned>(tokens)), dim3(128), 0, s, x, ldx, nwords, nullptr,
-                     0, 0.f, nwords / mx::kWords, int64_t{1}, reinterpret_cast<uint4*>(xq), xs, xc, CombineIn{});
+                     0, 0.f, nwords / mx::kWords, int64_t{1}, reinterpret_cast<uint4*>(xq),
+                     xs, xc, tokens, CombineIn{});
 }
 
 }  // namespace ma
@@ -308,6 +322,7 @@ int launch_tgemm_mx(const uint16_t* x, int64_t batch, int64_t ldx, const uint32_
   uint32_t* xs = reinterpret_cast<uint32_t*>(xq + rows * nwords * np);
   float2* xc = reinterpret_cast<float2*>(xs + rows * nsteps);
   const int64_t n_rtiles = cdiv(n_out, mx::kRows);
+  const dim3 grid(static_cast<unsigned>(cdiv(batch, kXcds) * kXcds));
   const int64_t n64 = n_rtiles * cdiv(batch, 64), n32 = n_rtiles * cdiv(batch, 32);
 #define MA_MX1(NP, TOK, NBUF, ADT)                                                                                   \
   hipLaunchKernelGGL((k_mx_gemm<NP, TOK, NBUF, ADT>),                                                                \
@@ -320,8 +335,8 @@ int launch_tgemm_mx(const uint16_t* x, int64_t batch, int64_t ldx, const uint32_
   // them fit on a CU, so they win wherever that saves a pass over the chip or
   // spreads a small call over more of it.
   if (rms_w) {
-    hipLaunchKernelGGL((k_mx_prep<4, false>), dim3(static_cast<unsigned>(batch)), dim3(128), 0, s, x, ldx, nwords, rms_w,
-                       rms_dt, rms_eps, int64_t{1}, rows, xq, xs, xc, cb);
+    hipLaunchKernelGGL((k_mx_prep<4, false>), grid, dim3(128), 0, s, x, ldx, nwords, rms_w, rms_dt, rms_eps,
+                       int64_t{1}, rows, xq, xs, xc, batch, cb);
     // 32 tokens with three buffers (two a CU) in one pass, with two buffers (three
     // a CU) as long as that takes no more passes than 64 tokens (two a CU).  K =
     // 2048, us: 256 x 2560 16.6 / 18.4 / 24.3 in that order, 777 x 2560 25.3 / 26.0
@@ -337,8 +352,8 @@ int launch_tgemm_mx(const uint16_t* x, int64_t batch, int64_t ldx, const uint32_
       MA_MX(4, 64, 2);
     }
   } else {
-    hipLaunchKernelGGL((k_mx_prep<2, false>), dim3(static_cast<unsigned>(batch)), dim3(128), 0, s, x, ldx, nwords,
-                       nullptr, 0, 0.f, int64_t{1}, rows, xq, xs, xc, CombineIn{});
+    hipLaunchKernelGGL((k_mx_prep<2, false>), grid, dim3(128), 0, s, x, ldx, nwords, nullptr, 0, 0.f,
+                       int64_t{1}, rows, xq, xs, xc, batch, CombineIn{});
     // 32 tokens with three buffers (four a CU) in one pass, else 64 with two
     // (three a CU).  K = 2048, us: 128 x 2560 12.8 / 16.4, 777 x 2048 16.9 / 19.3,
     // 777 x 5120 26.4 / 30.3, 1536 x 2560 26.5 / 25.8, 2048 x 2048 27.7 / 28.5, past
