@@ -916,8 +916,11 @@ static int64_t attn_grid_splits(int64_t batch, int nkv, int64_t max_len, int64_t
 // device at once: their number is capped at the kernel's resident capacity
 // (compute units x occupancy).  Workgroups are dispatched in index order and a
 // (row, KV head)'s splits are consecutive, so every earlier pair has all of
-// its splits placed and finishes; with the O projection in the launch the
-// whole grid meets at one barrier and must be resident.
+// its splits placed and finishes: a launch may hold more workgroups than the
+// device does at once (540 on the 512 places of head_dim 128, alone or queued
+// behind others).  Two launches that run at the same time are another matter:
+// each can hold the places the other's splits need.  With the O projection in
+// the launch the whole grid meets at one barrier and must be resident.
 template <int HD, bool XL>
 static const void* attn_kernel(bool fused) {
   return fused ? reinterpret_cast<const void*>(&k_decode_attn<true, HD, XL>)

@@ -10,7 +10,10 @@ one workspace must therefore not overlap.  Workspaces here are keyed by
 workspaces, and calls on one stream are ordered by it.
 A HIP graph keeps the workspace of the stream it was captured on; replay it
 in that stream's order relative to eager calls made on the capture stream.
-(The attention workspace belongs to its KV cache, ``gqa_workspace``.)
+(The attention workspace belongs to its KV cache, ``gqa_workspace``, and the
+caller keeps it as long as a graph that captured it: in memory that was freed
+and written to since, the arrival counters no longer start at zero, and every
+wait of the cross-XCD form runs out on every replay.)
 Per-call scratch that a kernel rewrites on every call may sit in the pool too;
 it carries no timeout word and is never zeroed here.
 

@@ -285,6 +285,47 @@ def test_attention_xcd_form_equals_grid_form(dev, monkeypatch, batch, window, he
         assert_bf16_close(np_f(outs[0][b, :, 0]), ref, atol_frac=ATTN_ATOL, what=f"row {b}")
 
 
+@pytest.mark.parametrize("batch,max_len", [(3, 5632), (9, 4224)])
+def test_attention_grid_form_past_the_resident_workgroups(dev, monkeypatch, batch, max_len):
+    """The cross-XCD form of more workgroups than the device holds at once (3 and
+    9 rows of 4 KV heads at head_dim 128: 516 and 540 on 512 places): three
+    states' graphs replayed in turn, with no synchronisation between the replays
+    of a round, give the XCD-local form's bits, no wait runs out and the arrival
+    counters end at zero."""
+    nq, nkv, d, rot = HEADS[1]
+    w = torch.ones(d, device=dev)
+    cos, sin = (torch.from_numpy(t).to(dev) for t in od.rope_tables(max_len, rot, 1e4))
+    kw = dict(num_heads=nq, num_kv_heads=nkv, head_dim=d, rotary_dim=rot, eps=1e-6, scale=d ** -0.5, window=None)
+    states = []
+    for s in range(3):
+        g = torch.Generator().manual_seed(10 * batch + s)
+        seqlen = torch.randint(0, max_len, (batch,), generator=g).to(dev)
+        seqlen[0] = max_len - 1
+        kv = [synthetic.randn_bf16((batch, nkv, max_len, d), 50 + 2 * s + i, dev) for i in range(2)]
+        qkv = synthetic.randn_bf16((batch, (nq + 2 * nkv) * d), 60 + s, dev)
+        ws = gqa_workspace(batch, nkv, max_len, dev, d)
+        monkeypatch.delenv("MAPLE_AMD_ATTN", raising=False)
+        want = decode_attention(qkv, w, w, cos, sin, *kv, seqlen, ws, **kw)
+        monkeypatch.setenv("MAPLE_AMD_ATTN", "grid")
+        assert attention_form(batch, nkv, d, max_len) == "grid"
+        assert torch.equal(decode_attention(qkv, w, w, cos, sin, *kv, seqlen, ws, **kw), want)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = decode_attention(qkv, w, w, cos, sin, *kv, seqlen, ws, **kw)
+        # everything a replay reads or writes lives as long as its graph
+        states.append((graph, out, want, ws, qkv, kv, seqlen))
+    for _ in range(4):
+        for graph, out, *_ in states:
+            out.zero_()
+            graph.replay()
+        torch.cuda.synchronize()
+        for _, out, want, ws, *_ in states:
+            assert torch.equal(out, want)
+            sync = ws[:256 * (1 + 2 * batch * nkv)].view(torch.int32)
+            assert int(sync[2]) == 0, "a wait ran out"
+            assert int(sync[64::128][:batch * nkv].count_nonzero()) == 0, "arrival counters not reset"
+
+
 def test_attention_rejects_bad_shapes(dev):
     q = torch.zeros(2, 32, 1, 96, device=dev, dtype=torch.bfloat16)
     kc = torch.zeros(2, 4, 64, 96, device=dev, dtype=torch.bfloat16)
