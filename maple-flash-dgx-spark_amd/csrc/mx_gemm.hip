@@ -251,8 +251,13 @@ __global__ __launch_bounds__(mx::kThreads) __attribute__((amdgpu_waves_per_eu(2,
   for (int mb = 0; mb < 4; ++mb)
 #pragma unroll
     for (int nb = 0; nb < T::kNb; ++nb) acc[mb][nb] = mx_f32x4_t{0.f, 0.f, 0.f, 0.f};
+  // step 0's copies before step 1's: the counted wait for them goes by issue
+  // order, and nothing else ties copies into distinct arrays together
+  MA_ISSUE_FENCE();
   t.copy(0, b0);
+  MA_ISSUE_FENCE();
   if constexpr (NBUF == 3) t.copy(1, b1);  // nsteps is even
+  MA_ISSUE_FENCE();
   // The loop's copies are unconditional: past a branch around them the compiler
   // counts on fewer being in flight, and waits for all of them.
   int64_t k = 0;
