@@ -525,6 +525,8 @@ extern "C" int ma_rtn4_gemv_mx(const void* x, int x_dtype, int64_t batch, int64_
                                int64_t n_out, int64_t nwords, int packed_kn, const void* scales, int scales_dtype,
                                const void* biases, int biases_dtype, int64_t group_size, void* y, int64_t ldy,
                                void* workspace, size_t workspace_bytes, void* stream) {
+  if (batch > 0 && n_out > 0 && (!x || !packed || !scales || !biases || !y))
+    return fail(MA_EVALUE, "rtn4_gemv_mx: null pointer");
   const size_t need = ma_rtn4_gemv_mx_workspace_bytes(batch, nwords, group_size);
   if (need && n_out > 0 && x_dtype == MA_BF16 && !packed_kn && scales_dtype == biases_dtype &&
       (scales_dtype == MA_BF16 || scales_dtype == MA_F32) && ldx % 8 == 0 && ldx >= nwords * 8 && ldy >= n_out &&

@@ -71,6 +71,18 @@ def test_size_errors_map_without_a_gpu():
                   fake, fake, None, 0, None, 0, fake, fake, 1 << 62, None)
 
 
+def test_rtn4_gemv_mx_rejects_null_pointers_without_a_gpu():
+    """A null x, codes, scales, biases or y is refused on the host: null passes the
+    alignment checks, and the launch would have read it."""
+    fake, bf16 = 0x10000, _lib.BF16
+    nbytes = _lib.load().ma_rtn4_gemv_mx_workspace_bytes(8, 256, 128)
+    for null in range(5):
+        x, w, sc, bs, y = (None if i == null else fake for i in range(5))
+        with pytest.raises(ValueError, match="null pointer"):
+            _lib.call("ma_rtn4_gemv_mx", x, bf16, 8, 2048, w, 128, 256, 0, sc, bf16, bs, bf16, 128, y, 128, fake,
+                      nbytes, None)
+
+
 def test_stamped_variant_exports_the_same_symbols_and_its_stamps_fit():
     """libmaple_amd_stamps.so (the one-launch layer with phase stamps) exports
     everything the header declares; only it reports a stamp layout, and the
