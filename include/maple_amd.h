@@ -262,10 +262,12 @@ int ma_rtn4_gemv_ws(const void* x, int x_dtype, int64_t batch, int64_t ldx,
  * of 64 or 128 with nwords a multiple of 32 (bf16 x, [N, K/8] codes, bf16 or
  * float32 scales and biases of one dtype; x, codes, scales and biases 16-byte
  * aligned): x is written once into the workspace as FP8 pieces that hold it
- * whole, and the codes multiply it as FP8.  Any other call is ma_rtn4_gemv's.
- * Same values as ma_rtn4_gemv up to float32 summation order.  workspace:
+ * whole, and the codes multiply it as FP8.  Any other call is
+ * ma_rtn4_gemv_ws's where the workspace has that call's bytes, else
+ * ma_rtn4_gemv's (workspace may then be NULL).  Same values as ma_rtn4_gemv up
+ * to float32 summation order.  workspace:
  * ma_rtn4_gemv_mx_workspace_bytes(batch, nwords, group_size) bytes (0: none
- * needed), 256-byte aligned; calls sharing one must not overlap.  Replaces
+ * used), 256-byte aligned; calls sharing one must not overlap.  Replaces
  * rtn4_gemv, src/maple_run/kernels/rtn4.py:285-415.
  */
 size_t ma_rtn4_gemv_mx_workspace_bytes(int64_t batch, int64_t nwords, int64_t group_size);

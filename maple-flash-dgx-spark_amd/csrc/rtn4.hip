@@ -516,9 +516,14 @@ extern "C" int ma_rtn4_gemv_ws(const void* x, int x_dtype, int64_t batch, int64_
                       biases_dtype, group_size, y, ldy, stream);
 }
 
+// Shapes of the scaled 8-bit form.
+static bool rtn4_mx_shape(int64_t batch, int64_t nwords, int64_t group_size) {
+  return batch >= 5 && (group_size == 64 || group_size == 128) && nwords >= 32 && nwords % 32 == 0;
+}
+
 extern "C" size_t ma_rtn4_gemv_mx_workspace_bytes(int64_t batch, int64_t nwords, int64_t group_size) {
-  if (batch < 5 || (group_size != 64 && group_size != 128) || nwords < 32 || nwords % 32) return 0;
-  return rtn4_mx_bytes(batch, nwords, group_size);
+  if (rtn4_mx_shape(batch, nwords, group_size)) return rtn4_mx_bytes(batch, nwords, group_size);
+  return ma_rtn4_gemv_workspace_bytes(batch, nwords, group_size);
 }
 
 extern "C" int ma_rtn4_gemv_mx(const void* x, int x_dtype, int64_t batch, int64_t ldx, const uint32_t* packed,
@@ -527,18 +532,27 @@ extern "C" int ma_rtn4_gemv_mx(const void* x, int x_dtype, int64_t batch, int64_
                                void* workspace, size_t workspace_bytes, void* stream) {
   if (batch > 0 && n_out > 0 && (!x || !packed || !scales || !biases || !y))
     return fail(MA_EVALUE, "rtn4_gemv_mx: null pointer");
-  const size_t need = ma_rtn4_gemv_mx_workspace_bytes(batch, nwords, group_size);
-  if (need && n_out > 0 && x_dtype == MA_BF16 && !packed_kn && scales_dtype == biases_dtype &&
-      (scales_dtype == MA_BF16 || scales_dtype == MA_F32) && ldx % 8 == 0 && ldx >= nwords * 8 && ldy >= n_out &&
+  const bool aligned = workspace && (reinterpret_cast<uintptr_t>(workspace) & 255u) == 0;
+  if (rtn4_mx_shape(batch, nwords, group_size) && n_out > 0 && x_dtype == MA_BF16 && !packed_kn &&
+      scales_dtype == biases_dtype && (scales_dtype == MA_BF16 || scales_dtype == MA_F32) && ldx % 8 == 0 &&
+      ldx >= nwords * 8 && ldy >= n_out &&
       ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(packed) | reinterpret_cast<uintptr_t>(scales) |
         reinterpret_cast<uintptr_t>(biases)) & 15u) == 0 &&
       (reinterpret_cast<uintptr_t>(y) & 3u) == 0) {
-    if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255u) || workspace_bytes < need)
+    const size_t need = rtn4_mx_bytes(batch, nwords, group_size);
+    if (!aligned || workspace_bytes < need)
       return fail(MA_EVALUE, "rtn4_gemv_mx: workspace missing, misaligned or under %zu bytes", need);
     return launch_rtn4_mx(static_cast<const uint16_t*>(x), batch, ldx, packed, n_out, nwords, group_size, scales,
                           biases, scales_dtype, static_cast<uint16_t*>(y), ldy, workspace,
                           static_cast<hipStream_t>(stream));
   }
+  // The other calls: x' built once where the workspace holds it (groups of 128;
+  // K = 1152 x 151,936 rows, us: 38.9 and 103.6 in one launch for 32 and 128
+  // tokens, 29.4 and 87.0 so), the same bits in one launch otherwise.
+  const size_t ws = ma_rtn4_gemv_workspace_bytes(batch, nwords, group_size);
+  if (ws && aligned && workspace_bytes >= ws)
+    return ma_rtn4_gemv_ws(x, x_dtype, batch, ldx, packed, n_out, nwords, packed_kn, scales, scales_dtype, biases,
+                           biases_dtype, group_size, y, ldy, workspace, workspace_bytes, stream);
   return ma_rtn4_gemv(x, x_dtype, batch, ldx, packed, n_out, nwords, packed_kn, scales, scales_dtype, biases,
                       biases_dtype, group_size, y, ldy, stream);
 }

@@ -104,8 +104,8 @@ def rtn4_gemv(
         _lib.ptr(sc), _lib.dtype_code(sc, "scales"), _lib.ptr(bs), _lib.dtype_code(bs, "biases"),
         int(group_size), _lib.ptr(y), n_out,
     )
-    # Batched calls write x once into a workspace, as the scaled 8-bit form reads it; calls that it does not take
-    # need none.
+    # Batched calls write x once into a workspace, as the scaled 8-bit form reads it, or the bf16 GEMM in groups of
+    # 128 where K is not a multiple of 256; the query says 0 where no workspace is used.
     nbytes = 0 if packed_kn else int(_lib.load().ma_rtn4_gemv_mx_workspace_bytes(batch, nwords, int(group_size)))
     if nbytes:
         ws = torch.empty(nbytes, device=x.device, dtype=torch.uint8)

@@ -83,6 +83,20 @@ def test_rtn4_gemv_mx_rejects_null_pointers_without_a_gpu():
                       nbytes, None)
 
 
+@pytest.mark.parametrize("batch", [5, 16, 17, 256])
+def test_rtn4_gemv_mx_workspace_covers_the_calls_it_passes_on(batch):
+    """The query's bytes hold the scaled form's rows and, for every K in groups of
+    128, those of ma_rtn4_gemv_ws too, which takes K a multiple of 128 but not of
+    256; no other shape uses a workspace."""
+    lib = _lib.load()
+    for nwords in range(16, 1025, 16):
+        ws, mx = (int(f(batch, nwords, 128)) for f in (lib.ma_rtn4_gemv_workspace_bytes,
+                                                       lib.ma_rtn4_gemv_mx_workspace_bytes))
+        assert mx >= ws > 0 and (nwords % 32 == 0 or mx == ws)
+    assert lib.ma_rtn4_gemv_mx_workspace_bytes(batch, 80, 64) == 0
+    assert lib.ma_rtn4_gemv_mx_workspace_bytes(4, 256, 128) == 0
+
+
 def test_stamped_variant_exports_the_same_symbols_and_its_stamps_fit():
     """libmaple_amd_stamps.so (the one-launch layer with phase stamps) exports
     everything the header declares; only it reports a stamp layout, and the

@@ -469,6 +469,34 @@ def test_rtn4_mx_vs_oracle(dev, batch, n_out, k_in, group, dtype):
     assert torch.equal(z[keep], y[keep]) and bool(z[batch // 2].isnan().all())
 
 
+@pytest.mark.parametrize("batch,n_out,k_in,group,dtype", [
+    (5, 130, 640, 64, torch.bfloat16), (33, 1000, 1152, 64, torch.float32),     # one launch
+    (16, 1056, 1152, 128, torch.bfloat16), (40, 96, 640, 128, torch.float32),   # x' built once: rows of whole 32s
+    (7, 1000, 640, 128, torch.bfloat16)])                                       # one launch: ragged rows
+def test_rtn4_k_not_a_multiple_of_256_vs_oracle(dev, batch, n_out, k_in, group, dtype):
+    """K a multiple of 128 but not of 256, which the scaled 8-bit form does not
+    take: the bf16 GEMM, in groups of 128 with x' built once into the workspace
+    (written then), against the oracle; the same bits as ma_rtn4_gemv."""
+    from maple_amd import _lib
+    w, sc, bs = synthetic.rtn4_table(n_out, k_in, group, 103 + batch, dev)
+    sc, bs = sc.to(dtype), bs.to(dtype)
+    x = synthetic.randn_bf16((batch, k_in), 104, dev)
+    y = rtn4_gemv(x, w, sc, bs, group_size=group)
+    ref = ok.rtn4_gemv(np_f(x), np_u32(w), np_f(sc), np_f(bs), group_size=group)
+    assert_bf16_close(np_f(y), ref, what=f"rtn4 B={batch} K={k_in} g={group}")
+    out = torch.empty(batch, n_out, device=dev, dtype=torch.bfloat16)
+    args = (_lib.ptr(x), _lib.BF16, batch, k_in, _lib.ptr(w), n_out, k_in // 8, 0, _lib.ptr(sc),
+            _lib.dtype_code(sc, "s"), _lib.ptr(bs), _lib.dtype_code(bs, "b"), group, _lib.ptr(out), n_out)
+    _lib.call("ma_rtn4_gemv", *args, _lib.stream_of(x))
+    assert torch.equal(out, y)
+    ws = torch.zeros(max(256, int(_lib.load().ma_rtn4_gemv_mx_workspace_bytes(batch, k_in // 8, group))), device=dev,
+                     dtype=torch.uint8)
+    _lib.call("ma_rtn4_gemv_mx", *args, _lib.ptr(ws), ws.numel(), _lib.stream_of(x))
+    assert torch.equal(out, y) and bool(ws.any()) == (group == 128 and n_out % 32 == 0)
+    _lib.call("ma_rtn4_gemv_mx", *args, None, 0, _lib.stream_of(x))  # no workspace: one launch
+    assert torch.equal(out, y)
+
+
 def test_rtn4_mx_workspace_refused(dev):
     from maple_amd import _lib
     w, sc, bs = synthetic.rtn4_table(128, 256, 64, 99, dev)
