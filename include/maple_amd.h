@@ -262,7 +262,8 @@ int ma_rtn4_gemv_ws(const void* x, int x_dtype, int64_t batch, int64_t ldx,
  * of 64 or 128 with nwords a multiple of 32 (bf16 x, [N, K/8] codes, bf16 or
  * float32 scales and biases of one dtype; x, codes, scales and biases 16-byte
  * aligned): x is written once into the workspace as FP8 pieces that hold it
- * whole, and the codes multiply it as FP8.  Any other call is
+ * whole, and the codes multiply it as FP8.  Short rows and a few tokens, where
+ * one launch is the faster, are ma_rtn4_gemv's; any other call is
  * ma_rtn4_gemv_ws's where the workspace has that call's bytes, else
  * ma_rtn4_gemv's (workspace may then be NULL).  Same values as ma_rtn4_gemv up
  * to float32 summation order.  workspace:

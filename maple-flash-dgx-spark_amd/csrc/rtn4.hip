@@ -521,6 +521,29 @@ static bool rtn4_mx_shape(int64_t batch, int64_t nwords, int64_t group_size) {
   return batch >= 5 && (group_size == 64 || group_size == 128) && nwords >= 32 && nwords % 32 == 0;
 }
 
+// Where the one-launch GEMM is the faster one all the same: the scaled form is
+// two launches, about 4 us more, and makes that up by its products.  One launch
+// against two, us:
+//  * K = 256, up to 3 x 2^20 outputs: 7.2 / 9.2 at 16 tokens x 32,000 rows in
+//    groups of 64, 10.1 / 10.9 at 64, 11.9 / 12.5 at 96, 15.6 / 13.3 at 128.
+//  * Up to 16 tokens, groups of 64, K = 512, up to 2^15 rows: 9.9 / 10.3 at 16 x
+//    32,000; 20.3 / 16.7 at 16 x 100,003, 11.6 / 11.1 at K = 768.
+//  * Up to 16 tokens, groups of 128, up to K = 768: 16.3 / 18.2 at 16 x 151,936,
+//    K = 512; 16.6 / 19.6 at 16 x 104,448, K = 768; 15.9 / 14.9 at 16 x 50,000,
+//    K = 1024.
+//  * Groups of 128 where the scaled form's tiles of 128 rows start another round
+//    of the chip (three a CU) that stays nearly empty, up to 8 tokens (16 to K =
+//    1024): 33.2 / 35.5 at 5 x 100,003, 36.0 / 36.0 at 8 x 131,072, 35.7 / 35.6 at
+//    12 x 100,003, 45.6 / 50.2 at 5 x 100,003, K = 3072 (58.0 / 51.1 at 131,072).
+static bool rtn4_one_launch(int64_t batch, int64_t n_out, int64_t k, int64_t group_size) {
+  if (k <= 256) return batch * n_out <= int64_t{3} << 20;
+  if (batch > 16) return false;
+  if (group_size == 64) return k <= 512 && n_out <= 32768;
+  if (k <= 768) return true;
+  const int64_t tiles = cdiv(n_out, 128);
+  return batch <= (k <= 1024 ? 16 : 8) && tiles > 3 * 256 && tiles <= 4 * 256 && k * tiles <= 2700000;
+}
+
 extern "C" size_t ma_rtn4_gemv_mx_workspace_bytes(int64_t batch, int64_t nwords, int64_t group_size) {
   if (rtn4_mx_shape(batch, nwords, group_size)) return rtn4_mx_bytes(batch, nwords, group_size);
   return ma_rtn4_gemv_workspace_bytes(batch, nwords, group_size);
@@ -542,6 +565,9 @@ extern "C" int ma_rtn4_gemv_mx(const void* x, int x_dtype, int64_t batch, int64_
     const size_t need = rtn4_mx_bytes(batch, nwords, group_size);
     if (!aligned || workspace_bytes < need)
       return fail(MA_EVALUE, "rtn4_gemv_mx: workspace missing, misaligned or under %zu bytes", need);
+    if (rtn4_one_launch(batch, n_out, nwords * 8, group_size) && (reinterpret_cast<uintptr_t>(y) & 15u) == 0)
+      return ma_rtn4_gemv(x, x_dtype, batch, ldx, packed, n_out, nwords, packed_kn, scales, scales_dtype, biases,
+                          biases_dtype, group_size, y, ldy, stream);
     return launch_rtn4_mx(static_cast<const uint16_t*>(x), batch, ldx, packed, n_out, nwords, group_size, scales,
                           biases, scales_dtype, static_cast<uint16_t*>(y), ldy, workspace,
                           static_cast<hipStream_t>(stream));

@@ -497,6 +497,35 @@ def test_rtn4_k_not_a_multiple_of_256_vs_oracle(dev, batch, n_out, k_in, group, 
     assert torch.equal(out, y)
 
 
+@pytest.mark.parametrize("batch,n_out,k_in,group,one", [
+    (96, 32768, 256, 64, True), (97, 32768, 256, 64, False), (5, 129, 256, 128, True),
+    (16, 1000, 512, 64, True), (17, 1000, 512, 64, False), (5, 32769, 512, 64, False), (16, 1000, 768, 64, False),
+    (16, 1000, 768, 128, True), (17, 1000, 768, 128, False), (5, 1000, 1024, 128, False),
+    (16, 98432, 1024, 128, True), (5, 98304, 1024, 128, False), (8, 98305, 2048, 128, True),
+    (9, 98305, 2048, 128, False)])
+def test_rtn4_one_launch_rule(dev, batch, n_out, k_in, group, one):
+    """Which calls of the scaled form's shapes take the one-launch GEMM: those give
+    its bits and leave the workspace alone, the others write it; both agree
+    within the scaled form's tolerance."""
+    from maple_amd import _lib
+    w, sc, bs = synthetic.rtn4_table(n_out, k_in, group, 105, dev)
+    x = synthetic.randn_bf16((batch, k_in), 106, dev)
+    y, out = (torch.empty(batch, n_out, device=dev, dtype=torch.bfloat16) for _ in range(2))
+    ws = torch.zeros(int(_lib.load().ma_rtn4_gemv_mx_workspace_bytes(batch, k_in // 8, group)), device=dev,
+                     dtype=torch.uint8)
+    args = lambda o: (_lib.ptr(x), _lib.BF16, batch, k_in, _lib.ptr(w), n_out, k_in // 8, 0,  # noqa: E731
+                      _lib.ptr(sc), _lib.BF16, _lib.ptr(bs), _lib.BF16, group, _lib.ptr(o), n_out)
+    _lib.call("ma_rtn4_gemv_mx", *args(y), _lib.ptr(ws), ws.numel(), _lib.stream_of(x))
+    _lib.call("ma_rtn4_gemv", *args(out), _lib.stream_of(x))
+    assert bool(ws.any()) != one
+    if one:
+        assert torch.equal(y, out)
+    # both are rounded to bf16: a sum next to the middle of two numbers may go to
+    # either, one ulp, 2^-7 of a value just above a power of two (each is within
+    # the default 2^-8 of the oracle)
+    assert_bf16_close(np_f(y), np_f(out), rtol=2.0 ** -7, what=f"rtn4 B={batch} K={k_in} g={group}")
+
+
 def test_rtn4_mx_workspace_refused(dev):
     from maple_amd import _lib
     w, sc, bs = synthetic.rtn4_table(128, 256, 64, 99, dev)
