@@ -706,50 +706,44 @@ int launch_rtn4_mx(const uint16_t* x, int64_t batch, int64_t ldx, const uint32_t
                        x3, batch, rows, w, n_out, nwords, scales, biases, y, ldy, static_cast<int>(tt),              \
                        static_cast<int>(tiles));                                                                     \
   } while (0)
-// Tile by batch: 32 or 64 tokens x 128 rows while the table's bytes are the
-// bound (151,936 rows, groups of 64: 57 us at 24 tokens, 75 at 64); past 64 the
-// ring's 128 x 256 (at 128 tokens in groups of 128 114 us, 118 in a tile of 128
-// x 128, 127 with the ring's size and two buffers).  The ring needs the bias
-// half's product, whole steps of 16 bf16 groups; without it 128 x 128 rows up to
-// one such token tile, x 256 above (203 against 217 at 256: half the x rows'
-// traffic).
-#define MA_MH_S(GW, SDT, BM)              \
-  if (batch <= 32)                        \
+// Tile by the number of tiles, so that a table of any height fills the chip.
+// 32 tokens x 128 rows while that is one token tile or at most 512 tiles, two a
+// CU (a wave's chain through K is the shorter one: 8,192 rows at 128 tokens, us,
+// groups of 128: 17 against 22 with 64 tokens and 34 in the ring; 16,384 at 64
+// 16 / 21; past it 50,000 at 64 35 / 26).  Above, 64 tokens x 128 rows, and from
+// 768 of those the ring's 128 x 256 (one workgroup a CU), unless that pads the
+// tokens by more than an eighth (groups of 128 (64): 32,000 rows at 128 27 (29)
+// against 35 (38), at 192 37 (40) / 38 (42), at 256 49 (52) / 39 (42); 151,936
+// at 128 99 (108) / 98 (106), at 192 136 (148) / 160 (173), at 256 179 (198) /
+// 161 (175)).  The ring needs the bias half's product, whole steps of 16 bf16
+// groups; float32 scales and other K keep to the small tiles (one of 128 x 128
+// took 106 us for 94 at 100,003 rows, 128 tokens, groups of 64).
+  const int64_t rtiles = cdiv(n_out, 128);
+  const int64_t t32 = cdiv(batch, 32) * rtiles, t64 = cdiv(batch, 64) * rtiles;
+  const int64_t tring = cdiv(batch, 128) * cdiv(n_out, 256);
+  const bool bias_mm = s_dt == MA_BF16 && nwords / gw % 16 == 0;
+#define MA_MH_T(GW, SDT, BM)              \
+  if (batch <= 32 || t32 <= 2 * 256)      \
     MA_MH(1, 1, 1, 4, 4, GW, SDT, BM, 3); \
   else                                    \
     MA_MH(2, 1, 1, 4, 2, GW, SDT, BM, 3);
-#define MA_MH_T(GW, SDT)                     \
-  if (batch <= 64) {                         \
-    MA_MH_S(GW, SDT, false)                  \
-  } else if (batch <= 128)                   \
-    MA_MH(2, 2, 2, 2, 2, GW, SDT, false, 2); \
-  else                                       \
-    MA_MH(2, 2, 2, 4, 2, GW, SDT, false, 2);
-#define MA_MR(G64)                                                                                                     \
-  const int64_t tt = cdiv(batch, 128), tiles = tt * cdiv(n_out, 256);                                                \
-  auto* const kernel = (G64) ? &k_mx_head_ring<8> : &k_mx_head_ring<16>;                                             \
-  hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(cdiv(tiles, kXcds) * kXcds)), dim3(512), 0, s, xq, xs, x3,    \
-                     batch, rows, w, n_out, nwords, static_cast<const uint16_t*>(scales),                            \
-                     static_cast<const uint16_t*>(biases), y, ldy, static_cast<int>(tt), static_cast<int>(tiles));
-#define MA_MH_G(SDT) \
-  if (group == 64) { MA_MH_T(8, SDT) } else { MA_MH_T(16, SDT) }
-  if (s_dt == MA_F32) {
-    MA_MH_G(MA_F32)
-  } else if (nwords / gw % 16 == 0) {
-    if (batch > 64) {
-      MA_MR(group == 64)
-    } else if (group == 64) {
-      MA_MH_S(8, MA_BF16, true)
-    } else {
-      MA_MH_S(16, MA_BF16, true)
-    }
+#define MA_MH_G(SDT, BM) \
+  if (group == 64) { MA_MH_T(8, SDT, BM) } else { MA_MH_T(16, SDT, BM) }
+  if (bias_mm && t64 > 3 * 256 && 32 * tring <= 9 * t64) {
+    const int64_t tt = cdiv(batch, 128);
+    auto* const kernel = group == 64 ? &k_mx_head_ring<8> : &k_mx_head_ring<16>;
+    hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(cdiv(tring, kXcds) * kXcds)), dim3(512), 0, s, xq, xs, x3,
+                       batch, rows, w, n_out, nwords, static_cast<const uint16_t*>(scales),
+                       static_cast<const uint16_t*>(biases), y, ldy, static_cast<int>(tt), static_cast<int>(tring));
+  } else if (s_dt == MA_F32) {
+    MA_MH_G(MA_F32, false)
+  } else if (bias_mm) {
+    MA_MH_G(MA_BF16, true)
   } else {
-    MA_MH_G(MA_BF16)
+    MA_MH_G(MA_BF16, false)
   }
 #undef MA_MH_G
-#undef MA_MR
 #undef MA_MH_T
-#undef MA_MH_S
 #undef MA_MH
   return check_launch("rtn4_gemv (mx)");
 }

@@ -441,11 +441,11 @@ def test_rtn4_mfma_batched_vs_oracle(dev, batch, group, n_out):
 
 
 @pytest.mark.parametrize("batch,n_out,k_in,group,dtype", [
-    (5, 1003, 256, 64, torch.bfloat16),     # 4 groups: biases by FMA; odd row count
+    (5, 1003, 256, 64, torch.bfloat16),     # short rows: the one-launch GEMM; odd row count
     (32, 129, 1024, 64, torch.bfloat16),    # 16 groups: biases by the matrix units
-    (33, 515, 2048, 128, torch.bfloat16),   # 64-token tiles, 16 groups
+    (33, 515, 2048, 128, torch.bfloat16),   # two 32-token tiles, 16 groups
     (64, 256, 768, 128, torch.float32),
-    (65, 1000, 2048, 64, torch.bfloat16),   # 128 x 128 tiles
+    (65, 1000, 2048, 64, torch.bfloat16),   # 32-token tiles: few of them
     (129, 1029, 1280, 128, torch.bfloat16),
     (256, 384, 512, 64, torch.float32),
 ])
@@ -495,6 +495,33 @@ def test_rtn4_k_not_a_multiple_of_256_vs_oracle(dev, batch, n_out, k_in, group, 
     assert torch.equal(out, y) and bool(ws.any()) == (group == 128 and n_out % 32 == 0)
     _lib.call("ma_rtn4_gemv_mx", *args, None, 0, _lib.stream_of(x))  # no workspace: one launch
     assert torch.equal(out, y)
+
+
+@pytest.mark.parametrize("batch,n_out,k_in,group,dtype", [
+    (1000, 6401, 1024, 64, torch.bfloat16),     # ring, 8 stages: 2 in its tail; several token tiles, ragged both ways
+    (512, 12545, 2048, 128, torch.bfloat16),    # 16 stages: 4
+    (1025, 6400, 3072, 64, torch.bfloat16),     # 24 stages: 3
+    (2000, 3201, 4096, 128, torch.bfloat16),    # 32 stages: 2, a scale for two stages
+    (1999, 3300, 6144, 128, torch.bfloat16),    # 48 stages: 3
+    (129, 33000, 1024, 64, torch.bfloat16),     # 64-token tiles: the ring's 128 would pad more than an eighth
+    (130, 25000, 1024, 128, torch.bfloat16),    # 64-token tiles, biases by FMA
+    (65, 32897, 512, 64, torch.float32),        # 64-token tiles from 513 of 32
+    (64, 32768, 512, 128, torch.bfloat16)])     # 32-token tiles, 512 of them
+def test_rtn4_mx_wide_tiles_vs_oracle(dev, batch, n_out, k_in, group, dtype):
+    """The tiles that tables and batches of some size take: the ring of 128 x 256
+    at each length of its tail, 64-token tiles and 32-token tiles at their ends;
+    the oracle's values, and the same bits on a second run."""
+    w, sc, bs = synthetic.rtn4_table(n_out, k_in, group, 107 + batch, dev)
+    sc, bs = sc.to(dtype), bs.to(dtype)
+    x = synthetic.randn_bf16((batch, k_in + 8), 108, dev)[:, :k_in]
+    y = rtn4_gemv(x, w, sc, bs, group_size=group)
+    assert torch.equal(rtn4_gemv(x, w, sc, bs, group_size=group), y)
+    # the oracle on rows of every tile: all of the first and last 300, and each 17th
+    rows = torch.unique(torch.cat([torch.arange(300), torch.arange(n_out - 300, n_out),
+                                   torch.arange(0, n_out, 17)])).to(dev)
+    pick = lambda t: t.view(torch.int32)[rows].view(torch.uint32) if t.dtype == torch.uint32 else t[rows]  # noqa: E731
+    ref = ok.rtn4_gemv(np_f(x), np_u32(pick(w)), np_f(pick(sc)), np_f(pick(bs)), group_size=group)
+    assert_bf16_close(np_f(y[:, rows]), ref, what=f"rtn4 B={batch} N={n_out} K={k_in} g={group}")
 
 
 @pytest.mark.parametrize("batch,n_out,k_in,group,one", [
