@@ -574,9 +574,10 @@ extern "C" int ma_rtn4_gemv_mx(const void* x, int x_dtype, int64_t batch, int64_
   }
   // The other calls: x' built once where the workspace holds it (groups of 128;
   // K = 1152 x 151,936 rows, us: 38.9 and 103.6 in one launch for 32 and 128
-  // tokens, 29.4 and 87.0 so), the same bits in one launch otherwise.
+  // tokens, 29.4 and 87.0 so; K = 640 at 5 tokens 16.2 in one launch, 17.1 so),
+  // the same bits in one launch otherwise.
   const size_t ws = ma_rtn4_gemv_workspace_bytes(batch, nwords, group_size);
-  if (ws && aligned && workspace_bytes >= ws)
+  if (ws && aligned && workspace_bytes >= ws && !rtn4_one_launch(batch, n_out, nwords * 8, group_size))
     return ma_rtn4_gemv_ws(x, x_dtype, batch, ldx, packed, n_out, nwords, packed_kn, scales, scales_dtype, biases,
                            biases_dtype, group_size, y, ldy, workspace, workspace_bytes, stream);
   return ma_rtn4_gemv(x, x_dtype, batch, ldx, packed, n_out, nwords, packed_kn, scales, scales_dtype, biases,
