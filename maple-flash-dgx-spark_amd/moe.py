@@ -38,11 +38,6 @@ from .kernels.ternary_expert import ternary_expert_down_sum, ternary_expert_swig
 from .synthetic import MoELayer
 
 GROUPED_MIN_TOKENS = 4
-# The grouped kernels' decode form: up to this many (token, slot) pairs per
-# expert on average; its tiles hold rows of up to GROUPED_TILE_VALUES values, and
-# the kernels for longer rows read x' pairs (grouped.hip).
-GROUPED_DECODE_PAIRS = 16
-GROUPED_TILE_VALUES = 4096
 
 _RESIDENT: dict[tuple, bool] = {}
 
@@ -400,12 +395,8 @@ def moe_layer(hidden: torch.Tensor, layer: MoELayer, top_k: int, norm_weight: to
     tokens = hidden.shape[0]
     if (tokens >= GROUPED_MIN_TOKENS and route_supported(layer, top_k, hidden)
             and hidden.shape[-1] % 256 == 0 and layer.inter % 256 == 0):
-        # (the routing launch takes hidden up to 4096, so the long rows here are h's; with the pairs a layer of
-        # hidden 2048, intermediate 4352, 8 experts takes 37 us at 8 tokens, 47 where every workgroup builds its own)
-        pairs = layer.inter > GROUPED_TILE_VALUES and tokens * top_k <= GROUPED_DECODE_PAIRS * layer.n_experts
-        h, xn, ids, wts, d, *xp = moe_route(hidden, layer, top_k, norm_weight, eps, add=add, pairs=pairs)
-        return moe_grouped(xn, layer, ids, wts, h, dispatch=d, x_pairs=xp[0] if xp else None,
-                           combine=not defer_combine), ids
+        h, xn, ids, wts, d = moe_route(hidden, layer, top_k, norm_weight, eps, add=add)
+        return moe_grouped(xn, layer, ids, wts, h, dispatch=d, combine=not defer_combine), ids
     if add is not None:
         h, xn = add_rms_norm(hidden, add, norm_weight, eps)
     else:

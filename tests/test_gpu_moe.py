@@ -246,30 +246,6 @@ def test_moe_layer_routed_pairs_vs_oracle(dev, layer, tokens):
     assert torch.equal(y, y2)  # deterministic
 
 
-@pytest.mark.parametrize("hidden,inter,n_exp,k,tokens", [(2048, 4352, 4, 2, 5), (512, 4608, 3, 1, 33)])
-def test_moe_layer_long_rows_read_pairs(dev, hidden, inter, n_exp, k, tokens):
-    """Decode batches with an intermediate past 4096: the K-split kernels reading
-    the x' pairs that the routing launch wrote, and those that build them from x
-    (whose correction sums have another order), give the oracle's values; the
-    layer's bits are the first's."""
-    from maple_amd.kernels import add_rms_norm
-    from maple_amd.moe import moe_layer, moe_route
-    L = synthetic.make_moe_layer(hidden, n_exp, inter, seed=23, device=dev)
-    assert tokens * k <= 16 * n_exp  # the decode form
-    x = synthetic.randn_bf16((tokens, hidden), 903, dev)
-    add = synthetic.randn_bf16((tokens, hidden), 904, dev)
-    nw = synthetic.uniform_bf16((hidden,), 0.5, 1.5, 905, dev)
-    y, ids = moe_layer(x, L, k, nw, 1e-6, add=add)
-    h, xn, ids2, wts, d, xp = moe_route(x, L, k, nw, 1e-6, add=add, pairs=True)
-    own = moe_grouped(xn, L, ids, wts, h, dispatch=d)
-    torch.cuda.synchronize()
-    assert torch.equal(ids, ids2) and torch.equal(h, add_rms_norm(x, add, nw, 1e-6)[0])
-    assert torch.equal(moe_grouped(xn, L, ids, wts, h, dispatch=d, x_pairs=xp), y)
-    ref, _ = ok.moe_experts(np_f(xn), ids.cpu().numpy(), wts.cpu().numpy(), *_oracle_inputs(L), residual=np_f(h))
-    for v, what in ((y, "pairs"), (own, "own operands")):
-        assert_bf16_close(np_f(v), ref, atol_frac=2.0 ** -7, what=f"long rows, {what} H={hidden} I={inter}")
-
-
 def test_moe_block_grouped_matches_per_slot(dev, layer):
     """The two plans agree on the same routing (bf16 tolerance)."""
     x = synthetic.randn_bf16((16, H), 400, dev)
