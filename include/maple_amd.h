@@ -121,7 +121,9 @@ int ma_router_topk(const void* x, int x_dtype, int64_t tokens, int64_t ldx,
  * ma_router_topk that also writes x in the form the grouped expert GEMMs
  * read (x_pairs uint32 [tokens, k_in / 2], 16-byte aligned; x_corr float32
  * [tokens]: each token's correction sum), from the same per-token launch as
- * the top-k; ma_moe_grouped given them returns the same bits.  x bfloat16, k_in
+ * the top-k; ma_moe_grouped reads them in decode batches of hidden past 4096
+ * (the same values; the correction sums have another order, so single bf16
+ * roundings may differ).  x bfloat16, k_in
  * a multiple of 16, rows 16-byte aligned.
  * No reference counterpart: a fused form of router_topk and the first step
  * of the grouped experts, for prefill-sized batches.
@@ -326,8 +328,9 @@ int ma_moe_route(const void* x, const void* x_add, int64_t tokens, int64_t hidde
  * workspace: ma_grouped_workspace_bytes(tokens * top_k, inter, hidden).
  * x_pairs / x_corr (optional, both or neither): x as ma_moe_route writes it
  * in x' pair form (uint32 [tokens, hidden / 2]) with each token's correction
- * (float32 [tokens]); read where hidden or inter is past 4096 in a decode batch,
- * and not elsewhere (the same bits; x is still passed).  The per-pair down
+ * (float32 [tokens]); read where hidden is past 4096 in a decode batch (at most
+ * 16 pairs an expert on average), and not elsewhere (x is still passed).  The
+ * per-pair down
  * outputs stay in the workspace at byte offset tokens * top_k * inter * 2
  * rounded up to a multiple of 256 (bf16 [tokens * top_k, hidden]); with
  * y = NULL the combine is skipped

@@ -130,17 +130,21 @@ __device__ __forceinline__ float pairs_cst(const uint32_t pr[8]) {
 // 16-word chunks w, w + KW, ... of K.  PAIRS: the activations arrive as x'
 // pairs with their per-token correction (x_pairs, x_corr: built once per
 // token upstream) and are loaded as B operands directly; otherwise each lane
-// builds its B operands from x.
-template <int MBH, int ADT, int KW, bool PAIRS>
+// builds its B operands from x.  MX: h goes out as mx rows (hp, scale words hs)
+// for the tile-resident down stage, with a correction part per 32 outputs
+// (hcorr); otherwise as x' pairs for the K-split one.
+template <int MBH, int ADT, int KW, bool PAIRS, bool MX>
 __global__ __launch_bounds__(64 * KW) void k_grouped_swiglu_ks(
     const uint16_t* __restrict__ x, int64_t ldx, const uint32_t* __restrict__ x_pairs,
     const float* __restrict__ x_corr, int64_t topk,
     const uint32_t* __restrict__ w, int64_t n_half, int64_t nwords,
     const void* __restrict__ alpha, const int32_t* __restrict__ offsets,
     const int32_t* __restrict__ pair_ids, int n_exp,
-    uint16_t* __restrict__ hp, uint16_t* __restrict__ h, int64_t ldh) {
+    uint16_t* __restrict__ hp, uint32_t* __restrict__ hs, float* __restrict__ hcorr,
+    uint16_t* __restrict__ h, int64_t ldh) {
   constexpr int MB = 2 * MBH;  // row blocks: up 0 .. MBH-1, gate MBH .. MB-1
   static_assert(KW >= MBH, "the epilogue takes 64 threads per up block");
+  static_assert(!MX || MBH == 2, "a workgroup's outputs are one scale block");
   __shared__ float red[KW][MB][4][64];
   __shared__ float red_c[KW][4][16];
   int e, pos0, np;
@@ -224,41 +228,88 @@ __global__ __launch_bounds__(64 * KW) void k_grouped_swiglu_ks(
   if constexpr (!PAIRS) red_c[wv][g][r16] = cp;
   __syncthreads();
   // Thread t < 64 MBH: pair column col = t % 16, rows 4 rq .. +3 of up block mbu.
-  if (tid >= 64 * MBH) return;
   const int col = tid & 15, rq = (tid >> 4) & 3, mbu = tid >> 6;
-  if (col >= np) return;
-  const int pid = pair_ids[pos0 + col];
-  float c = 0.f;
-  if constexpr (PAIRS) {
-    c = x_corr[pid / topk];
-  } else {
-#pragma unroll
-    for (int k = 0; k < KW; ++k)
-#pragma unroll
-      for (int gg = 0; gg < 4; ++gg) c += red_c[k][gg][col];
-  }
-  const int ln = col + 16 * rq;
+  if (tid >= 64 * MBH) return;  // (a later barrier waits for the waves that are left)
+  const bool live = col < np;
+  if (!MX && !live) return;
   const int64_t nwh = n_half / 16;
+  float hv[4] = {0.f, 0.f, 0.f, 0.f}, hsum = 0.f;
+  uint32_t ex = 0;
+  if (live) {
+    const int pid = pair_ids[pos0 + col];
+    float c = 0.f;
+    if constexpr (PAIRS) {
+      c = x_corr[pid / topk];
+    } else {
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int64_t i = i0 + 16 * mbu + 4 * rq + r;
-    if (i >= n_half) continue;
-    float su = 0.f, sg = 0.f;
+      for (int k = 0; k < KW; ++k)
 #pragma unroll
-    for (int k = 0; k < KW; ++k) {
-      su += red[k][mbu][r][ln];
-      sg += red[k][mbu + MBH][r][ln];
+        for (int gg = 0; gg < 4; ++gg) c += red_c[k][gg][col];
     }
-    const float au = ld_t<ADT>(alpha, static_cast<int64_t>(e) * 2 * n_half + i);
-    const float ag = ld_t<ADT>(alpha, static_cast<int64_t>(e) * 2 * n_half + n_half + i);
-    const uint16_t hb = f32_to_bf16(swiglu_act(au * (su - c), ag * (sg - c)));
-    if (hp) {
-      const int pos = static_cast<int>(i & 15), j = pos & 7, hh = pos >> 3;
-      const float hv = bf16_to_f32(hb) * pair_scale(j);  // exact: power-of-two scale
-      hp[((static_cast<int64_t>(pos0 + col) * nwh + (i >> 4)) * 8 + j) * 2 + hh] =
-          static_cast<uint16_t>(bf16_bits_exact(hv));
+    const int ln = col + 16 * rq;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int64_t i = i0 + 16 * mbu + 4 * rq + r;
+      if (i >= n_half) continue;
+      float su = 0.f, sg = 0.f;
+#pragma unroll
+      for (int k = 0; k < KW; ++k) {
+        su += red[k][mbu][r][ln];
+        sg += red[k][mbu + MBH][r][ln];
+      }
+      const float au = ld_t<ADT>(alpha, static_cast<int64_t>(e) * 2 * n_half + i);
+      const float ag = ld_t<ADT>(alpha, static_cast<int64_t>(e) * 2 * n_half + n_half + i);
+      const uint16_t hb = f32_to_bf16(swiglu_act(au * (su - c), ag * (sg - c)));
+      if constexpr (MX) {
+        hv[r] = bf16_to_f32(hb);
+        hsum += hv[r];
+        ex = mx_exponent(ex, hv[r]);
+      } else {
+        const int pos = static_cast<int>(i & 15), j = pos & 7, hh = pos >> 3;
+        const float hx = bf16_to_f32(hb) * pair_scale(j);  // exact: power-of-two scale
+        hp[((static_cast<int64_t>(pos0 + col) * nwh + (i >> 4)) * 8 + j) * 2 + hh] =
+            static_cast<uint16_t>(bf16_bits_exact(hx));
+      }
+      if (h) h[static_cast<int64_t>(pid) * ldh + i] = hb;
     }
-    if (h) h[static_cast<int64_t>(pid) * ldh + i] = hb;
+  }
+  if constexpr (MX) {
+    // the 32 outputs' exponent and sum: over a wave's lane groups, then its two waves
+    __shared__ uint32_t s_ex[MBH][16];
+    __shared__ float s_sum[MBH][16];
+    uint32_t eo = __shfl_xor(ex, 16, 64);
+    ex = ex > eo ? ex : eo;
+    eo = __shfl_xor(ex, 32, 64);
+    ex = ex > eo ? ex : eo;
+    hsum += __shfl_xor(hsum, 16, 64);
+    hsum += __shfl_xor(hsum, 32, 64);
+    if (rq == 0) {
+      s_ex[mbu][col] = ex;
+      s_sum[mbu][col] = hsum;
+    }
+    // s_barrier leaves out waves that have ended (the other six, whose slots the
+    // next workgroup's waves take meanwhile: 59.9 us with them held here, 54.2 now,
+    // for 256 pairs of 64 experts, 5120 -> 768)
+    __syncthreads();
+    if (!live) return;
+    ex = s_ex[0][col] > s_ex[1][col] ? s_ex[0][col] : s_ex[1][col];
+    // word wd of the row: block pos / 2 of its step, word pos of the step's 8 (launch_mx_prep_wide's order)
+    const int64_t wd = i0 / 16 + mbu, row = pos0 + col;
+    const int64_t step = wd / 16 * 2 + (wd >> 1 & 1), nsteps = n_half / kMxStep;
+    const int pos = static_cast<int>((wd >> 2 & 3) * 2 + (wd & 1));
+    const float f = mx_factor(ex);
+    float v[4] = {hv[0] * f, hv[2] * f, hv[1] * f, hv[3] * f};
+    uint16_t* dst = hp + (row * nsteps + step) * kMxStep + 8 * pos + rq;  // even values, then the odd ones
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      const uint32_t w4 = mx_piece4(v);
+      dst[64 * p] = static_cast<uint16_t>(w4);
+      dst[64 * p + 4] = static_cast<uint16_t>(w4 >> 16);
+    }
+    if (mbu == 0 && rq == 0) {
+      reinterpret_cast<uint8_t*>(hs + row * nsteps + step)[pos / 2] = static_cast<uint8_t>(mx_scale_byte(ex));
+      hcorr[row * (n_half / 32) + i0 / 32] = s_sum[0][col] + s_sum[1][col];
+    }
   }
 }
 
@@ -471,8 +522,9 @@ __device__ __forceinline__ void kloop(const uint32_t* const (&rp)[2], int nch, u
 }  // namespace gd
 
 // SwiGLU: 128 outputs (8 up blocks and the matching gate blocks, one of each a
-// wave) of a tile of 16 pairs.
-template <int ADT, int NCH>
+// wave) of a tile of 16 pairs.  PAIRS: h goes out as x' pairs, for the K-split
+// down stage.
+template <int ADT, int NCH, bool PAIRS>
 __global__ __launch_bounds__(gd::kThreads) void k_gd_swiglu(
     const uint16_t* __restrict__ x, int64_t ldx, int64_t topk, const uint32_t* __restrict__ w, int64_t n_half,
     int nch_arg, const void* __restrict__ alpha, const int32_t* __restrict__ offsets,
@@ -584,7 +636,13 @@ __global__ __launch_bounds__(gd::kThreads) void k_gd_swiglu(
     hsum += hv[r];
     ex = mx_exponent(ex, hv[r]);
     if (h && r16 < np) h[static_cast<int64_t>(s_pid[r16]) * ldh + i0 + r] = hb;
+    if (PAIRS && r16 < np) {
+      const int pos = 4 * g + r, j = pos & 7;
+      hp[((static_cast<int64_t>(pos0 + r16) * (n_half / 16) + blk) * 8 + j) * 2 + (pos >> 3)] =
+          static_cast<uint16_t>(bf16_bits_exact(hv[r] * pair_scale(j)));  // exact: power-of-two scale
+    }
   }
+  if constexpr (PAIRS) return;
   uint32_t eo = __shfl_xor(ex, 16, 64);
   ex = ex > eo ? ex : eo;
   eo = __shfl_xor(ex, 32, 64);
@@ -633,8 +691,9 @@ __global__ __launch_bounds__(gd::kThreads) void k_gd_swiglu(
 }
 
 // Down: 256 output rows (two blocks a wave) of a tile of 16 pairs, whose mx rows
-// of h, scale words and correction parts the SwiGLU stage wrote.
-template <int ADT, int NCH>
+// of h, scale words and correction parts (CP to each 128 values) the SwiGLU stage
+// wrote.
+template <int ADT, int NCH, int CP>
 __global__ __launch_bounds__(gd::kThreads) void k_gd_down(const uint32_t* __restrict__ hp,
                                                           const uint32_t* __restrict__ hs,
                                                           const float* __restrict__ hcorr,
@@ -671,7 +730,8 @@ __global__ __launch_bounds__(gd::kThreads) void k_gd_down(const uint32_t* __rest
   const int sc = tid / nsteps, ss = tid % nsteps;  // 16 nsteps <= 512
   if (sc < np) {
     sw = hs[static_cast<int64_t>(pos0 + sc) * nsteps + ss];
-    cp = hcorr[static_cast<int64_t>(pos0 + sc) * nsteps + ss];
+#pragma unroll
+    for (int q = 0; q < CP; ++q) cp += hcorr[(static_cast<int64_t>(pos0 + sc) * nsteps + ss) * CP + q];
   }
   MA_ISSUE_FENCE();
   const uint32_t* we = w + static_cast<int64_t>(e) * n_out * nwk;
@@ -1294,6 +1354,8 @@ static size_t grouped_bytes(int64_t n_pairs, int64_t tokens, int64_t inter, int6
   if (prefill)
     b += align256(static_cast<size_t>(tokens) * hidden * 2) + align256(static_cast<size_t>(tokens) * 8) +
          align256(static_cast<size_t>(tokens) * (hidden / kMxStep) * 4);
+  else if (hidden > 256 * gd::kMaxChunks && inter <= 256 * gd::kMaxChunks)
+    b += align256(3 * static_cast<size_t>(n_pairs) * (inter / kMxStep) * 4);  // four correction parts instead of one
   return b;
 }
 
@@ -1338,45 +1400,57 @@ static int grouped_launch(const void* x, int64_t ldx, const uint32_t* x_pairs, c
   if (!grouped_prefill_form(n_pairs, n_experts)) {
     // decode: 16-pair tiles
     const unsigned max_tiles = static_cast<unsigned>(n_pairs / 16 + n_experts);
-    if (hidden <= 256 * gd::kMaxChunks && inter <= 256 * gd::kMaxChunks) {
-      const int64_t hsteps = inter / kMxStep;
-      const int uch = static_cast<int>(hidden / 256), dch = static_cast<int>(inter / 256);
-      uint32_t* hs = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(out) +
-                                                 align256(static_cast<size_t>(n_pairs) * hidden * 2));
-      float* hcorr = reinterpret_cast<float*>(reinterpret_cast<char*>(hs) +
-                                              align256(static_cast<size_t>(n_pairs) * hsteps * 4));
-      const dim3 g1(static_cast<unsigned>(hsteps), max_tiles), g2(static_cast<unsigned>(hidden / 256), max_tiles);
-#define MA_GD_UP(ADT, NCH)                                                                                           \
-  hipLaunchKernelGGL((k_gd_swiglu<ADT, NCH>), g1, dim3(gd::kThreads), 0, s, xb, ldx, top_k, up_gate, inter, uch,      \
-                     up_gate_alpha, offsets, pair_ids, ne, hp, hs, hcorr, hb, ldh)
-#define MA_GD_DOWN(ADT, NCH)                                                                                         \
-  hipLaunchKernelGGL((k_gd_down<ADT, NCH>), g2, dim3(gd::kThreads), 0, s, reinterpret_cast<const uint32_t*>(hp), hs, \
-                     hcorr, down, hidden, dch, down_alpha, offsets, ne, out)
-#define MA_GD(ADT)                                                                            \
-  if (uch == 8) MA_GD_UP(ADT, 8); else MA_GD_UP(ADT, 0);                                      \
-  if (dch == 2) MA_GD_DOWN(ADT, 2); else if (dch == 3) MA_GD_DOWN(ADT, 3); else MA_GD_DOWN(ADT, 0);
-      if (alpha_dtype == MA_BF16) { MA_GD(MA_BF16) } else { MA_GD(MA_F32) }
-#undef MA_GD
+    // Each stage by its own K: tiles in LDS up to 256 * gd::kMaxChunks values, K
+    // split over the waves past that; h goes between them as the down stage reads
+    // it (mx rows, or x' pairs).  One rule over both stages cost the one that
+    // fits: hidden 2048, intermediate 4352, 8 experts, 8 tokens x 8 44.9 us a block for 32.8,
+    // hidden 5120, intermediate 768, 64 experts, 8 tokens x 8 70.3 for 55.9.
+    const bool up_tile = hidden <= 256 * gd::kMaxChunks, down_tile = inter <= 256 * gd::kMaxChunks;
+    const int64_t hsteps = inter / kMxStep;
+    const int uch = static_cast<int>(hidden / 256), dch = static_cast<int>(inter / 256);
+    uint32_t* hs = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(out) +
+                                               align256(static_cast<size_t>(n_pairs) * hidden * 2));
+    float* hcorr = reinterpret_cast<float*>(reinterpret_cast<char*>(hs) +
+                                            align256(static_cast<size_t>(n_pairs) * hsteps * 4));
+#define MA_GD_UP(ADT, NCH, PAIRS)                                                                                    \
+  hipLaunchKernelGGL((k_gd_swiglu<ADT, NCH, PAIRS>), dim3(static_cast<unsigned>(hsteps), max_tiles),                  \
+                     dim3(gd::kThreads), 0, s, xb, ldx, top_k, up_gate, inter, uch, up_gate_alpha, offsets, pair_ids, \
+                     ne, hp, hs, hcorr, hb, ldh)
+#define MA_KS_UP(ADT, XP, MX)                                                                                        \
+  hipLaunchKernelGGL((k_grouped_swiglu_ks<2, ADT, 8, XP, MX>), dim3(static_cast<unsigned>(cdiv(inter, 32)), max_tiles), \
+                     dim3(512), 0, s, xb, ldx, x_pairs, x_corr, top_k, up_gate, inter, hidden / 16, up_gate_alpha,    \
+                     offsets, pair_ids, ne, hp, hs, hcorr, hb, ldh)
+#define MA_GD_DOWN(ADT, NCH, CP)                                                                                     \
+  hipLaunchKernelGGL((k_gd_down<ADT, NCH, CP>), dim3(static_cast<unsigned>(hidden / 256), max_tiles),                 \
+                     dim3(gd::kThreads), 0, s, reinterpret_cast<const uint32_t*>(hp), hs, hcorr, down, hidden, dch,   \
+                     down_alpha, offsets, ne, out)
+#define MA_GD_DOWNS(ADT, CP) \
+  if (dch == 2) MA_GD_DOWN(ADT, 2, CP); else if (dch == 3) MA_GD_DOWN(ADT, 3, CP); else MA_GD_DOWN(ADT, 0, CP);
+#define MA_DECODE(ADT)                                                                                              \
+  if (up_tile && down_tile) {                                                                                        \
+    if (uch == 8) MA_GD_UP(ADT, 8, false); else MA_GD_UP(ADT, 0, false);                                             \
+  } else if (up_tile) {                                                                                              \
+    if (uch == 8) MA_GD_UP(ADT, 8, true); else MA_GD_UP(ADT, 0, true);                                               \
+  } else if (down_tile) {                                                                                            \
+    if (x_pairs) MA_KS_UP(ADT, true, true); else MA_KS_UP(ADT, false, true);                                         \
+  } else {                                                                                                           \
+    if (x_pairs) MA_KS_UP(ADT, true, false); else MA_KS_UP(ADT, false, false);                                       \
+  }                                                                                                                  \
+  if (!down_tile) {                                                                                                  \
+    hipLaunchKernelGGL((k_grouped_down_ks<4, ADT, 8, 2>), dim3(static_cast<unsigned>(cdiv(hidden, 64)), max_tiles),   \
+                       dim3(512), 0, s, reinterpret_cast<const uint32_t*>(hp), down, hidden, inter / 16, down_alpha,  \
+                       offsets, ne, out);                                                                            \
+  } else if (up_tile) {                                                                                              \
+    MA_GD_DOWNS(ADT, 1)                                                                                              \
+  } else {                                                                                                           \
+    MA_GD_DOWNS(ADT, 4)                                                                                              \
+  }
+    if (alpha_dtype == MA_BF16) { MA_DECODE(MA_BF16) } else { MA_DECODE(MA_F32) }
+#undef MA_DECODE
+#undef MA_GD_DOWNS
 #undef MA_GD_DOWN
+#undef MA_KS_UP
 #undef MA_GD_UP
-    } else {
-      // rows too long for a tile in LDS: K split over the waves of a workgroup
-      const dim3 g1(static_cast<unsigned>(cdiv(inter, 32)), max_tiles), g2(static_cast<unsigned>(cdiv(hidden, 64)), max_tiles);
-#define MA_GROUPED_KS(ADT)                                                                       \
-  if (x_pairs)                                                                                   \
-    hipLaunchKernelGGL((k_grouped_swiglu_ks<2, ADT, 8, true>), g1, dim3(512), 0, s, xb, ldx,     \
-                       x_pairs, x_corr, top_k, up_gate, inter, hidden / 16, up_gate_alpha,      \
-                       offsets, pair_ids, ne, hp, hb, ldh);                                      \
-  else                                                                                           \
-    hipLaunchKernelGGL((k_grouped_swiglu_ks<2, ADT, 8, false>), g1, dim3(512), 0, s, xb, ldx,    \
-                       x_pairs, x_corr, top_k, up_gate, inter, hidden / 16, up_gate_alpha,      \
-                       offsets, pair_ids, ne, hp, hb, ldh);                                      \
-  hipLaunchKernelGGL((k_grouped_down_ks<4, ADT, 8, 2>), g2, dim3(512), 0, s,                     \
-                     reinterpret_cast<const uint32_t*>(hp), down, hidden, inter / 16,            \
-                     down_alpha, offsets, ne, out);
-      if (alpha_dtype == MA_BF16) { MA_GROUPED_KS(MA_BF16) } else { MA_GROUPED_KS(MA_F32) }
-#undef MA_GROUPED_KS
-    }
   } else {
     // prefill: the tokens' mx rows once (x_pairs are the decode form's), then
     // tiles of 128 pairs x 256 weight rows.  The tiles' copy sources are

@@ -204,6 +204,41 @@ def test_moe_grouped_decode_tiles_edges(dev, hidden, n_exp, inter, k, tokens, al
     assert torch.equal(z[keep], y[keep])
 
 
+@pytest.mark.parametrize("hidden,n_exp,inter,k,tokens,alpha", [
+    (2048, 4, 4352, 2, 5, torch.bfloat16), (512, 3, 4608, 1, 33, torch.float32),      # SwiGLU in tiles, down by K
+    (4352, 8, 768, 8, 16, torch.bfloat16), (4608, 5, 512, 2, 9, torch.float32),       # SwiGLU by K, down in tiles
+    (5120, 3, 4096, 1, 17, torch.bfloat16), (4352, 2, 256, 2, 3, torch.float32),
+    (4608, 2, 4352, 2, 7, torch.bfloat16)])                                           # both by K
+def test_moe_grouped_decode_long_rows(dev, hidden, n_exp, inter, k, tokens, alpha):
+    """Decode batches with rows past a tile's 4096 values in one stage or both, so
+    that h passes between the stages in either layout: h and y against the oracle
+    on the kernel's own routing, the same with x as pairs (read past 4096 values
+    of hidden), the same bits on a second run, and a token with an infinity leaves
+    the others alone."""
+    L = synthetic.make_moe_layer(hidden, n_exp, inter, seed=19, device=dev)
+    L.up_gate_alpha, L.down_alpha = L.up_gate_alpha.to(alpha), L.down_alpha.to(alpha)
+    assert tokens * k <= 16 * n_exp  # the decode form
+    rng = np.random.default_rng(tokens)
+    x = synthetic.randn_bf16((tokens, hidden + 8), 660 + tokens, dev)[:, :hidden]
+    x.copy_((x.double() * torch.from_numpy(2.0 ** rng.integers(-6, 3, size=x.shape)).to(dev)).to(torch.bfloat16))
+    ids, wts, xp = router_topk(x, L.gate_weight, k, pairs=True)
+    ref, href = ok.moe_experts(np_f(x), ids.cpu().numpy(), wts.cpu().numpy(), *_oracle_inputs(L))
+    for pairs in (None, xp):
+        y, h = moe_grouped(x, L, ids, wts, return_h=True, x_pairs=pairs)
+        what = f"H={hidden} I={inter} T={tokens} pairs={pairs is not None}"
+        # (2^-8 of the scale for h: see test_moe_grouped_decode_tiles_edges)
+        assert_bf16_close(np_f(h), href, atol_frac=2.0 ** -8, what="h " + what)
+        assert_bf16_close(np_f(y), ref, atol_frac=2.0 ** -7, what="y " + what)
+        y2, h2 = moe_grouped(x, L, ids, wts, return_h=True, x_pairs=pairs)
+        assert torch.equal(y2, y) and torch.equal(h2, h)
+    y = moe_grouped(x, L, ids, wts)
+    x = x.clone()
+    x[tokens // 2, 1] = float("inf")
+    z = moe_grouped(x, L, ids, wts)
+    keep = torch.arange(tokens, device=dev) != tokens // 2
+    assert torch.equal(z[keep], y[keep])
+
+
 @pytest.mark.parametrize("n_exp,inter,tokens,alpha", [
     (8, 256, 4, torch.bfloat16), (8, 256, 16, torch.float32), (256, 512, 17, torch.float32),
     (256, 512, 33, torch.bfloat16), (40, 1024, 65, torch.bfloat16), (40, 1280, 20, torch.float32)])
