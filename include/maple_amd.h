@@ -70,6 +70,11 @@ int ma_ternary_gemv(const void* x, int x_dtype, int64_t batch, int64_t ldx,
  * src/maple_run/kernels/ternary_gemv.py:261-388 (its batched path :156-258).
  */
 size_t ma_ternary_gemv_workspace_bytes(int64_t batch, int64_t nwords, int rms);
+/*
+ * The bytes that a call of n_out rows uses, at most those of the query above:
+ * from 64 tokens it may take the forms of fewer tokens (0: it uses none).
+ */
+size_t ma_ternary_gemv_call_workspace_bytes(int64_t batch, int64_t n_out, int64_t nwords, int rms);
 int ma_ternary_gemv_ws(const void* x, int x_dtype, int64_t batch, int64_t ldx,
                        const uint32_t* packed, int64_t n_out, int64_t nwords, int packed_kn,
                        const void* row_alpha, int alpha_dtype,

@@ -33,6 +33,7 @@ _SIGNATURES = {
     "ma_last_error": [],
     "ma_ternary_gemv": [_P, _I, _L, _L, _P, _L, _L, _I, _P, _I, _P, _I, _F, _P, _L, _P],
     "ma_ternary_gemv_workspace_bytes": [_L, _L, _I],
+    "ma_ternary_gemv_call_workspace_bytes": [_L, _L, _L, _I],
     "ma_ternary_gemv_ws": [_P, _I, _L, _L, _P, _L, _L, _I, _P, _I, _P, _I, _F, _P, _L, _P, _Z, _P],
     "ma_router_workspace_bytes": [_L, _L],
     "ma_router_topk": [_P, _I, _L, _L, _P, _I, _L, _L, _P, _I, _P, _P, _P, _Z, _P],
@@ -101,7 +102,7 @@ _RESTYPES = {"ma_last_error": ctypes.c_char_p, "ma_router_workspace_bytes": _Z,
              "ma_moe_fused_workspace_bytes": _Z, "ma_moe_route_workspace_bytes": _Z,
              "ma_moe_grouped_noalloc_max_bytes": _Z, "ma_sampler_workspace_bytes": _Z,
              "ma_flash_head_workspace_bytes": _Z, "ma_rtn4_gemv_workspace_bytes": _Z,
-             "ma_rtn4_gemv_mx_workspace_bytes": _Z}
+             "ma_rtn4_gemv_mx_workspace_bytes": _Z, "ma_ternary_gemv_call_workspace_bytes": _Z}
 
 _lib = None
 

@@ -170,6 +170,14 @@ extern "C" size_t ma_ternary_gemv_workspace_bytes(int64_t batch, int64_t nwords,
   return rms && batch >= kXpMinBatch ? tgemm_xp_bytes(batch, nwords) : 0;
 }
 
+// One call's bytes: those of the form it takes (the query above does not know
+// n_out and answers for the larger form).
+extern "C" size_t ma_ternary_gemv_call_workspace_bytes(int64_t batch, int64_t n_out, int64_t nwords, int rms) {
+  if (nwords < 1 || nwords % 16 != 0 || n_out < 1) return 0;
+  if (mx_faster(batch, n_out)) return tgemm_mx_bytes(batch, nwords, rms != 0);
+  return rms && batch >= kXpMinBatch ? tgemm_xp_bytes(batch, nwords) : 0;
+}
+
 extern "C" int ma_ternary_gemv_ws(const void* x, int x_dtype, int64_t batch, int64_t ldx,
                                   const uint32_t* packed, int64_t n_out, int64_t nwords,
                                   int packed_kn, const void* row_alpha, int alpha_dtype,

@@ -3,8 +3,8 @@
 Drop-in for reference ``src/maple_run/kernels/ternary_gemv.py:261-388``: same
 signature, argument meaning, output shape/dtype and exceptions.  The work is
 ``ma_ternary_gemv`` (one launch) or, for the RMS-folded form at 17 tokens and
-more and for any form at 64, ``ma_ternary_gemv_ws`` (operand build + GEMM), HIP on gfx950, on the
-current stream.
+more and for any form from 64 tokens of enough rows, ``ma_ternary_gemv_ws``
+(operand build + GEMM), HIP on gfx950, on the current stream.
 """
 
 from __future__ import annotations
@@ -87,10 +87,10 @@ def ternary_gemv(
         float(rms_eps),
         _lib.ptr(y), n_out,
     )
-    # With the RMSNorm folded in, from 17 tokens, and always from 64, a two-launch form
-    # builds each token's operands once into a workspace (the query says 0 where
-    # no workspace is used).
-    ws_bytes = _lib.load().ma_ternary_gemv_workspace_bytes(batch, nwords, int(rms_w is not None))
+    # With the RMSNorm folded in, from 17 tokens, and from 64 tokens of enough rows, a two-launch
+    # form builds each token's operands once into a workspace (the query says 0 where none is used).
+    ws_bytes = 0 if packed_kn or x_mat.dtype != torch.bfloat16 else _lib.load().ma_ternary_gemv_call_workspace_bytes(
+        batch, n_out, nwords, int(rms_w is not None))
     if ws_bytes:
         ws = torch.empty(ws_bytes, device=x.device, dtype=torch.uint8)
         _lib.call("ma_ternary_gemv_ws", *args, _lib.ptr(ws), ws_bytes, _lib.stream_of(x))
@@ -115,7 +115,7 @@ def ternary_gemv_combine(pending, packed_weight: torch.Tensor, row_alpha: torch.
     rms_w = rms_weight.reshape(-1).contiguous()
     alpha = row_alpha.reshape(-1).contiguous()
     pw = packed_weight.contiguous()
-    ws_bytes = _lib.load().ma_ternary_gemv_workspace_bytes(tokens, nwords, 1)
+    ws_bytes = _lib.load().ma_ternary_gemv_call_workspace_bytes(tokens, n_out, nwords, 1)
     ws = torch.empty(max(int(ws_bytes), 1), device=x.device, dtype=torch.uint8)
     _lib.call(
         "ma_ternary_gemv_combine_ws",

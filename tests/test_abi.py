@@ -7,6 +7,7 @@ entry points.
 from __future__ import annotations
 
 import ctypes
+import importlib
 
 import torch
 import re
@@ -69,6 +70,39 @@ def test_size_errors_map_without_a_gpu():
         _lib.call("ma_moe_grouped", fake, 2048, None, None, 1 << 22, 8, fake, fake, fake, fake,
                   _lib.dtype_code(torch.empty(0, dtype=torch.bfloat16), "a"), 64, 2048, 768, fake, fake,
                   fake, fake, None, 0, None, 0, fake, fake, 1 << 62, None)
+
+
+@pytest.mark.parametrize("rms", [0, 1])
+def test_ternary_gemv_call_workspace_is_what_the_call_uses(rms):
+    """The scaled 8-bit form's bytes only for calls it takes (from 64 tokens, past
+    4 x 2^16 outputs); below, the two-launch RMS form's, or none; never above the
+    query that does not know the rows."""
+    lib = _lib.load()
+    call, most = lib.ma_ternary_gemv_call_workspace_bytes, lib.ma_ternary_gemv_workspace_bytes
+    for batch in (1, 16, 17, 63, 64, 65, 127, 128, 2048):
+        for n_out in (8, 2048, 2049, 4096, 4097, 5120):
+            used = call(batch, n_out, 128, rms)
+            assert used <= most(batch, 128, rms)
+            if batch >= 64 and batch * n_out > 4 * 65536:
+                assert used == most(batch, 128, rms) > 0
+            else:
+                assert (used > 0) == (rms == 1 and batch >= 17)
+    assert call(2048, 5120, 120, rms) == 0
+
+
+def test_ternary_gemv_takes_no_workspace_it_does_not_use(monkeypatch):
+    """The wrapper allocates by that query (the launch is a stand-in): 64 tokens x
+    2048 rows without the RMSNorm go to ma_ternary_gemv, 64 x 5120 to the
+    workspace entry; float16 x, which no workspace form takes, to the first."""
+    mod = importlib.import_module("maple_amd.kernels.ternary_gemv")  # (the package has a function of that name)
+    called = []
+    monkeypatch.setattr(mod._lib, "call", lambda name, *args: called.append(name))
+    monkeypatch.setattr(mod._lib, "stream_of", lambda t: None)
+    monkeypatch.setattr(torch.Tensor, "is_cuda", property(lambda self: True))
+    for rows, dtype in ((2048, torch.bfloat16), (5120, torch.bfloat16), (5120, torch.float16)):
+        mod.ternary_gemv(torch.zeros(64, 2048, dtype=dtype), torch.zeros(rows, 128, dtype=torch.uint32),
+                         torch.ones(rows, dtype=torch.bfloat16))
+    assert called == ["ma_ternary_gemv", "ma_ternary_gemv_ws", "ma_ternary_gemv"]
 
 
 def test_rtn4_gemv_mx_rejects_null_pointers_without_a_gpu():
