@@ -425,7 +425,7 @@ def test_rtn4_gemv_vs_oracle(dev, batch, group):
 @pytest.mark.parametrize("batch,group,n_out", [(5, 64, 4000), (16, 128, 4096), (32, 64, 1000),
                                                (40, 128, 4096)])
 def test_rtn4_mfma_batched_vs_oracle(dev, batch, group, n_out):
-    """Batch >= 5 runs the MFMA RTN4 GEMM (both group sizes, partial row
+    """A batch from 5 tokens as rtn4_gemv runs it (both group sizes, partial row
     tiles, several token tiles); batched == per-row within 8e-3
     (reference tests/test_rtn4.py:151-169)."""
     w, sc, bs = synthetic.rtn4_table(n_out, 2048, group, 93 + batch, dev)
@@ -438,6 +438,27 @@ def test_rtn4_mfma_batched_vs_oracle(dev, batch, group, n_out):
     # every sum has a fixed order: the same bits on every run
     for _ in range(3):
         assert torch.equal(rtn4_gemv(x, w, sc, bs, group_size=group), y)
+
+
+@pytest.mark.parametrize("batch,group,n_out,dtype", [
+    (5, 64, 4000, torch.bfloat16), (16, 128, 4096, torch.bfloat16), (17, 64, 1000, torch.float32),
+    (40, 128, 1003, torch.bfloat16)])
+def test_rtn4_bf16_gemm_vs_oracle(dev, batch, group, n_out, dtype):
+    """ma_rtn4_gemv's bf16 GEMM (from 5 tokens; what rtn4_gemv keeps it for is short
+    rows and few tokens) at K = 2048: both group sizes and scale types, partial row
+    tiles, one and several token tiles, the same bits on a second run."""
+    from maple_amd import _lib
+    w, sc, bs = synthetic.rtn4_table(n_out, 2048, group, 109 + batch, dev)
+    sc, bs = sc.to(dtype), bs.to(dtype)
+    x = synthetic.randn_bf16((batch, 2048), 110, dev)
+    out = [torch.empty(batch, n_out, device=dev, dtype=torch.bfloat16) for _ in range(2)]
+    for y in out:
+        _lib.call("ma_rtn4_gemv", _lib.ptr(x), _lib.BF16, batch, 2048, _lib.ptr(w), n_out, 256, 0, _lib.ptr(sc),
+                  _lib.dtype_code(sc, "s"), _lib.ptr(bs), _lib.dtype_code(bs, "b"), group, _lib.ptr(y), n_out,
+                  _lib.stream_of(x))
+    ref = ok.rtn4_gemv(np_f(x), np_u32(w), np_f(sc), np_f(bs), group_size=group)
+    assert_bf16_close(np_f(out[0]), ref, what=f"rtn4 bf16 B={batch} g={group}")
+    assert torch.equal(out[0], out[1])
 
 
 @pytest.mark.parametrize("batch,n_out,k_in,group,dtype", [

@@ -97,9 +97,10 @@ def test_moe_grouped_zipf_vs_oracle(dev, layer, tokens):
 
 @pytest.mark.parametrize("tokens", [256, 2048])
 def test_router_pairs_equal_grouped_own_prep(dev, layer, tokens):
-    """router_topk(pairs=True) writes x' from its top-k launch; moe_block's
-    prefill path hands them to the grouped kernels: the same ids, weights, x'
-    and y bits as router_topk + moe_grouped building x' itself."""
+    """router_topk(pairs=True) writes x' from its top-k launch: the same ids and
+    weights as without, and x' as the oracle forms it.  The grouped kernels do not
+    read it at these shapes (test_moe_grouped_decode_long_rows has those that do):
+    the same y given it or not, and from moe_block."""
     L = synthetic.MoELayer(layer.gate_weight, layer.up_gate_packed, layer.up_gate_alpha,
                            layer.down_packed, layer.down_alpha, zipf_bias(dev))
     x = synthetic.randn_bf16((tokens, H), 700 + tokens, dev)
@@ -122,8 +123,8 @@ def test_router_pairs_equal_grouped_own_prep(dev, layer, tokens):
 
 @pytest.mark.parametrize("hidden,n_exp,inter,k,tokens", [(3072, 8, 1024, 4, 96), (1024, 16, 512, 2, 200)])
 def test_moe_grouped_prefill_form_other_shapes(dev, hidden, n_exp, inter, k, tokens):
-    """The prefill-form grouped kernels (more than 16 pairs per expert: x'
-    copied into LDS a K step ahead, 128-pair x 256-row tiles) at hidden sizes
+    """The prefill-form grouped kernels (more than 16 pairs per expert: mx rows
+    copied into LDS a K step ahead, tiles of 32 or 64 pairs x 256 rows) at hidden sizes
     and expert widths other than the synthetic layer's (K loops of 24 / 8 /
     64 / 4 steps): h and y against the oracle on the kernel's own routing, and
     the same bits on a second run."""
@@ -175,7 +176,7 @@ def test_moe_grouped_prefill_tiles_edges(dev, hidden, n_exp, inter, k, tokens, a
     (512, 2, 4096, 1, 31, torch.bfloat16),    # the widest h; a full and a ragged tile
     (2048, 8, 768, 8, 16, torch.bfloat16),    # 16 pairs an expert: one whole tile each
     (768, 20, 512, 3, 33, torch.float32),
-    (4352, 2, 256, 2, 8, torch.bfloat16)])    # past a tile: K split over the waves
+    (4352, 2, 256, 2, 8, torch.bfloat16)])    # past a tile: the SwiGLU stage's K split over the waves
 def test_moe_grouped_decode_tiles_edges(dev, hidden, n_exp, inter, k, tokens, alpha):
     """The decode form at the edges of its 16-pair tiles, over values of very
     different size and rows with a stride: h and y against the oracle on the
@@ -259,9 +260,9 @@ def test_moe_block_decode_batches_other_shapes(dev, n_exp, inter, tokens, alpha)
 
 @pytest.mark.parametrize("tokens", [8, 32, 128])
 def test_moe_layer_routed_pairs_vs_oracle(dev, layer, tokens):
-    """The decoder's batched MoE half: one routing launch that also writes xn
-    as x' pairs, then the tile-resident expert kernels reading those pairs
-    (hidden 2048, intermediate 768), against the oracle on the same routing."""
+    """The decoder's batched MoE half: one routing launch that also writes xn, then
+    the tile-resident expert kernels reading it (hidden 2048, intermediate 768),
+    against the oracle on the same routing."""
     from maple_amd.moe import moe_layer
     L = synthetic.MoELayer(layer.gate_weight, layer.up_gate_packed, layer.up_gate_alpha,
                            layer.down_packed, layer.down_alpha, zipf_bias(dev))
