@@ -57,9 +57,11 @@ int ma_ternary_gemv(const void* x, int x_dtype, int64_t batch, int64_t ldx,
  * (rms_weight != NULL) and 17 tokens or more, every token's GEMM operands
  * (the x' pairs of the hi and lo halves of x * w_rms, the correction and the
  * RMS scale) are built once into the workspace by a first launch and the MFMA
- * GEMM reads them from there.  From 64 tokens, with or without the RMSNorm,
- * the operands are FP8 pieces of x (two hold bf16 x whole, four carry x *
- * w_rms) and the codes multiply them as FP4.  workspace: 256-byte aligned, at
+ * GEMM reads them from there.  From 64 tokens and 4 x 2^16 outputs, with or
+ * without the RMSNorm, the operands are FP8 pieces and the codes multiply them
+ * as FP4: two pieces hold a bf16 x down to 2^-13 of the largest of its 32
+ * neighbours, and to 2^-20 of that below; four carry x * w_rms to 2^-19 of
+ * itself or 2^-29 of that largest.  workspace: 256-byte aligned, at
  * least ma_ternary_gemv_workspace_bytes(batch, nwords, rms_weight != NULL)
  * bytes; that query returns 0 where no workspace is used (batch < 64 without
  * the RMSNorm, batch < 17, nwords % 16 != 0), and then -- as for any input the
@@ -268,8 +270,9 @@ int ma_rtn4_gemv_ws(const void* x, int x_dtype, int64_t batch, int64_t ldx,
  * ma_rtn4_gemv on the scaled 8-bit matrix instructions, from batch 5 in groups
  * of 64 or 128 with nwords a multiple of 32 (bf16 x, [N, K/8] codes, bf16 or
  * float32 scales and biases of one dtype; x, codes, scales and biases 16-byte
- * aligned): x is written once into the workspace as FP8 pieces that hold it
- * whole, and the codes multiply it as FP8.  Short rows and a few tokens, where
+ * aligned): x is written once into the workspace as two FP8 pieces, which hold
+ * it down to 2^-13 of the largest of its 64 neighbours and to 2^-20 of that
+ * below, and the codes multiply it as FP8.  Short rows and a few tokens, where
  * one launch is the faster, are ma_rtn4_gemv's; any other call is
  * ma_rtn4_gemv_ws's where the workspace has that call's bytes, else
  * ma_rtn4_gemv's (workspace may then be NULL).  Same values as ma_rtn4_gemv up

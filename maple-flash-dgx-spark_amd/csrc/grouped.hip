@@ -4,23 +4,26 @@
 // [tokens x K] operand, so the SwiGLU up+gate projection and the down
 // projection become per-expert GEMMs: y = W_e (rows x K) . X_e^T (K x tokens).
 //
-// A operand (weights): each lane expands its own packed words with
-// expand_word (common.h) into bf16x2 dwords of 1 + c/f -- exactly the dword
-// order of the bf16 x' pairs, an (arbitrary but shared) permutation of K
-// inside each word.  B operand (activations): x' = f * x pairs.  The MFMA then
-// accumulates sum (f + c) x; subtracting C_t = sum (f + 1) x per token
+// Forms, by pairs per expert and by K:
+//  * decode batches (few pairs): 16-pair tiles whose rows lie in LDS for all of
+//    K, up to 4096 values (gd), else K split over the waves with operands in
+//    registers (ks), each stage by its own K;
+//  * prefill: tiles of 64 or 32 pairs x 256 rows, K in steps through LDS (gp).
+// gd and gp multiply on the scaled 8-bit matrix instructions: codes as FP4,
+// activations as mx rows (mx.h).  ks multiplies in bf16: each lane expands its
+// packed words with expand_word (common.h) into bf16x2 dwords of 1 + c/f --
+// exactly the dword order of the bf16 x' pairs, an (arbitrary but shared)
+// permutation of K inside each word -- against x' = f * x pairs; the MFMA then
+// accumulates sum (f + c) x, and subtracting C_t = sum (f + 1) x per token
 // leaves sum (c - 1) x, the ternary product (float32 accumulation).
 //
 // v_mfma_f32_16x16x32_bf16 lane layout (checked on the device):
 //   A: lane l holds row l%16, k 8(l/16)..+8;  B: col l%16, k 8(l/16)..+8;
 //   C: lane l holds col l%16, rows 4(l/16)..+4.
 //
-// Two forms: decode batches (few pairs per expert: 16-pair tiles, K split
-// over the waves, operands in registers) and prefill (128-pair x 256-row
-// tiles with the x' operands staged in LDS).  Stage 1 computes h (each wave
-// holds up rows and the matching gate rows, so SwiGLU is applied in
-// registers), rounded to bf16 like the reference's x.dtype store
-// (ternary_expert.py:441), in the x' pair layout the down stage reads and
+// Stage 1 computes h (each wave holds up rows and the matching gate rows, so
+// SwiGLU is applied in registers), rounded to bf16 like the reference's x.dtype
+// store (ternary_expert.py:441), in the layout the down stage reads and
 // optionally in the plain [slot, I] layout.  Stage 2 writes each pair's down
 // output rounded to bf16 (ternary_expert.py:208); a gather kernel then forms
 // y[t] = sum_j w[t,j] out[pair(t,j)] (+ residual) in float32
@@ -118,7 +121,7 @@ __device__ __forceinline__ float pairs_cst(const uint32_t pr[8]) {
 }
 
 // ---------------------------------------------------------------------------
-// Decode form (few pairs per expert): 16-pair tiles, K split over the KW waves
+// Decode form of rows past 4096 values: 16-pair tiles, K split over the KW waves
 // of a workgroup, each wave's operands loaded and built in registers (no LDS
 // staging) and the partial tiles added in wave order through LDS; with a
 // handful of tokens per expert, a K walk per workgroup left the chip idle.
@@ -439,16 +442,22 @@ __global__ __launch_bounds__(64 * KW) void k_grouped_down_ks(
 // FP4: three instructions a word where the bf16 operands took twelve, and the
 // products need no spacing by hand.  The SwiGLU stage writes the tile's mx rows
 // of x itself (with every pair's sum), so it needs x alone, and h's like the
-// prefill form; both stages' operands are exact, so a row differs from its
-// float64 value by its bf16 rounding and little else.  Every load of a tile (x
-// or h, scales, sums, the first weights) is issued unconditionally up front, a
-// lane past the tile's end reading its last pair again: under a branch the
-// compiler moves a load next to its use and waits for it there, one round trip a
-// row (256 experts, 32 tokens x 8: the down stage 27 us that way).  Bound by the
+// prefill form; both stages' operands hold the bf16 values to 2^-20 of their
+// block's largest (mx.h), so a row differs from its float64 value by its bf16
+// rounding and little else.  The down stage issues its loads of h and of the
+// first weights unconditionally up front, a lane past the tile's end reading its
+// last pair again: under a branch the compiler moved them next to their uses and
+// waited there, one round trip a row (256 experts, 32 tokens x 8: 27 us that way).
+// (The SwiGLU stage's x rows are under a wave's own branch and are issued
+// together all the same; scales and sums are one load a thread.)  Bound by the
 // weights' bytes and a few such round trips.  Hidden 2048: a block of 64 experts
 // (inter 768) 24 us at 4 tokens x 8 and 38 at 32 (30 and 41 with bf16 operands),
 // of 256 (inter 512) 53 at 32 and 66 at 64 (57 and 74).
 // NCH: chunks of 256 values of K (0: at run time, up to 16; the others unroll).
+// The run-time instances reserve LDS for 16 chunks, so one workgroup runs on a
+// CU whatever K is; they are still no slower than the bf16 kernels at any size
+// tried (32 tokens x 8, us a block, bf16 / now: hidden 1024, inter 512, 64 experts
+// 37 / 25; 3072, 768, 32 44 / 36; 4096, 1024, 32 68 / 50; 2048, 256, 64 37 / 30).
 // ---------------------------------------------------------------------------
 namespace gd {
 constexpr int kWaves = 8, kThreads = 64 * kWaves;
@@ -856,7 +865,8 @@ __global__ __launch_bounds__(256) void k_combine8(const uint16_t* __restrict__ o
 // Prefill form (many pairs per expert): tiles of 64 or 32 pairs x 256 weight
 // rows, four waves of 64 rows, K walked in steps of 8 words (128 codes) on
 // v_mfma_scale_f32_16x16x128_f8f6f4: the codes as FP4, the activations as mx
-// rows of two FP8 pieces (mx.h), which hold bf16 values whole.  A step's mx
+// rows of two FP8 pieces (mx.h), which hold bf16 values to 2^-20 of their block's
+// largest.  A step's mx
 // rows of the pairs are copied into LDS by the LDS DMA
 // (global_load_lds_dwordx4: no staging registers), one step ahead with the
 // step's weights, one barrier per step; three workgroups run on a CU (two steps
@@ -864,8 +874,8 @@ __global__ __launch_bounds__(256) void k_combine8(const uint16_t* __restrict__ o
 // tokens' mx rows are written once (launch_mx_prep_wide) and h's by the SwiGLU
 // epilogue, so staging is a copy.  Each lane expands its own weight words with
 // two ANDs and a shift a word: words 4g .. 4g+3 of two steps' 16 for lane group
-// g, loaded at once (64 bytes of a row), the first two in the even step.  Tiles go to workgroups so that the row tiles of one pair tile share an
-// XCD (workgroups are placed on the 8 XCDs round-robin), which keeps that
+// g, loaded at once (64 bytes of a row), the first two in the even step.  Tiles
+// go to workgroups so that the row tiles of one pair tile share an XCD (workgroups are placed on the 8 XCDs round-robin), which keeps that
 // tile's rows in one L2.
 //
 // 2048 tokens x 8 on 64 experts (103 GFLOP SwiGLU, 52 down): 104 and 60 us with
@@ -1452,8 +1462,8 @@ static int grouped_launch(const void* x, int64_t ldx, const uint32_t* x_pairs, c
 #undef MA_KS_UP
 #undef MA_GD_UP
   } else {
-    // prefill: the tokens' mx rows once (x_pairs are the decode form's), then
-    // tiles of 128 pairs x 256 weight rows.  The tiles' copy sources are
+    // prefill: the tokens' mx rows once (x_pairs are the K-split form's), then
+    // tiles of 64 or 32 pairs x 256 weight rows.  The tiles' copy sources are
     // 32-bit offsets in 16-byte chunks into the mx rows of x and h.
     if (static_cast<uint64_t>(tokens) * hidden / 2 >= (uint64_t{1} << 32) ||
         static_cast<uint64_t>(n_pairs) * inter / 2 >= (uint64_t{1} << 32))

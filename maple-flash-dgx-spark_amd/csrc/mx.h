@@ -3,8 +3,8 @@
 // v_mfma_scale_f32_16x16x128_f8f6f4 takes each operand in its own small float
 // format with one power-of-two scale per 32 values of K, and this card reaches
 // 4.3 PFLOP/s with it against 1.3 with v_mfma_f32_16x16x32_bf16 (eight
-// independent accumulators a wave, both measured).  Two properties make it
-// exact for packed codes and bf16 activations:
+// independent accumulators a wave, both measured).  Two properties fit it to
+// packed codes and bf16 activations:
 //
 //  * A code c in 0..3 as the bits of an FP4 (E2M1) number reads as c / 2, so a
 //    packed ternary word becomes two operand registers with one shift and two
@@ -14,8 +14,8 @@
 //  * A bf16 value has 8 significant bits and FP8 (E4M3) 4, so x = p0 + p1 / 16
 //    exactly, p0 the nearest E4M3 number and p1 sixteen times what is left
 //    (values 2^13 below their block's largest lose bits below 2^-20 of that
-//    largest).  Each further piece takes 4 to 5 more bits: four carry a
-//    float32 product as far as two bf16 numbers do.  The pieces cost what one
+//    largest).  Each further piece takes 4 to 5 more bits: four carry a float32
+//    product to 2^-19 of itself or 2^-29 of that largest.  The pieces cost what one
 //    bf16 pass would at twice the rate; what is saved is the expansion.
 //
 // Lane layout of 16x16x128 (checked on the device; logical K index k):

@@ -18,14 +18,15 @@ constexpr int kMxTok = 64;  // tokens of the larger tile; the workspace's rows a
 
 // One token per workgroup: x (times w_rms) as an mx row of NP pieces, xs[t *
 // s_row + step * s_step] its scale bytes, xc[t] = (sum x_hat, RMS factor) with the sums in a
-// fixed order.  Two pieces hold bf16 x; the RMS-folded product is float32 and
-// takes four, which is no less than the two bf16 numbers of the smaller
-// batches' operands (relative 2^-19 against 2^-17).  Latency: about 5 us for 2048
+// fixed order.  Two pieces hold bf16 x (mx.h); the RMS-folded product is float32
+// and takes four, which hold it to 2^-19 of itself or 2^-29 of its block's
+// largest (the two bf16 numbers of the smaller batches' operands: 2^-17 of
+// itself).  Latency: about 5 us for 2048
 // x 2048 with two pieces and 8 with four (16 MB written).  XCD x takes the
 // tokens of its eighth, whose tiles it multiplies too (k_mx_gemm), and a step's
 // scale word is one store: with tokens dealt to the XCDs in turn and a byte a
 // block, a line of scale words was written by all eight (both launches for 2048
-// tokens at K = 2048: 27.2 -> 23.9 us to 2048 rows, with the RMSNorm 48.7 -> 45.1
+// tokens at K = 2048: 27.2 -> 23.9 us to 2048 rows, with the RMSNorm 49.4 -> 43.0
 // to 2560 and 31.5 -> 26.1 to 1024).  (WIDE rows are gathered
 // by expert from every XCD: in order.)  With a MoE combine in front (cb.slot_out
 // set, NP 4) the rows are combined first instead of read from x.
@@ -114,8 +115,8 @@ constexpr int mx_vmcnt(int n) { return (n & 0xF) | (0x7 << 4) | ((n >> 4) << 14)
 // operands need two ANDs and a shift a word, so a tile is bound by the matrix
 // instructions and the steps' fixed parts: both launches for 2048 tokens x 2048
 // -> 2560 take 28.4 us (208 as bf16 MFMAs of 16-row tiles, which read each
-// token's operands 160 times), 45.1 with the RMSNorm (149), 777 x 2048 -> 2048
-// 16.1 (68).
+// token's operands 160 times), 43.1 with the RMSNorm (149), 777 x 2048 -> 2048
+// 17.4 (68).
 template <int NP, int TOK, int NBUF>
 struct MxTile {
   // (a wave's lanes copy 64 scale words; those past a tile of 32 tokens are the

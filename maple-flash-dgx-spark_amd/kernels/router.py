@@ -32,9 +32,9 @@ def router_topk(
     Returns ``(topk_idx int32 [..., top_k], topk_weight float32 [..., top_k])``
     in descending probability order, ties to the lowest expert index.  With
     ``pairs`` (bf16 ``x``, K a multiple of 16), a third item ``(x_pairs,
-    x_corr)``: ``x`` in the form the grouped experts read, written by the same
-    launch as the top-k (``moe_grouped(..., x_pairs=...)`` then skips its own
-    x' launch; same bits).
+    x_corr)``: ``x`` as x' pairs, written by the same launch as the top-k, for
+    ``moe_grouped(..., x_pairs=...)``, which reads them in decode batches of more
+    than 4096 values a row.
     """
     if not x.is_cuda or not gate_weight.is_cuda:
         raise RuntimeError("router_topk requires CUDA tensors.")

@@ -18,7 +18,7 @@ device):
   rounding points: each slot's down output rounded to bf16 before the
   float32 combine, the residual added last (``model.py:470-473``).
 * batched decode / prefill: dispatch the (token, slot) pairs into per-expert
-  lists and run grouped MFMA GEMMs (``ma_moe_grouped``), so each selected
+  lists and run grouped GEMMs (``ma_moe_grouped``), so each selected
   expert's weights are read once per tile of its tokens instead of once per
   pair.  Rounding points match the reference (bf16 h, bf16 per-slot output,
   float32 combine).
@@ -239,8 +239,8 @@ def moe_route(x: torch.Tensor, layer: MoELayer, top_k: int, norm_weight: torch.T
     when ``add`` is None), ``xn = rms_norm(h) * norm_weight``, the router's
     int32 ids / float32 weights ``[T, top_k]`` and the :class:`Dispatch` lists.
     Equal, bit for bit, to add_rms_norm + router_topk + moe_dispatch.  With
-    ``pairs``, a sixth item ``(xn_pairs, xn_corr)``: xn in the x' pair form the
-    grouped experts read, and each token's correction."""
+    ``pairs``, a sixth item ``(xn_pairs, xn_corr)``: xn in the x' pair form, and
+    each token's correction."""
     from .kernels.dispatch import Dispatch
     tokens, hidden = x.shape
     dev = x.device
@@ -299,7 +299,8 @@ def moe_grouped(x: torch.Tensor, layer: MoELayer, ids: torch.Tensor, wts: torch.
 
     ``dispatch``: the lists for ``ids`` if already built (``moe_route``);
     ``x_pairs``: ``(xn_pairs, xn_corr)`` of ``x`` from ``moe_route(pairs=True)``
-    or ``router_topk(..., pairs=True)``.
+    or ``router_topk(..., pairs=True)``, read where hidden is past 4096 in a
+    decode batch.
     Returns ``y [T, H]`` (bf16), and with ``return_h`` also ``h [T, k, I]``;
     with ``combine=False`` a ``PendingCombine`` in place of ``y``.
     """
