@@ -735,12 +735,17 @@ __global__ __launch_bounds__(gd::kThreads) void k_gd_down(const uint32_t* __rest
     for (int k = 0; k < kPer; ++k) hv[ci][k] = src[lane + 64 * k < nsteps * 16 ? lane + 64 * k : 0];
   }
   uint32_t sw = 0;
-  float cp = 0.f;
+  float cp[CP] = {};  // (added up where they are stored: an addition here waits for its load)
   const int sc = tid / nsteps, ss = tid % nsteps;  // 16 nsteps <= 512
   if (sc < np) {
     sw = hs[static_cast<int64_t>(pos0 + sc) * nsteps + ss];
+    if constexpr (CP == 1) {
+      cp[0] = hcorr[static_cast<int64_t>(pos0 + sc) * nsteps + ss];
+    } else {
+      const float* const parts = hcorr + (static_cast<int64_t>(pos0 + sc) * nsteps + ss) * CP;
 #pragma unroll
-    for (int q = 0; q < CP; ++q) cp += hcorr[(static_cast<int64_t>(pos0 + sc) * nsteps + ss) * CP + q];
+      for (int q = 0; q < CP; ++q) cp[q] = parts[q];
+    }
   }
   MA_ISSUE_FENCE();
   const uint32_t* we = w + static_cast<int64_t>(e) * n_out * nwk;
@@ -762,7 +767,10 @@ __global__ __launch_bounds__(gd::kThreads) void k_gd_down(const uint32_t* __rest
   }
   if (sc < np) {
     sh.scale[sc][ss] = sw;
-    s_cp[sc][ss] = cp;
+    float c = cp[0];
+#pragma unroll
+    for (int q = 1; q < CP; ++q) c += cp[q];
+    s_cp[sc][ss] = c;
   }
   __syncthreads();
   mx_f32x4_t acc[2][2];
