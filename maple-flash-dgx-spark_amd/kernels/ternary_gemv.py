@@ -14,6 +14,7 @@ import torch
 from .. import _lib
 
 _CODES_PER_WORD = 16
+_WORKSPACE_MIN_TOKENS = 17  # no form of fewer tokens uses a workspace (the query says 0)
 
 
 def ternary_gemv(
@@ -89,8 +90,9 @@ def ternary_gemv(
     )
     # With the RMSNorm folded in, from 17 tokens, and from 64 tokens of enough rows, a two-launch
     # form builds each token's operands once into a workspace (the query says 0 where none is used).
-    ws_bytes = 0 if packed_kn or x_mat.dtype != torch.bfloat16 else _lib.load().ma_ternary_gemv_call_workspace_bytes(
-        batch, n_out, nwords, int(rms_w is not None))
+    ws_bytes = 0
+    if batch >= _WORKSPACE_MIN_TOKENS and not packed_kn and x_mat.dtype == torch.bfloat16:
+        ws_bytes = _lib.load().ma_ternary_gemv_call_workspace_bytes(batch, n_out, nwords, int(rms_w is not None))
     if ws_bytes:
         ws = torch.empty(ws_bytes, device=x.device, dtype=torch.uint8)
         _lib.call("ma_ternary_gemv_ws", *args, _lib.ptr(ws), ws_bytes, _lib.stream_of(x))
